@@ -621,10 +621,10 @@ int aps_linear(const float* x, const float* weight, const float* bias, int64_t r
     if ((addr_bits & 3u) != 0) return fail(APS_ERR_ARG, "linear: arrays must be 4-byte aligned");
     if (y == x) return fail(APS_ERR_ARG, "linear: y must not alias x");
     const hipStream_t s = static_cast<hipStream_t>(stream);
-    // in % 16, out % 4 and 16-byte alignment take the vector / matrix-core
-    // kernels; any other shape the SIMT kernel (same chains, same bits)
-    if (in_features % 16 == 0 && out_features % 4 == 0 && (addr_bits & 15u) == 0 && (rows + 63) / 64 <= 65535)
-        APS_HIP(aps::launch_linear_f32(x, weight, bias, y, rows, in_features, out_features, s), "linear launch");
+    // in % 16, out % 4 and 16-byte alignment take the matrix-core kernels; any
+    // other shape the SIMT kernel (same chains, same bits)
+    if (aps::linear_mfma_fits(rows, in_features, out_features) && (addr_bits & 15u) == 0)
+        APS_HIP(aps::launch_linear_mfma_f32(x, weight, bias, y, rows, in_features, out_features, s), "linear launch");
     else
         APS_HIP(aps::launch_linear_any_f32(x, weight, bias, y, rows, in_features, out_features, s),
                 "linear launch");
@@ -644,7 +644,6 @@ int aps_linear_multi(const float* x, int64_t rows, int32_t in_features, int32_t 
     if (!x || !weights || !ys) return fail(APS_ERR_ARG, "linear multi: NULL pointer");
     const float* ws[3] = {};
     const float* bs[3] = {};
-    bool fits = aps::linear_mfma_fits(rows, in_features, out_features[0]);
     for (int32_t j = 0; j < count; ++j) {
         ws[j] = weights[j];
         bs[j] = biases ? biases[j] : nullptr;
@@ -655,17 +654,10 @@ int aps_linear_multi(const float* x, int64_t rows, int32_t in_features, int32_t 
         if (ys[j] == x) return fail(APS_ERR_ARG, "linear multi: output %d aliases x", j);
         for (int32_t i = 0; i < j; ++i)
             if (ys[i] == ys[j]) return fail(APS_ERR_ARG, "linear multi: outputs %d and %d are the same array", i, j);
-        fits = fits && aps::linear_mfma_fits(rows, in_features, out_features[j]);
     }
     const hipStream_t s = static_cast<hipStream_t>(stream);
-    if (fits) {
-        APS_HIP(aps::launch_linear_mfma_multi(x, rows, in_features, count, ws, bs, ys, out_features, s),
-                "linear multi launch");
-    } else {
-        for (int32_t j = 0; j < count; ++j)
-            APS_HIP(aps::launch_linear_f32(x, ws[j], bs[j], ys[j], rows, in_features, out_features[j], s),
-                    "linear multi launch");
-    }
+    APS_HIP(aps::launch_linear_mfma_multi(x, rows, in_features, count, ws, bs, ys, out_features, s),
+            "linear multi launch");
     return APS_OK;
 }
 

@@ -271,18 +271,14 @@ hipError_t launch_linear_tc_multi(const uint16_t* xhi, const uint16_t* xlo, int 
                                   const float* const* bias, float* const* y, const int* out_f, int64_t rows, int in_f,
                                   bool all_terms, hipStream_t s);
 
-// y = x w^T (+ bias): fp32 FMA chain over k ascending per output, bias added
-// once (in_f % 16 == 0, out_f % 4 == 0).
-// fp32 Linear on the K = 1 fp32 MFMA (same bits as the FMA chain); shapes
-// with in_f % 32 == 0
+// y = x w^T (+ bias) on the fp32 MFMAs: the FMA chain over k ascending per
+// output, bias added once (in_f % 16 == 0, out_f % 4 == 0, 16-byte aligned).
 bool linear_mfma_fits(int64_t rows, int in_f, int out_f);
 hipError_t launch_linear_mfma_f32(const float* x, const float* w, const float* bias, float* y, int64_t rows,
                                   int in_f, int out_f, hipStream_t s);
 // count (1..3) outputs of one x in one grid, every shape linear_mfma_fits
 hipError_t launch_linear_mfma_multi(const float* x, int64_t rows, int in_f, int count, const float* const* w,
                                     const float* const* bias, float* const* y, const int* out_f, hipStream_t s);
-hipError_t launch_linear_f32(const float* x, const float* w, const float* bias, float* y, int64_t rows, int in_f,
-                             int out_f, hipStream_t s);
 // the same chains for any in_f, out_f and 4-byte alignment (SIMT, scalar loads)
 hipError_t launch_linear_any_f32(const float* x, const float* w, const float* bias, float* y, int64_t rows, int in_f,
                                  int out_f, hipStream_t s);

@@ -215,11 +215,13 @@ class DecoderLayer:
                                         (ctypes.c_int32 * cnt)(*[n for _, _, n in names]), int(self.tc_terms == 4),
                                         vp(*[_p(dst) for _, dst, _ in names]), stream))
         else:
-            # an output wide enough to fill the grid alone (q, o) by itself;
-            # the narrow ones (k and v) share one grid, so that no CU holds a
-            # third workgroup of one while others hold two
-            wide = [x for x in names if x[2] >= 2048]
-            narrow = [x for x in names if x[2] < 2048]
+            # few rows: every output of the input in one grid (q, k and v of
+            # 37 rows 27 us against 46 us as two launches, of 613 rows 126
+            # against 170).  Past 1,024 rows each grid fills the chip by
+            # itself and q alone, then k and v together, balance better
+            # (2,048 rows 361 us against 368, 10,240 rows 1775 against 1861)
+            wide = [x for x in names if x[2] >= 2048 and T > 1024]
+            narrow = [x for x in names if x[2] < 2048 or T <= 1024]
             for nm, dst, n in wide:
                 _call(L.aps_linear(_p(src), _p(self.w.proj[nm][0]), _p(self.w.proj[nm][1]), T, K, n, _p(dst),
                                    stream))
