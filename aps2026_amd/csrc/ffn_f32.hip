@@ -8,28 +8,51 @@
 //
 // These kernels keep exactly that arithmetic, so for fp32 weights the result
 // equals the CPU oracle bit for bit (the only libm call, exp in double, is
-// rounded to float afterwards).  They are SIMT kernels: each thread owns a
-// 4 x 4 block of outputs per operand and walks k in order; operand tiles are
-// staged k-major in LDS so the inner step is three ds_read_b128 + 32 FMAs.
-// This is the exactness path (config C1, fp32); the throughput path is
-// the bf16 MFMA kernel.
-#include "common.hpp"
+// rounded to float afterwards).  The chains run on the fp32 MFMAs, which give
+// the same bits (chain_mfma.hpp); k_linear_any, for Linear shapes those do not
+// take, is a SIMT kernel.
+#include "chain_mfma.hpp"
 
 namespace aps {
 namespace {
 
 constexpr int kBK = 16;
+constexpr int kFXcds = 8;   // XCDs of an MI355X
 
-__device__ inline bool locate_tile(const uint32_t* __restrict__ offsets, int E, int tile, int bm,
-                                   int& expert, uint32_t& m0, uint32_t& end) {
-    uint32_t lo, hi;
-    int incl;
-    const int total = wave_tile_scan(offsets, E, bm, lo, hi, incl);
-    if (tile >= total) return false;
-    const RowTile r = wave_find_tile(tile, bm, lo, hi, incl, E);
-    expert = r.expert;
-    m0 = r.m0;
-    end = r.end;
+// The work of a grouped kernel: expert e's rows in tiles of bm positions
+// against ncol column blocks.  Workgroup b runs on XCD b % 8, so the column
+// blocks (e, c) are dealt to the XCDs by (e ncol + c) % 8 and an XCD walks
+// them with the row tiles innermost: the row tiles that read the same weights
+// follow one another in one L2, and every XCD gets the same number of columns
+// (to one).  b / 8 counts an XCD's items; false past its last.
+struct GroupTile {
+    int expert, col;
+    uint32_t m0, end;
+};
+__device__ inline bool locate_group_tile(const uint32_t* __restrict__ offsets, int E, int bm, int ncol, GroupTile& g) {
+    const int lane = threadIdx.x & 63;
+    const int xcd = blockIdx.x % kFXcds, item = blockIdx.x / kFXcds;
+    const uint32_t lo = lane < E ? offsets[lane] : 0u;
+    uint32_t hi = __shfl_down(lo, 1);
+    if (lane == E - 1) hi = offsets[E];
+    const int nt = lane < E ? static_cast<int>((hi - lo + bm - 1) / bm) : 0;
+    const int c0 = (xcd + kFXcds * ncol - lane * (ncol % kFXcds)) & (kFXcds - 1);   // first column of this XCD
+    const int nc = c0 < ncol ? (ncol - 1 - c0) / kFXcds + 1 : 0;
+    int incl = nt * nc;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const int v = __shfl_up(incl, d);
+        if (lane >= d) incl += v;
+    }
+    const uint64_t m = __ballot(lane < E && incl > item);
+    if (m == 0) return false;
+    const int e = __ffsll(static_cast<unsigned long long>(m)) - 1;
+    const int i = item - (__shfl(incl, e) - __shfl(nt * nc, e));
+    const int ent = __shfl(nt, e);
+    g.expert = e;
+    g.col = __shfl(c0, e) + kFXcds * (i / ent);
+    g.m0 = __shfl(lo, e) + static_cast<uint32_t>(i % ent) * bm;
+    g.end = __shfl(hi, e);
     return true;
 }
 
@@ -40,126 +63,94 @@ __device__ inline float swiglu_exact(float g, float u) {
     return __fmul_rn(__fdiv_rn(g, __fadd_rn(1.0f, ex)), u);
 }
 
-// 64 rows x 64 intermediate columns of gate AND up per block.
-__global__ void __launch_bounds__(256)
+// act = SwiGLU of the gate and up chains, blocks of 16 RT WR positions.
+// CT = 2: a wave's two column tiles are w1's and w3's same 16 columns, so that
+// the gate and the up value meet in one lane; 16 WC columns per block.  CT = 1
+// (WC = 2): the first column of waves computes gate, the second up, and they
+// meet in LDS; 16 columns per block, half the chain length per wave.
+template <int RT, int CT, int WR, int WC, int S>
+__global__ void __launch_bounds__(64 * WR * WC)
 k_ffn_up_f32(const float* __restrict__ x, const uint32_t* __restrict__ offsets,
              const uint32_t* __restrict__ assignment_rows, const float* __restrict__ w1,
              const float* __restrict__ w3, float* __restrict__ act, int H, int F, int E) {
-    __shared__ __align__(16) float As[kBK][kF32BM];
-    __shared__ __align__(16) float Gs[kBK][kF32BN];
-    __shared__ __align__(16) float Us[kBK][kF32BN];
-
-    int e;
-    uint32_t m0, end;
-    if (!locate_tile(offsets, E, blockIdx.y, kF32BM, e, m0, end)) return;
-    const int n0 = blockIdx.x * kF32BN;
-    const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
-    // staging: one float4 of A, of w1 and of w3 per thread per k tile
-    const int sr = tid >> 2, sk = (tid & 3) * 4;
-    const uint32_t p = m0 + sr;
-    const bool a_ok = p < end;
-    const float* a_src = x + static_cast<int64_t>(a_ok ? assignment_rows[p] : 0) * H + sk;
-    const bool b_ok = n0 + sr < F;
-    const int64_t brow = static_cast<int64_t>(e) * F + (b_ok ? n0 + sr : 0);
-    const float* g_src = w1 + brow * H + sk;
-    const float* u_src = w3 + brow * H + sk;
-
-    float ga[4][4], ua[4][4];
+    using Ring = ChainRing<RT, CT, WR, WC, S>;
+    static_assert(CT == 2 || (CT == 1 && WC == 2), "gate and up tiles");
+    constexpr int kCols = CT == 2 ? 16 * WC : 16;
+    __shared__ __align__(16) uint8_t ring[Ring::kBytes];
+    GroupTile g;
+    if (!locate_group_tile(offsets, E, Ring::kARows, F / kCols, g)) return;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int n0 = g.col * kCols;
+    cf4_t acc[RT][CT];
+    Ring::run(
+        ring,
+        [&](int r) __attribute__((always_inline)) {
+            if (r < Ring::kARows) {   // positions past the end re-read the last one; their rows are not stored
+                const uint32_t p = g.m0 + r < g.end ? g.m0 + r : g.end - 1;
+                return x + static_cast<int64_t>(assignment_rows[p]) * H;
+            }
+            const int b = r - Ring::kARows, t = b / 16;
+            const int c = n0 + (CT == 2 ? (t / 2) * 16 : 0) + b % 16;
+            return (t % 2 ? w3 : w1) + (static_cast<int64_t>(g.expert) * F + c) * H;
+        },
+        H, acc);
+    const int row = (wave % WR) * 16 * RT + (lane & 15), c4 = 4 * (lane >> 4);
+    auto put = [&](int i, int col, const cf4_t& gate, const cf4_t& up) __attribute__((always_inline)) {
+        const uint32_t p = g.m0 + row + 16 * i;
+        if (p >= g.end) return;
+        cf4_t o;
 #pragma unroll
-    for (int r = 0; r < 4; ++r)
+        for (int v = 0; v < 4; ++v) o[v] = swiglu_exact(gate[v], up[v]);
+        *reinterpret_cast<cf4_t*>(act + static_cast<int64_t>(p) * F + col + c4) = o;
+    };
+    if constexpr (CT == 2) {
 #pragma unroll
-        for (int c = 0; c < 4; ++c) { ga[r][c] = 0.0f; ua[r][c] = 0.0f; }
-
-    for (int k0 = 0; k0 < H; k0 += kBK) {
-        const float4 av = a_ok ? *reinterpret_cast<const float4*>(a_src + k0) : make_float4(0.f, 0.f, 0.f, 0.f);
-        const float4 gv = b_ok ? *reinterpret_cast<const float4*>(g_src + k0) : make_float4(0.f, 0.f, 0.f, 0.f);
-        const float4 uv = b_ok ? *reinterpret_cast<const float4*>(u_src + k0) : make_float4(0.f, 0.f, 0.f, 0.f);
+        for (int i = 0; i < RT; ++i) put(i, n0 + (wave / WR) * 16, acc[i][0], acc[i][1]);
+    } else {
+        __syncthreads();   // every wave is done with the ring
+        auto* up = reinterpret_cast<cf4_t*>(ring) + (wave % WR) * RT * 64 + lane;
+        if (wave / WR == 1)
+#pragma unroll
+            for (int i = 0; i < RT; ++i) up[64 * i] = acc[i][0];
         __syncthreads();
-        As[sk + 0][sr] = av.x; As[sk + 1][sr] = av.y; As[sk + 2][sr] = av.z; As[sk + 3][sr] = av.w;
-        Gs[sk + 0][sr] = gv.x; Gs[sk + 1][sr] = gv.y; Gs[sk + 2][sr] = gv.z; Gs[sk + 3][sr] = gv.w;
-        Us[sk + 0][sr] = uv.x; Us[sk + 1][sr] = uv.y; Us[sk + 2][sr] = uv.z; Us[sk + 3][sr] = uv.w;
-        __syncthreads();
+        if (wave / WR == 0)
 #pragma unroll
-        for (int kk = 0; kk < kBK; ++kk) {
-            const float4 a = *reinterpret_cast<const float4*>(&As[kk][ty * 4]);
-            const float4 g = *reinterpret_cast<const float4*>(&Gs[kk][tx * 4]);
-            const float4 u = *reinterpret_cast<const float4*>(&Us[kk][tx * 4]);
-            const float ar[4] = {a.x, a.y, a.z, a.w};
-            const float gr[4] = {g.x, g.y, g.z, g.w};
-            const float ur[4] = {u.x, u.y, u.z, u.w};
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-#pragma unroll
-                for (int c = 0; c < 4; ++c) {
-                    ga[r][c] = __builtin_fmaf(ar[r], gr[c], ga[r][c]);
-                    ua[r][c] = __builtin_fmaf(ar[r], ur[c], ua[r][c]);
-                }
-        }
-    }
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const uint32_t pr = m0 + ty * 4 + r;
-        if (pr >= end) continue;
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            const int col = n0 + tx * 4 + c;
-            if (col < F) act[static_cast<int64_t>(pr) * F + col] = swiglu_exact(ga[r][c], ua[r][c]);
-        }
+            for (int i = 0; i < RT; ++i) put(i, n0, acc[i][0], up[64 * i]);
     }
 }
 
-// 64 rows x 64 hidden columns per block; K = F walked ascending.
-__global__ void __launch_bounds__(256)
+// y = act . w2^T, blocks of 16 RT WR positions x 16 CT WC hidden columns.
+template <int RT, int CT, int WR, int WC, int S>
+__global__ void __launch_bounds__(64 * WR * WC)
 k_ffn_down_f32(const float* __restrict__ act, const uint32_t* __restrict__ offsets,
                const float* __restrict__ w2, float* __restrict__ y, int H, int F, int E) {
-    __shared__ __align__(16) float As[kBK][kF32BM];
-    __shared__ __align__(16) float Bs[kBK][kF32BN];
-
-    int e;
-    uint32_t m0, end;
-    if (!locate_tile(offsets, E, blockIdx.y, kF32BM, e, m0, end)) return;
-    const int n0 = blockIdx.x * kF32BN;
-    const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
-    const int sr = tid >> 2, sk = (tid & 3) * 4;
-    const uint32_t p = m0 + sr;
-    const bool a_ok = p < end;
-    const float* a_src = act + static_cast<int64_t>(a_ok ? p : m0) * F + sk;
-    const bool b_ok = n0 + sr < H;
-    const float* b_src = w2 + (static_cast<int64_t>(e) * H + (b_ok ? n0 + sr : 0)) * F + sk;
-
-    float acc[4][4];
+    using Ring = ChainRing<RT, CT, WR, WC, S>;
+    __shared__ __align__(16) uint8_t ring[Ring::kBytes];
+    GroupTile g;
+    if (!locate_group_tile(offsets, E, Ring::kARows, H / Ring::kBRows, g)) return;
+    const int lane = threadIdx.x & 63;
+    const int wave = WR * WC > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
+    const int n0 = g.col * Ring::kBRows;
+    cf4_t acc[RT][CT];
+    Ring::run(
+        ring,
+        [&](int r) __attribute__((always_inline)) {
+            if (r < Ring::kARows) {
+                const uint32_t p = g.m0 + r < g.end ? g.m0 + r : g.end - 1;
+                return act + static_cast<int64_t>(p) * F;
+            }
+            return w2 + (static_cast<int64_t>(g.expert) * H + n0 + r - Ring::kARows) * F;
+        },
+        F, acc);
 #pragma unroll
-    for (int r = 0; r < 4; ++r)
+    for (int i = 0; i < RT; ++i) {
+        const uint32_t p = g.m0 + (wave % WR) * 16 * RT + 16 * i + (lane & 15);
+        if (p >= g.end) continue;
 #pragma unroll
-        for (int c = 0; c < 4; ++c) acc[r][c] = 0.0f;
-
-    for (int k0 = 0; k0 < F; k0 += kBK) {
-        const float4 av = a_ok ? *reinterpret_cast<const float4*>(a_src + k0) : make_float4(0.f, 0.f, 0.f, 0.f);
-        const float4 bv = b_ok ? *reinterpret_cast<const float4*>(b_src + k0) : make_float4(0.f, 0.f, 0.f, 0.f);
-        __syncthreads();
-        As[sk + 0][sr] = av.x; As[sk + 1][sr] = av.y; As[sk + 2][sr] = av.z; As[sk + 3][sr] = av.w;
-        Bs[sk + 0][sr] = bv.x; Bs[sk + 1][sr] = bv.y; Bs[sk + 2][sr] = bv.z; Bs[sk + 3][sr] = bv.w;
-        __syncthreads();
-#pragma unroll
-        for (int kk = 0; kk < kBK; ++kk) {
-            const float4 a = *reinterpret_cast<const float4*>(&As[kk][ty * 4]);
-            const float4 b = *reinterpret_cast<const float4*>(&Bs[kk][tx * 4]);
-            const float ar[4] = {a.x, a.y, a.z, a.w};
-            const float br[4] = {b.x, b.y, b.z, b.w};
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-#pragma unroll
-                for (int c = 0; c < 4; ++c) acc[r][c] = __builtin_fmaf(ar[r], br[c], acc[r][c]);
-        }
-    }
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const uint32_t pr = m0 + ty * 4 + r;
-        if (pr >= end) continue;
-        const int col = n0 + tx * 4;
-        if (col + 3 < H)
-            *reinterpret_cast<float4*>(y + static_cast<int64_t>(pr) * H + col) =
-                make_float4(acc[r][0], acc[r][1], acc[r][2], acc[r][3]);
+        for (int j = 0; j < CT; ++j)
+            *reinterpret_cast<cf4_t*>(y + static_cast<int64_t>(p) * H + n0 + (wave / WR) * 16 * CT + 16 * j +
+                                      4 * (lane >> 4)) = acc[i][j];
     }
 }
 
@@ -245,29 +236,50 @@ hipError_t launch_linear_any_f32(const float* x, const float* w, const float* bi
     return hipGetLastError();
 }
 
+// Rows per block by the mean number of positions per expert.
+#define APS_GROUPED(KERNEL, RT, CT, WR, WC, S, NCOL, ...)                                                        \
+    do {                                                                                                          \
+        const int64_t t = max_row_tiles(2 * rows, 16 * RT * WR, experts) * ceil_div(NCOL, kFXcds) * kFXcds;        \
+        hipLaunchKernelGGL((KERNEL<RT, CT, WR, WC, S>), dim3(static_cast<unsigned>(t)), dim3(64 * WR * WC), 0, s, \
+                           __VA_ARGS__, hidden, ffn, experts);                                                    \
+        return hipGetLastError();                                                                                 \
+    } while (0)
+
 hipError_t launch_ffn_up_f32(const float* x, const uint32_t* offsets,
                              const uint32_t* assignment_rows, const float* w1,
                              const float* w3, float* act, int64_t rows, int hidden, int ffn,
                              int experts, hipStream_t s) {
     if (rows <= 0) return hipSuccess;
-    if (hidden % kBK != 0 || ffn % 4 != 0) return hipErrorInvalidValue;
-    const dim3 grid(static_cast<unsigned>(ceil_div(ffn, kF32BN)),
-                    static_cast<unsigned>(max_row_tiles(2 * rows, kF32BM, experts)));
-    hipLaunchKernelGGL(k_ffn_up_f32, grid, dim3(256), 0, s, x, offsets, assignment_rows, w1, w3,
-                       act, hidden, ffn, experts);
-    return hipGetLastError();
+    if (hidden % kBK != 0 || ffn % 64 != 0) return hipErrorInvalidValue;
+    const int64_t mean = ceil_div(2 * rows, experts);
+    // us at hidden 4096, ffn 448, 16 experts, for 1 / 43 / 512 / 1,024 / 2,048
+    // tokens; the SIMT kernel before these took 468 to 476 us up to 512
+    //   16 rows x 16 columns, gate and up on two waves   23  52 136 225 428
+    //   32 x 16, the same                                26  53 114 177 332
+    //   32 x 32, gate and up in a lane                   41  57 121 165 307
+    //   64 x 32                                          66  78 141 203 279
+    // Few rows are bound by the length of a chain or by the weights (235 MB,
+    // 48 us), many by the MFMAs on rows that pad each expert's last tile.
+    if (mean <= 8) APS_GROUPED(k_ffn_up_f32, 1, 1, 1, 2, 8, ffn / 16, x, offsets, assignment_rows, w1, w3, act);
+    if (mean <= 96) APS_GROUPED(k_ffn_up_f32, 1, 1, 2, 2, 4, ffn / 16, x, offsets, assignment_rows, w1, w3, act);
+    if (mean <= 192) APS_GROUPED(k_ffn_up_f32, 1, 2, 2, 2, 4, ffn / 32, x, offsets, assignment_rows, w1, w3, act);
+    APS_GROUPED(k_ffn_up_f32, 2, 2, 2, 2, 4, ffn / 32, x, offsets, assignment_rows, w1, w3, act);
 }
 
 hipError_t launch_ffn_down_f32(const float* act, const uint32_t* offsets, const float* w2,
                                float* y, int64_t rows, int hidden, int ffn, int experts,
                                hipStream_t s) {
     if (rows <= 0) return hipSuccess;
-    if (ffn % kBK != 0 || hidden % kF32BN != 0) return hipErrorInvalidValue;
-    const dim3 grid(static_cast<unsigned>(hidden / kF32BN),
-                    static_cast<unsigned>(max_row_tiles(2 * rows, kF32BM, experts)));
-    hipLaunchKernelGGL(k_ffn_down_f32, grid, dim3(256), 0, s, act, offsets, w2, y, hidden, ffn,
-                       experts);
-    return hipGetLastError();
+    if (ffn % kBK != 0 || hidden % 64 != 0) return hipErrorInvalidValue;
+    const int64_t mean = ceil_div(2 * rows, experts);
+    // as above; the SIMT kernel took 63 us for 43 tokens, 89 for 512
+    //   16 rows x 64 columns    8  25  60 107 199
+    //   32 x 64                 9  27  54  92 175
+    //   64 x 64                12  39  58  93 160
+    if (mean <= 16) APS_GROUPED(k_ffn_down_f32, 1, 2, 1, 2, 4, hidden / 64, act, offsets, w2, y);
+    if (mean <= 192) APS_GROUPED(k_ffn_down_f32, 1, 2, 2, 2, 4, hidden / 64, act, offsets, w2, y);
+    APS_GROUPED(k_ffn_down_f32, 2, 2, 2, 2, 4, hidden / 64, act, offsets, w2, y);
 }
+#undef APS_GROUPED
 
 }  // namespace aps

@@ -5,7 +5,7 @@ import pytest
 import torch
 
 import oracle
-from aps2026_amd import attention
+from aps2026_amd import attention, moe, synth
 
 pytestmark = pytest.mark.gpu
 
@@ -35,3 +35,29 @@ def test_linear_block_and_stage_edges(gpu_device, rows, k, n):
     b = (0.1 * rng.standard_normal(n)).astype(np.float32)
     got = attention.linear_gpu(dev(x, gpu_device), dev(w, gpu_device), dev(b, gpu_device)).cpu().numpy()
     np.testing.assert_array_equal(got.view(np.uint32), oracle.linear(x, w, b).view(np.uint32))
+
+
+# tokens and experts on both sides of the dispatch's lines (8, 96 and 192
+# positions per expert for w1||w3, 16 and 192 for w2), ffn widths that deal an
+# uneven number of column blocks to the XCDs, k = 64 .. 512 through the rings
+@pytest.mark.parametrize("T,E,H,F", [(5, 16, 256, 64), (64, 16, 512, 192), (65, 16, 256, 64), (130, 16, 512, 320),
+                                     (97, 2, 256, 192), (192, 2, 512, 64), (193, 2, 256, 448), (700, 3, 256, 64),
+                                     (900, 3, 512, 192)])
+def test_fp32_experts_block_edges(gpu_device, T, E, H, F):
+    note(f"fp32 experts T={T} E={E} H={H} F={F}")
+    inp = synth.make_moe_inputs(T=T, H=H, E=E, F=F, dtype="f32", seed=T + E + F)
+    d = lambda a: [dev(a[e], gpu_device) for e in range(E)]
+    w = moe.register_moe_weights_gpu(d(inp.w1), d(inp.w2), d(inp.w3), torch.float32)
+    moe.moe_forward_gpu(dev(inp.x, gpu_device), dev(inp.gate, gpu_device), w)
+    plan = w.plan_views(T)
+    plan["y"].fill_(float("nan"))   # a row or column that no block writes stays NaN
+    plan["act"].fill_(float("nan"))
+    out = moe.moe_forward_gpu(dev(inp.x, gpu_device), dev(inp.gate, gpu_device), w)
+    ref = oracle.reference_path(inp.x, inp.gate, inp.w1, inp.w3, inp.w2)
+    y, got = plan["y"].cpu().numpy(), out.cpu().numpy()
+    w.release()
+    # the chains are exact; SiLU's exp in double is the GPU's against glibc's,
+    # at most the last fp32 bit of a hidden value: 2^-23 of it, row by row
+    for a, b in ((y, ref["y"]), (got, ref["out"])):
+        err = np.linalg.norm(a.astype(np.float64) - b, axis=1) / np.linalg.norm(b.astype(np.float64), axis=1)
+        assert err.max() <= 2.0 ** -23
