@@ -14,175 +14,281 @@
 // root, so every other operation is rounded on its own).
 //
 // gfx950 mapping.  The sums are dependent chains of h additions: their length,
-// not bandwidth, sets the time, and only one lane can own a row.  A wave owns
-// 4 rows (lanes 0..3 run their chains), so T = 4096 rows make 1024 one-wave
-// workgroups, one per SIMD.  The whole wave stages the rows through LDS in
-// chunks of 256 columns: per row one coalesced 1 KB load (64 lanes x 16 B) of
-// x (and of the residual, added here and stored back to x), then one 16-byte
-// LDS write per lane; the chain lanes read their row four values at a time
-// (rows padded by 16 bytes: distinct bank groups).  Loads run kLnDepth chunks
-// ahead in a register ring (a chunk's chain, ~0.6 us, is shorter than a load's
-// latency), always to a valid address (the last chunk is re-read past the
-// end) so that the compiler can count the loads in flight.
-//   pass 1: stage x (+ residual), mean chain;
-//   pass 2: stage v again (now in x), variance chain;
-//   pass 3: y for the 4 rows, coalesced (w and b loaded with each chunk).
+// not bandwidth, sets the time, and only one lane can hold a row's sum.  A row
+// belongs to the 16 lanes of a DPP row (a wave owns 4 rows): lane i holds the
+// elements 16 i .. 16 i + 15 of each 256-column chunk, and the running sum
+// walks through the lanes.  Every lane runs the same 16 additions on its own
+// registers 16 times over; before each round the accumulators rotate one lane
+// (DPP row_ror:1, folded into the add in pass 1), so after round i lane i's
+// accumulator is the sum up to its last element and the others' are unused.
+// A step is one vector instruction on registers, with no LDS reads and no
+// broadcasts, and the deviation v - mean, elementwise, is taken 16 lanes at a
+// time before the variance chain.
+//   A row of 16 chunks (h = 4096) stays in its lanes' registers from the first
+// load to the last store (256 VGPRs, one wave per SIMD), so x is read once;
+// other widths stream the chunks again for each pass.
+//   Bound by the two chains up to one wave per SIMD (4,096 rows), by the row
+// traffic with them past that.  Measured at h = 4096 (with the residual):
+// 43 rows 27 (29) us, 4,096 rows 39 (52), 10,240 rows 99 (149: 4.5 TB/s).
+// One lane per row reading staged rows from LDS four values at a time, three
+// passes over memory, took 64 (65), 78 (80), 162 (193) us; loading and storing
+// in the chains' layout (64 bytes apart across lanes) 28 (29), 49 (69), 123
+// (182) us.
 #include "common.hpp"
 
 namespace aps {
 namespace {
 
-constexpr int kLnRows = 4;      // rows per wave (chain lanes)
-constexpr int kLnChunk = 256;   // columns per staged chunk: 1 KB of fp32 per row
-constexpr int kLnPitch = kLnChunk + 4;  // staged row pitch in floats (16-byte pad)
-constexpr int kLnMaxDepth = 4;  // chunks of loads in flight (NC % depth == 0)
+constexpr int kLnRows = 4;       // rows per wave, one per 16-lane DPP row
+constexpr int kLnElems = 16;     // consecutive elements per lane and chunk
+constexpr int kLnChunk = 256;    // columns per chunk (16 lanes x 16 elements)
+constexpr int kLnResident = 16;  // chunks of a row that stays in registers
+constexpr int kLnAhead = 4;      // chunks of loads in flight
 
 typedef float lf4 __attribute__((ext_vector_type(4)));
 
-template <bool ADD, int kLnDepth>
+// lane i of each 16-lane row <- lane i - 1 (lane 0 <- lane 15)
+__device__ inline float ln_ror1(float v) {
+    const int i = __builtin_bit_cast(int, v);
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(i, i, 0x121, 0xF, 0xF, true));
+}
+// lane 15's value in every lane of its row
+__device__ inline float ln_last(float v) {
+    const int i = __builtin_bit_cast(int, v);
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(i, i, 0x15F, 0xF, 0xF, true));
+}
+
+struct LnChunk {
+    lf4 q[kLnElems / 4];
+};
+
+// The chains over one chunk: on entry lane 15 (or, at the first chunk, every
+// lane) holds the sum so far, on exit lane 15 holds the new one.
+__device__ inline float ln_sum(float acc, const LnChunk& v) {
+#pragma unroll 4
+    for (int i = 0; i < 16; ++i) {
+        acc = __fadd_rn(ln_ror1(acc), v.q[0][0]);
+#pragma unroll
+        for (int e = 1; e < kLnElems; ++e) acc = __fadd_rn(acc, v.q[e / 4][e % 4]);
+    }
+    return acc;
+}
+__device__ inline float ln_sum_sq(float acc, const LnChunk& t) {
+#pragma unroll 4
+    for (int i = 0; i < 16; ++i) {
+        acc = ln_ror1(acc);
+#pragma unroll
+        for (int e = 0; e < kLnElems; ++e) acc = __fmaf_rn(t.q[e / 4][e % 4], t.q[e / 4][e % 4], acc);
+    }
+    return acc;
+}
+
+__device__ inline void ln_load(LnChunk& d, const float* src) {
+#pragma unroll
+    for (int p = 0; p < kLnElems / 4; ++p) d.q[p] = reinterpret_cast<const lf4*>(src)[p];
+}
+__device__ inline void ln_store(float* dst, const LnChunk& v) {
+#pragma unroll
+    for (int p = 0; p < kLnElems / 4; ++p) reinterpret_cast<lf4*>(dst)[p] = v.q[p];
+}
+__device__ inline void ln_add(LnChunk& v, const LnChunk& r) {
+#pragma unroll
+    for (int p = 0; p < kLnElems / 4; ++p)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) v.q[p][k] = __fadd_rn(v.q[p][k], r.q[p][k]);
+}
+__device__ inline void ln_deviation(LnChunk& v, float mean) {
+#pragma unroll
+    for (int p = 0; p < kLnElems / 4; ++p)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) v.q[p][k] = __fsub_rn(v.q[p][k], mean);
+}
+// y = fma(t * inv, w, b)
+__device__ inline void ln_scale(LnChunk& t, float inv, const LnChunk& w, const LnChunk& b) {
+#pragma unroll
+    for (int p = 0; p < kLnElems / 4; ++p)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) t.q[p][k] = __fmaf_rn(__fmul_rn(t.q[p][k], inv), w.q[p][k], b.q[p][k]);
+}
+__device__ inline float ln_inv(float var, int h, float eps) {
+    // sqrtf, not __fsqrt_rn: under -fhip-fp32-correctly-rounded-divide-sqrt
+    // sqrtf is correctly rounded (v_sqrt_f32 plus a neighbour check),
+    // while __fsqrt_rn lowers to the bare v_sqrt_f32, off by an ulp at
+    // times (rows of a GPU test disagreed with the oracle by one ulp)
+    return __fdiv_rn(1.0f, sqrtf(__fadd_rn(__fdiv_rn(var, static_cast<float>(h)), eps)));
+}
+
+// This lane's place: its row (rows past the end load the last one and store
+// nothing) and its first element in every chunk.
+struct LnLane {
+    int64_t at;
+    bool valid;
+    int col;
+    __device__ LnLane(int64_t rows, int h) {
+        const int lane = threadIdx.x;
+        const int64_t r = static_cast<int64_t>(blockIdx.x) * kLnRows + (lane >> 4);
+        valid = r < rows;
+        col = kLnElems * (lane & 15);
+        at = (valid ? r : rows - 1) * static_cast<int64_t>(h) + col;
+    }
+};
+
+// h = 4096: the row in registers throughout.  Memory is read and written whole
+// 1 KB row chunks at a time (lane s holds 16 bytes of each of the 4 rows); LDS
+// turns a chunk between that layout and the chains' (64 consecutive bytes of
+// one row per lane).  Lane s's 16 bytes are columns io .. io + 3 of the chunk,
+// slot s; the piece p of chain lane L lies in slot 4 L + (p ^ (L / 4)), so that
+// 16 chain lanes read 16 different bank groups.
+template <bool ADD>
+__global__ void __launch_bounds__(64, 1)
+k_layer_norm_resident(float* __restrict__ x, const float* __restrict__ residual, const float* __restrict__ w,
+                      const float* __restrict__ b, float* __restrict__ y, int64_t rows, float eps) {
+    constexpr int NC = kLnResident, h = NC * kLnChunk;
+    __shared__ lf4 turn[2][kLnRows][64];
+    const int s = threadIdx.x, L = s & 15;
+    const int io = 16 * (s >> 2) + 4 * ((s & 3) ^ ((s >> 4) & 3));
+    const int64_t r0 = static_cast<int64_t>(blockIdx.x) * kLnRows;
+    const int nr = rows - r0 < kLnRows ? static_cast<int>(rows - r0) : kLnRows;   // wave-uniform
+    int64_t at[kLnRows];   // rows past the end load the last one and store nothing
+#pragma unroll
+    for (int k = 0; k < kLnRows; ++k) at[k] = (r0 + (k < nr ? k : nr - 1)) * h + io;
+    auto ld = [](const float* p) __attribute__((always_inline)) { return *reinterpret_cast<const lf4*>(p); };
+
+    LnChunk v[NC];
+    lf4 xs[kLnAhead][kLnRows], rs[ADD ? kLnAhead : 1][kLnRows];
+    auto load = [&](int c) __attribute__((always_inline)) {
+#pragma unroll
+        for (int k = 0; k < kLnRows; ++k) {
+            xs[c % kLnAhead][k] = ld(x + at[k] + c * kLnChunk);
+            if (ADD) rs[c % kLnAhead][k] = ld(residual + at[k] + c * kLnChunk);
+        }
+        __builtin_amdgcn_sched_barrier(0);   // chunk order, so that a chunk's wait leaves the later ones in flight
+    };
+    // chunk c as it was loaded (+ residual, written back to x) into its chain lanes' registers
+    auto take = [&](int c) __attribute__((always_inline)) {
+#pragma unroll
+        for (int k = 0; k < kLnRows; ++k) {
+            lf4 u = xs[c % kLnAhead][k];
+            if (ADD) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j) u[j] = __fadd_rn(u[j], rs[c % kLnAhead][k][j]);
+                if (k < nr) *reinterpret_cast<lf4*>(x + at[k] + c * kLnChunk) = u;
+            }
+            turn[c & 1][k][s] = u;
+        }
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int p = 0; p < 4; ++p) v[c].q[p] = turn[c & 1][s >> 4][4 * L + (p ^ (L >> 2))];
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+    };
+#pragma unroll
+    for (int c = 0; c < kLnAhead; ++c) load(c);
+    take(0);
+    float acc = 0.0f;
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+        if (c + kLnAhead < NC) load(c + kLnAhead);
+        if (c + 1 < NC) take(c + 1);
+        acc = ln_sum(acc, v[c]);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    const float mean = __fdiv_rn(ln_last(acc), static_cast<float>(h));
+    // w and b in the loads' layout, the first chunks' under the variance chain
+    lf4 wv[kLnAhead], bv[kLnAhead];
+    auto load_wb = [&](int c) __attribute__((always_inline)) {
+        wv[c % kLnAhead] = ld(w + c * kLnChunk + io);
+        bv[c % kLnAhead] = ld(b + c * kLnChunk + io);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+#pragma unroll
+    for (int c = 0; c < kLnAhead; ++c) load_wb(c);
+    float var = 0.0f;
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+        ln_deviation(v[c], mean);
+        var = ln_sum_sq(var, v[c]);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    const float inv_row = ln_inv(ln_last(var), h, eps);
+    float inv[kLnRows];
+#pragma unroll
+    for (int k = 0; k < kLnRows; ++k)
+        inv[k] = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, inv_row), 16 * k));
+    // chunk c of t into the loads' layout, one chunk ahead of its use
+    lf4 t[2][kLnRows];
+    auto turn_back = [&](int c) __attribute__((always_inline)) {
+#pragma unroll
+        for (int p = 0; p < 4; ++p) turn[c & 1][s >> 4][4 * L + (p ^ (L >> 2))] = v[c].q[p];
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int k = 0; k < kLnRows; ++k) t[c & 1][k] = turn[c & 1][k][s];
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    turn_back(0);
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+        if (c + 1 < NC) turn_back(c + 1);
+#pragma unroll
+        for (int k = 0; k < kLnRows; ++k) {
+            lf4 o;
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                o[j] = __fmaf_rn(__fmul_rn(t[c & 1][k][j], inv[k]), wv[c % kLnAhead][j], bv[c % kLnAhead][j]);
+            if (k < nr) *reinterpret_cast<lf4*>(y + at[k] + c * kLnChunk) = o;
+        }
+        if (c + kLnAhead < NC) load_wb(c + kLnAhead);
+    }
+}
+
+// Any h (a multiple of 256): the chunks are read again for each pass, two
+// ahead.
+template <bool ADD>
 __global__ void __launch_bounds__(64)
 k_layer_norm(float* __restrict__ x, const float* __restrict__ residual, const float* __restrict__ w,
              const float* __restrict__ b, float* __restrict__ y, int64_t rows, int h, float eps) {
-    __shared__ __align__(16) float stage[2][kLnRows][kLnPitch];
-    __shared__ float s_mean[kLnRows], s_inv[kLnRows];
-    const int lane = threadIdx.x;
-    const int64_t r0 = static_cast<int64_t>(blockIdx.x) * kLnRows;
-    const int nr = rows - r0 < kLnRows ? static_cast<int>(rows - r0) : kLnRows;  // wave-uniform
+    const LnLane l(rows, h);
     const int NC = h / kLnChunk;
-    const bool chain = lane < nr;
-    // lane's 16-byte piece of row rr, chunk c.  Rows past the end map to the
-    // last row (its loads and stores repeat that row's, with equal data), and
-    // chunks past the end to the last chunk (loaded ahead, never used), so
-    // every load and store is unconditional and the compiler counts them.
-    auto piece = [&](const float* base, int rr, int c) -> const lf4* {
-        const int64_t row = r0 + (rr < nr ? rr : nr - 1);
-        const int cc = c < NC ? c : NC - 1;
-        return reinterpret_cast<const lf4*>(base + row * static_cast<int64_t>(h) + cc * kLnChunk) + lane;
-    };
-
-    lf4 xs[kLnDepth][kLnRows], rs[kLnDepth][kLnRows];
-    auto load = [&](int slot_dummy, lf4 (&xd)[kLnRows], lf4 (&rd)[kLnRows], int c, bool with_residual) {
-        (void)slot_dummy;
-#pragma unroll
-        for (int rr = 0; rr < kLnRows; ++rr) {
-            xd[rr] = *piece(x, rr, c);
-            if (ADD && with_residual) rd[rr] = *piece(residual, rr, c);
+    // f(c, chunk c of x); chunks past the end re-read the last one
+    auto each = [&](auto f) __attribute__((always_inline)) {
+        LnChunk v[2];
+        auto load = [&](LnChunk& d, int c) __attribute__((always_inline)) {
+            ln_load(d, x + l.at + (c < NC ? c : NC - 1) * kLnChunk);
+        };
+        load(v[0], 0);
+        for (int c = 0; c < NC; c += 2) {
+            load(v[1], c + 1);
+            f(c, v[0]);
+            load(v[0], c + 2);
+            if (c + 1 < NC) f(c + 1, v[1]);
         }
     };
-    // v = x (+ residual) into LDS buffer c % 2; pass 1 also writes v back to x
-    auto put = [&](const lf4 (&xd)[kLnRows], const lf4 (&rd)[kLnRows], int c, bool with_residual) {
-#pragma unroll
-        for (int rr = 0; rr < kLnRows; ++rr) {
-            lf4 v = xd[rr];
-            if (ADD && with_residual) {
-                v = lf4{__fadd_rn(v[0], rd[rr][0]), __fadd_rn(v[1], rd[rr][1]), __fadd_rn(v[2], rd[rr][2]),
-                        __fadd_rn(v[3], rd[rr][3])};
-                *const_cast<lf4*>(piece(x, rr, c)) = v;
-            }
-            *reinterpret_cast<lf4*>(&stage[c & 1][rr][4 * lane]) = v;
+    float acc = 0.0f;
+    each([&](int c, LnChunk& v) __attribute__((always_inline)) {
+        if (ADD) {
+            LnChunk r;
+            ln_load(r, residual + l.at + c * kLnChunk);
+            ln_add(v, r);
+            if (l.valid) ln_store(x + l.at + c * kLnChunk, v);
         }
-        // every lane stages its pieces, then the chain lanes read whole
-        // rows: the wave barrier keeps the compiler from running the two on
-        // divergent paths one after the other (a data race between lanes)
-        __builtin_amdgcn_wave_barrier();
-    };
-    // one staged pass over the rows; step(acc, v) folds four values in order
-    auto pass = [&](bool with_residual, auto step) {
-        float acc = 0.0f;
-#pragma unroll
-        for (int d = 0; d < kLnDepth; ++d) {
-            load(d, xs[d], rs[d], d, with_residual);
-            // keep the chunks' loads in order, so that a chunk's wait leaves
-            // every later chunk in flight
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        for (int c0 = 0; c0 < NC; c0 += kLnDepth) {
-#pragma unroll
-            for (int d = 0; d < kLnDepth; ++d) {
-                const int c = c0 + d;
-                put(xs[d], rs[d], c, with_residual);
-                load(d, xs[d], rs[d], c + kLnDepth, with_residual);
-                __builtin_amdgcn_sched_barrier(0);
-                if (chain) {
-                    const float* row = &stage[c & 1][lane][0];
-#pragma unroll 8
-                    for (int j = 0; j < kLnChunk; j += 4) acc = step(acc, *reinterpret_cast<const lf4*>(row + j));
-                }
-            }
-        }
-        return acc;
-    };
-
-    // pass 1: the mean (ascending adds)
-    const float sum = pass(ADD, [](float a, lf4 v) {
-        a = __fadd_rn(a, v[0]);
-        a = __fadd_rn(a, v[1]);
-        a = __fadd_rn(a, v[2]);
-        return __fadd_rn(a, v[3]);
+        acc = ln_sum(acc, v);
     });
-    const float mean = __fdiv_rn(sum, static_cast<float>(h));
-    // pass 2: the variance (fused chain of squared deviations); v is in x now,
-    // once this wave's stores of pass 1 have completed
-    if (ADD) __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
-    const float var = pass(false, [mean](float a, lf4 v) {
-        float t = __fsub_rn(v[0], mean);
-        a = __fmaf_rn(t, t, a);
-        t = __fsub_rn(v[1], mean);
-        a = __fmaf_rn(t, t, a);
-        t = __fsub_rn(v[2], mean);
-        a = __fmaf_rn(t, t, a);
-        t = __fsub_rn(v[3], mean);
-        return __fmaf_rn(t, t, a);
+    const float mean = __fdiv_rn(ln_last(acc), static_cast<float>(h));
+    float var = 0.0f;
+    each([&](int c, LnChunk& v) __attribute__((always_inline)) {
+        ln_deviation(v, mean);
+        var = ln_sum_sq(var, v);
     });
-    if (chain) {
-        s_mean[lane] = mean;
-        // sqrtf, not __fsqrt_rn: under -fhip-fp32-correctly-rounded-divide-sqrt
-        // sqrtf is correctly rounded (v_sqrt_f32 plus a neighbour check),
-        // while __fsqrt_rn lowers to the bare v_sqrt_f32, off by an ulp at
-        // times (rows of a GPU test disagreed with the oracle by one ulp)
-        s_inv[lane] = __fdiv_rn(1.0f, sqrtf(__fadd_rn(__fdiv_rn(var, static_cast<float>(h)), eps)));
-    }
-    __syncthreads();
-    float m[kLnRows], iv[kLnRows];
-#pragma unroll
-    for (int rr = 0; rr < kLnRows; ++rr) {
-        m[rr] = s_mean[rr];
-        iv[rr] = s_inv[rr];
-    }
-
-    // pass 3: y, coalesced, loads kLnDepth chunks ahead
-    lf4 wv[kLnDepth], bv[kLnDepth];
-    auto load_wb = [&](int d, int c) {
-        const int cc = c < NC ? c : NC - 1;
-        wv[d] = reinterpret_cast<const lf4*>(w + cc * kLnChunk)[lane];
-        bv[d] = reinterpret_cast<const lf4*>(b + cc * kLnChunk)[lane];
-    };
-#pragma unroll
-    for (int d = 0; d < kLnDepth; ++d) {
-        load(d, xs[d], rs[d], d, false);
-        load_wb(d, d);
-        __builtin_amdgcn_sched_barrier(0);
-    }
-    for (int c0 = 0; c0 < NC; c0 += kLnDepth) {
-#pragma unroll
-        for (int d = 0; d < kLnDepth; ++d) {
-            const int c = c0 + d;
-            lf4 o[kLnRows];
-#pragma unroll
-            for (int rr = 0; rr < kLnRows; ++rr)
-#pragma unroll
-                for (int k = 0; k < 4; ++k)
-                    o[rr][k] = __fmaf_rn(__fmul_rn(__fsub_rn(xs[d][rr][k], m[rr]), iv[rr]), wv[d][k], bv[d][k]);
-            load(d, xs[d], rs[d], c + kLnDepth, false);
-            load_wb(d, c + kLnDepth);
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int rr = 0; rr < kLnRows; ++rr) {
-                const int64_t row = r0 + (rr < nr ? rr : nr - 1);
-                *reinterpret_cast<lf4*>(y + row * static_cast<int64_t>(h) + c * kLnChunk + 4 * lane) = o[rr < nr ? rr : nr - 1];
-            }
-        }
-    }
+    const float inv = ln_inv(ln_last(var), h, eps);
+    each([&](int c, LnChunk& v) __attribute__((always_inline)) {
+        LnChunk wv, bv;
+        ln_load(wv, w + c * kLnChunk + l.col);
+        ln_load(bv, b + c * kLnChunk + l.col);
+        ln_deviation(v, mean);
+        ln_scale(v, inv, wv, bv);
+        if (l.valid) ln_store(y + l.at + c * kLnChunk, v);
+    });
 }
 
 }  // namespace
@@ -192,21 +298,16 @@ hipError_t launch_layer_norm(float* x, const float* residual, const float* weigh
     if (rows <= 0) return hipSuccess;
     if (hidden <= 0 || hidden % kLnChunk != 0) return hipErrorInvalidValue;
     const dim3 grid(static_cast<unsigned>(ceil_div(rows, kLnRows)));
-    const int nc = hidden / kLnChunk;
-    const int depth = nc % kLnMaxDepth == 0 ? kLnMaxDepth : nc % 2 == 0 ? 2 : 1;
-#define APS_LN_LAUNCH(ADD, D)                                                                          \
-    hipLaunchKernelGGL((k_layer_norm<ADD, D>), grid, dim3(64), 0, s, x, residual, weight, bias, y, rows, \
-                       hidden, eps)
-    if (residual) {
-        if (depth == 4) APS_LN_LAUNCH(true, 4);
-        else if (depth == 2) APS_LN_LAUNCH(true, 2);
-        else APS_LN_LAUNCH(true, 1);
+    if (hidden == kLnResident * kLnChunk) {
+        if (residual)
+            hipLaunchKernelGGL(k_layer_norm_resident<true>, grid, dim3(64), 0, s, x, residual, weight, bias, y, rows, eps);
+        else
+            hipLaunchKernelGGL(k_layer_norm_resident<false>, grid, dim3(64), 0, s, x, residual, weight, bias, y, rows, eps);
+    } else if (residual) {
+        hipLaunchKernelGGL(k_layer_norm<true>, grid, dim3(64), 0, s, x, residual, weight, bias, y, rows, hidden, eps);
     } else {
-        if (depth == 4) APS_LN_LAUNCH(false, 4);
-        else if (depth == 2) APS_LN_LAUNCH(false, 2);
-        else APS_LN_LAUNCH(false, 1);
+        hipLaunchKernelGGL(k_layer_norm<false>, grid, dim3(64), 0, s, x, residual, weight, bias, y, rows, hidden, eps);
     }
-#undef APS_LN_LAUNCH
     return hipGetLastError();
 }
 

@@ -51,6 +51,23 @@ def test_layer_norm_bit_exact(gpu_device, rows, h, add):
     np.testing.assert_array_equal(xd.cpu().numpy().view(np.uint32), (want_v if add else x).view(np.uint32))
 
 
+@pytest.mark.parametrize("rows,h", [(2, 4096), (4, 4096), (6, 512), (3, 768)])
+def test_layer_norm_row_groups(gpu_device, rows, h):
+    """Rows per wave: partly and exactly filled waves, an even and an odd
+    number of streamed 256-column chunks; with the residual, values of large
+    and small magnitude so that the order of the sums shows.  Bit-exact."""
+    note(f"layer norm groups rows={rows} h={h}")
+    x, r, w, b = _inputs(rows, h, rows + h)
+    x *= np.exp2(np.random.default_rng(h).integers(-12, 13, (rows, h))).astype(np.float32)
+    xd, rd, wd, bd = (_dev(a, gpu_device) for a in (x, r, w, b))
+    y = torch.empty_like(xd)
+    moe.add_layer_norm_gpu(xd, rd, wd, bd, moe.NORM_EPS, y)
+    torch.cuda.synchronize()
+    want_y, want_v, _, _ = oracle.layer_norm(x, w, b, eps=moe.NORM_EPS, residual=r)
+    np.testing.assert_array_equal(y.cpu().numpy().view(np.uint32), want_y.view(np.uint32))
+    np.testing.assert_array_equal(xd.cpu().numpy().view(np.uint32), want_v.view(np.uint32))
+
+
 def test_layer_norm_known_answer_rows(gpu_device):
     """The oracle's order and fused-variance known-answer rows (the mean of
     [1e8, 1, -1e8, 0...] is 0, that of [1e8, -1e8, 1, 0...] is 2^-12; the
