@@ -19,9 +19,9 @@
 // double, so the float e_w agree except when a double lands within an ulp of
 // a float rounding boundary.
 //
-// gfx950 mapping.  Path groups (4 consecutive rows on one ancestor chain,
-// the common case) go to k_attention_group on the matrix cores (its own
-// comment has the mapping); k_attention_tree serves the other rows: one
+// gfx950 mapping.  k_attention_group takes the rows four at a time on the
+// matrix cores (its own comment has the mapping); k_attention_tree serves
+// windows whose scores do not fit LDS that way, and unaligned arrays: one
 // 256-thread workgroup per (row, KV head) serves the four query heads of the
 // group, as in the reference.  Scores: a thread owns a key and reads its
 // 128-float row as 16-byte vectors, one element per partial sum a_0..a_3
@@ -40,112 +40,106 @@ constexpr int kGroup = 4;            // query heads per KV head (GQA-4)
 constexpr int kAttnThreads = 256;
 
 typedef float af4 __attribute__((ext_vector_type(4)));
+typedef float af2 __attribute__((ext_vector_type(2)));
 
+// q and k in one launch: a row holds q_heads + kv_heads heads of half / P
+// runs of P pairs (j, j + half).  P = 4 (16-byte accesses) when the head
+// dimension and the alignment allow, else 1.  Bound by the traffic (4.7 TB/s
+// at 4,096 and more rows).  Measured, 43 / 4,096 / 10,240 rows: 5 / 16 / 35 us,
+// against 10 / 24 / 56 us in two launches of one pair per thread.
+template <int P>
 __global__ void __launch_bounds__(256)
-k_rope_tree(float* __restrict__ x, const uint32_t* __restrict__ row_pos, int64_t rows, int heads, int half,
-            const float* __restrict__ cosv, const float* __restrict__ sinv, int64_t max_seq) {
-    const int64_t pair = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
-    if (pair >= rows * heads * half) return;
-    const int j = static_cast<int>(pair % half);
-    const int64_t rh = pair / half;  // row * heads + head
+k_rope_tree(float* __restrict__ q, float* __restrict__ k, const uint32_t* __restrict__ row_pos, int64_t rows,
+            int q_heads, int kv_heads, int half, const float* __restrict__ cosv, const float* __restrict__ sinv,
+            int64_t max_seq) {
+    typedef float rv_t __attribute__((ext_vector_type(P)));
+    const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+    const int runs = half / P, heads = q_heads + kv_heads;
+    const int64_t rh = i / runs;   // row * heads + head
     const int64_t row = rh / heads;
+    if (row >= rows) return;
+    const int j = static_cast<int>(i - rh * runs) * P, head = static_cast<int>(rh - row * heads);
     const uint32_t pos = row_pos[row];
     if (pos >= max_seq) return;  // outside the table: left as is (the C++ layer checks positions)
-    float* base = x + rh * (2 * half);
+    float* base = head < q_heads ? q + (row * q_heads + head) * (2 * half)
+                                 : k + (row * kv_heads + (head - q_heads)) * (2 * half);
     const int64_t t = static_cast<int64_t>(pos) * half + j;
-    const float c = cosv[t], s = sinv[t];
-    const float x0 = base[j], x1 = base[j + half];
-    base[j] = __fmaf_rn(x0, c, -__fmul_rn(x1, s));
-    base[j + half] = __fmaf_rn(x1, c, __fmul_rn(x0, s));
+    auto ld = [](const float* p) { return *reinterpret_cast<const rv_t*>(p); };
+    const rv_t c = ld(cosv + t), s = ld(sinv + t), x0 = ld(base + j), x1 = ld(base + j + half);
+    rv_t o0, o1;
+#pragma unroll
+    for (int e = 0; e < P; ++e) {
+        o0[e] = __fmaf_rn(x0[e], c[e], -__fmul_rn(x1[e], s[e]));
+        o1[e] = __fmaf_rn(x1[e], c[e], __fmul_rn(x0[e], s[e]));
+    }
+    *reinterpret_cast<rv_t*>(base + j) = o0;
+    *reinterpret_cast<rv_t*>(base + j + half) = o1;
 }
 
 // ---------------------------------------------------------------------------
 // Row groups on the matrix cores.  Rows are taken 4 at a time (group g =
-// rows 4g .. 4g+3).  A group is a path group when every row lies on the
-// ancestor chain of the group's last row (tree: anc[last][pos[r]] == r;
-// packed: one sequence), so each row's keys are a contiguous range of that
-// one chain.  k_attention_group serves path groups; the row kernel below the
-// others.  Both evaluate this predicate the same way, on the same clamped
-// positions.
+// rows 4g .. 4g+3); a group is worked off in runs of rows that lie on the
+// ancestor chain of the run's last row (tree: anc[last][pos[r]] == r; packed:
+// one sequence), so each row's keys are a contiguous range of that one chain.
+// Most groups are one run; a trie branch or a sequence's end splits one.
 constexpr int kGroupRows = 4;
 constexpr int kGroupQueries = kGroupRows * kGroup;   // 16: query q = 4 row + head
 constexpr int kKeyTile = 16;                         // keys per score tile / value group
 
+// Bit 4 l + r: row r0 + r (r < l < nr) lies on the chain of row r0 + l.
 template <bool PACKED>
-__device__ inline bool group_is_path(const uint32_t* __restrict__ row_pos, const uint32_t* __restrict__ anc,
-                                     int64_t anc_stride, int64_t rows, int64_t r0, int wmax, int cap, int lane) {
-    const int nr = static_cast<int>(rows - r0 < kGroupRows ? rows - r0 : kGroupRows);
-    const int64_t last = r0 + nr - 1;
-    bool ok = true;
-    int64_t pr = 0;
-    if (lane < nr) {
-        const int64_t r = r0 + lane;
-        pr = row_pos[r];
+__device__ inline uint32_t chain_pairs(const uint32_t* __restrict__ row_pos, const uint32_t* __restrict__ anc,
+                                       int64_t anc_stride, int64_t r0, int nr, int lane) {
+    const int r = lane & 3, l = (lane >> 2) & 3;
+    bool ok = false;
+    if (lane < 16 && r < l && l < nr) {
+        const int64_t row = r0 + r, last = r0 + l;
+        int64_t pr = row_pos[row], pl = row_pos[last];
         pr = pr < anc_stride ? pr : anc_stride - 1;
-        if (PACKED) ok = anc[r] == anc[last];
-        else ok = anc[last * anc_stride + pr] == static_cast<uint32_t>(r);
+        pl = pl < anc_stride ? pl : anc_stride - 1;
+        ok = pr <= pl && (PACKED ? anc[row] == anc[last] : anc[last * anc_stride + pr] == static_cast<uint32_t>(row));
     }
-    // the group's key range chain[dlo .. plast] must hold every row's window
-    // and fit the kernel's LDS (cap keys)
-    const int64_t p0 = __shfl(pr, 0), plast = __shfl(pr, nr - 1);
-    if (lane < nr) ok = ok && pr >= p0 && pr <= plast;
-    const int64_t dlo = p0 + 1 > wmax ? p0 + 1 - wmax : 0;
-    return __all(ok) && plast - dlo + 1 <= cap;
+    return static_cast<uint32_t>(__ballot(ok));
 }
 
-typedef float ag16_t __attribute__((ext_vector_type(16)));
+typedef float ag4_t __attribute__((ext_vector_type(4)));
 
-// 4 x 4 transpose across the four 16-lane rows of a wave: on entry row R
-// holds x[c] = element 4 R + c of a 16-element run; on exit row R holds
-// x[r] = element 4 r + R.  Two v_permlane32_swap (rows 2, 3 of the first
-// operand <-> rows 0, 1 of the second) and two v_permlane16_swap (odd rows of
-// the first <-> even rows of the second).
-__device__ inline void rows_transpose4(af4& x) {
-    // (__float_as_uint on the element values: a bit cast of an element
-    // lvalue of a vector reads element 0)
-    const uint32_t a = __float_as_uint(x[0]), b = __float_as_uint(x[1]);
-    const uint32_t c = __float_as_uint(x[2]), d = __float_as_uint(x[3]);
-    auto ac = __builtin_amdgcn_permlane32_swap(a, c, false, false);
-    auto bd = __builtin_amdgcn_permlane32_swap(b, d, false, false);
-    auto ab = __builtin_amdgcn_permlane16_swap(ac[0], bd[0], false, false);
-    auto cd = __builtin_amdgcn_permlane16_swap(ac[1], bd[1], false, false);
-    x[0] = __uint_as_float(ab[0]);
-    x[1] = __uint_as_float(ab[1]);
-    x[2] = __uint_as_float(cd[0]);
-    x[3] = __uint_as_float(cd[1]);
-}
-
-// One workgroup = one path group x one KV head: 16 queries (4 rows x the
-// group's 4 query heads) against the keys chain[dlo .. dhi] of the group's
-// last row; row r attends to chain[begin_r .. pos_r].  The arithmetic is the
+// One workgroup = one row group x one KV head.  Per run of rows: 16 queries
+// (up to 4 rows x the KV head's 4 query heads) against the keys chain[dlo ..
+// dhi] of the run's last row; row r attends to chain[begin_r .. pos_r].  The arithmetic is the
 // row kernel's, operation for operation:
-//   scores on the K = 1 fp32 MFMA v_mfma_f32_16x16x1_4b_f32 (one fused
-//     multiply-add per element and step, the fmaf chain): its four blocks are
-//     the four partial chains a_j over d = j, j + 4, .. (block j: A = q[d],
-//     B = k[d] with d = 4 i + j at step i), for 16 queries x 16 keys; then
-//     s = ((a0 + a1) + (a2 + a3)) * scale in registers, into LDS;
+//   scores on v_mfma_f32_16x16x4_f32, whose products join the accumulator one
+//     after the other (chain_mfma.hpp): one accumulator per partial chain a_j
+//     over d = j, j + 4, .., 16 queries x 16 keys; then s = ((a0 + a1) + (a2 +
+//     a3)) * scale in registers, into LDS;
 //   per query over its window: m = max s, e = (float)exp((double)(s - m)),
 //     den = sum of e in key order (one lane per query), p = e / den;
-//   out[d] = chain over keys of p v[d] on the same MFMA: blocks are four
-//     16-dimension groups, A = p (lane = query), B = v.
-// Every score is computed once: the group's 16 x window scores sit in LDS.
+//   out[d] = chain over keys of p v[d] on the same MFMA, 16 queries x 16
+//     dimensions, four keys a step.
+// Every score is computed once: the run's 16 x window scores sit in LDS.
 // Keys after a row's window take p = 0, which leaves its value chains
 // unchanged except that a -0 would turn +0; keys before it keep the chain
-// at its +0 start.
+// at its +0 start; the last tile's padding has p = 0 and v = 0.
 //   K and V go from global memory straight to registers (LDS holds only the
 // scores and the chain's key rows, so two workgroups fit a CU at 1,024-key
-// windows, and three, MINB = 3 with 168 registers, at key spans up to 784).  Scores: wave w takes the 16-key tiles w, w + 4, ..; a lane
-// (key lane % 16, row j = lane / 16) loads 16 bytes of elements 16 a + 4 j ..
-// per a < 8 and a 4 x 4 transpose across the rows gives it d = 4 i + j,
-// tiles two ahead in flight.  Softmax: the 16 threads of query q are in
-// wave q / 4, so exp, the ordered denominator and p = e / den need no
-// workgroup barrier.  Values: two waves (0, 1 on even workgroups, 2, 3 on
-// odd ones, so that two resident workgroups spread them over the SIMDs) take
-// dimensions 64 w' .. 64 w' + 63, one coalesced 256-byte load per key, 64
-// keys ahead; the K / V row offsets are 32-bit byte offsets off a uniform
-// base.
-template <bool PACKED, int MINB>
-__global__ void __launch_bounds__(256, MINB)
+// windows, and three at key spans up to 784).  Scores: wave w takes the
+// 16-key tiles w, w + 4, ..; a lane (key lane % 16, k slot lane / 16) loads 16
+// bytes, elements 16 a + 4 (lane / 16) .. + 3 for a < 8, which are the operands of
+// the four partial chains at one step: no lane transposes.  The tile two
+// ahead goes into the registers a step has used up.  Softmax: the 16 threads
+// of query q are in wave q / 4, so exp, the ordered denominator and p = e /
+// den need no workgroup barrier.  Values: wave w takes dimensions 32 w .. 32 w
+// + 31, two per lane, one 8-byte load per four keys, 64 keys ahead; the K / V
+// row offsets are 32-bit byte offsets off a uniform base.
+//   Bound by the fp32 MFMAs with the vector work that cannot run beside them
+// (exp, division, addresses).  Measured, 4,096 rows of 512-token prompts: 249
+// us -> 177; 10,240 rows, 16 prompts of 1,024 with shared halves: 1345 -> 1016,
+// against the K = 1 MFMA with its operands transposed across lanes and the
+// values on two of the four waves.  Serving every group here, run by run,
+// instead of leaving branching groups to a second launch over all rows saves
+// that launch: 9.7 and 22 us, and 19 -> 12 us for 43 rows.
+template <bool PACKED>
+__global__ void __launch_bounds__(256, 3)
 k_attention_group(const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v,
                   float* __restrict__ out, const uint32_t* __restrict__ row_pos, const uint32_t* __restrict__ anc,
                   int64_t anc_stride, int64_t rows, int q_heads, int kv_heads, int wmax, float scale, int sw) {
@@ -155,20 +149,35 @@ k_attention_group(const float* __restrict__ q, const float* __restrict__ k, cons
     __shared__ int qlo[kGroupQueries], qhi[kGroupQueries];   // window of each query, relative to dlo
     __shared__ float wmx[4][kGroupQueries];                  // per-wave maxima
 
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     // groups in reverse row order: later rows (longer chains in trie and
     // packed order) start first, so the short ones fill the last round
-    const int64_t r0 = static_cast<int64_t>(gridDim.x / kv_heads - 1 - blockIdx.x / kv_heads) * kGroupRows;
+    const int64_t g0 = static_cast<int64_t>(gridDim.x / kv_heads - 1 - blockIdx.x / kv_heads) * kGroupRows;
     const int kh = static_cast<int>(blockIdx.x % kv_heads);
-    // sw = key capacity + 1; groups that are not path groups are the row kernel's
-    if (!group_is_path<PACKED>(row_pos, anc, anc_stride, rows, r0, wmax, sw - 1, lane)) return;
-    const int nr = static_cast<int>(rows - r0 < kGroupRows ? rows - r0 : kGroupRows);
-    const int64_t last = r0 + nr - 1;
+    const int gn = static_cast<int>(rows - g0 < kGroupRows ? rows - g0 : kGroupRows);
+    const uint32_t pairs = __builtin_amdgcn_readfirstlane(chain_pairs<PACKED>(row_pos, anc, anc_stride, g0, gn, threadIdx.x & 63));
     auto pos_of = [&](int64_t r) -> int64_t {
         const int64_t p = row_pos[r];
         return p < anc_stride ? p : anc_stride - 1;
     };
+    for (int i0 = 0, nr; i0 < gn; i0 += nr) {
+    const int64_t r0 = g0 + i0;
+    // (opaque per run: addresses hoisted out of the loop cost spills)
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));
+    const int lane = tid & 63;
+    // the longest run from row i0 whose key range, from its first row's
+    // window on, fits the LDS (sw - 1 keys: a single row always does)
+    for (nr = gn - i0; nr > 1; --nr) {
+        const int l = i0 + nr - 1;
+        const uint32_t need = ((1u << nr) - 1u) >> 1 << i0;   // rows i0 .. l - 1
+        const int64_t p0 = pos_of(r0);
+        bool fits = ((pairs >> (4 * l)) & need) == need &&
+                    pos_of(g0 + l) - (p0 + 1 > wmax ? p0 + 1 - wmax : 0) + 1 <= sw - 1;
+        for (int r = 1; r + 1 < nr; ++r) fits = fits && pos_of(r0 + r) >= p0;
+        if (fits) break;
+    }
+    const int64_t last = r0 + nr - 1;
     const int64_t plast = pos_of(last);
     const int64_t p0 = pos_of(r0);
     const int dlo = static_cast<int>(p0 + 1 > wmax ? p0 + 1 - wmax : 0);
@@ -188,14 +197,15 @@ k_attention_group(const float* __restrict__ q, const float* __restrict__ k, cons
         }
     }
     // q operand: lane l -> query l % 16 (row (l % 16) / 4, head (l % 16) % 4),
-    // element d = 4 i + l / 16 at step i (loads in flight during the staging)
+    // elements 16 a + 4 (l / 16) .. + 3, one per partial chain (loads in
+    // flight during the staging)
     const int qq = lane & 15, qj = lane >> 4;
     const int qrow = qq / kGroup;
     const int64_t qr = r0 + (qrow < nr ? qrow : nr - 1);
-    const float* qsrc = q + (qr * q_heads + kh * kGroup + qq % kGroup) * kHeadDim + qj;
-    float qv[32];
+    const af4* qsrc = reinterpret_cast<const af4*>(q + (qr * q_heads + kh * kGroup + qq % kGroup) * kHeadDim + 4 * qj);
+    af4 qv[8];
 #pragma unroll
-    for (int i = 0; i < 32; ++i) qv[i] = qsrc[4 * i];
+    for (int a = 0; a < 8; ++a) qv[a] = qsrc[4 * a];
     // the chain's key rows (clamped to the chain and the rows) in LDS, as
     // byte offsets of the key's K / V row (below 2^32: the launcher's check)
     const uint32_t kvs_bytes = static_cast<uint32_t>(kv_heads) * kHeadDim * sizeof(float);
@@ -215,10 +225,8 @@ k_attention_group(const float* __restrict__ q, const float* __restrict__ k, cons
 
     // ---- scores: tiles wave, wave + 4, .. ----
     const char* const kbase = reinterpret_cast<const char*>(k + kh * kHeadDim);
-    auto kload = [&](int t, af4* buf) __attribute__((always_inline)) {
-        const af4* src = reinterpret_cast<const af4*>(kbase + (chain[16 * t + qq] + 16u * qj));
-#pragma unroll
-        for (int a = 0; a < 8; ++a) buf[a] = src[4 * a];
+    auto ksrc = [&](int t) __attribute__((always_inline)) {
+        return reinterpret_cast<const af4*>(kbase + (chain[16 * t + qq] + 16u * qj));
     };
     float m[4] = {-3.402823466e+38f, -3.402823466e+38f, -3.402823466e+38f, -3.402823466e+38f};
     // the loads of every step are unconditional (a step past the end reloads
@@ -226,37 +234,42 @@ k_attention_group(const float* __restrict__ q, const float* __restrict__ k, cons
     // buffer's loads in flight
     auto tclamp = [&](int t) { return t < ntiles ? t : ntiles - 1; };
     auto tile = [&](int t, af4* buf) __attribute__((always_inline)) {
-        float kvv[32];
+        const af4* next = ksrc(tclamp(t + 8));
+        ag4_t acc[4] = {};   // partial chain j
 #pragma unroll
         for (int a = 0; a < 8; ++a) {
-            af4 x = buf[a];
-            rows_transpose4(x);
 #pragma unroll
-            for (int r = 0; r < 4; ++r) kvv[4 * a + r] = x[r];
+            for (int j = 0; j < 4; ++j)
+                acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(qv[a][j], buf[a][j], acc[j], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            buf[a] = next[4 * a];   // this wave's tile two ahead into the freed registers
+            __builtin_amdgcn_sched_barrier(0);
         }
-        kload(tclamp(t + 8), buf);   // this wave's tile two ahead into the freed registers
-        if (t >= ntiles) return;     // wave-uniform
-        ag16_t acc = {};
-#pragma unroll
-        for (int i = 0; i < 32; ++i) acc = __builtin_amdgcn_mfma_f32_16x16x1f32(qv[i], kvv[i], acc, 0, 0, 0);
-        // register 4 j + u: partial j of query 4 qj + u, key lane % 16
+        // register u of chain j: partial j of query 4 qj + u, key lane % 16
         const int w = 16 * t + qq;
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
-            const float sx = __fmul_rn(__fadd_rn(__fadd_rn(acc[u], acc[4 + u]), __fadd_rn(acc[8 + u], acc[12 + u])),
-                                       scale);
+            const float sx = __fmul_rn(__fadd_rn(__fadd_rn(acc[0][u], acc[1][u]), __fadd_rn(acc[2][u], acc[3][u])), scale);
             sc[(4 * qj + u) * sw + w] = sx;
             if (w >= lo[u] && w <= hi[u]) m[u] = fmaxf(m[u], sx);
         }
     };
     if (wave < ntiles) {
         af4 kb0[8], kb1[8];
-        kload(wave, kb0);
-        kload(tclamp(wave + 4), kb1);
-        for (int t = wave; t < ntiles; t += 8) {
+        const af4* s0 = ksrc(wave);
+        const af4* s1 = ksrc(tclamp(wave + 4));
+#pragma unroll
+        for (int a = 0; a < 8; ++a) kb0[a] = s0[4 * a];
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int a = 0; a < 8; ++a) kb1[a] = s1[4 * a];
+        __builtin_amdgcn_sched_barrier(0);
+        int t = wave;
+        for (; t + 4 < ntiles; t += 8) {
             tile(t, kb0);
             tile(t + 4, kb1);
         }
+        if (t < ntiles) tile(t, kb0);
     }
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
@@ -269,30 +282,19 @@ k_attention_group(const float* __restrict__ q, const float* __restrict__ k, cons
     // ---- softmax, per query on the 16 threads of one wave (queries
     // 4 w .. 4 w + 3 on wave w), so it needs no workgroup barrier ----
     const int qi = tid / 16, part = tid % 16;
-    const int pw0 = 2 * (blockIdx.x & 1);             // waves pw0, pw0 + 1 take the values
-    const int pwave = wave - pw0;                     // 0, 1 on those waves
-    const int dim = 64 * pwave + 16 * qj + qq;        // their B column
     const char* const vbase = reinterpret_cast<const char*>(v + kh * kHeadDim);   // uniform: 32-bit lane offsets
-    const uint32_t dbytes = static_cast<uint32_t>(dim) * sizeof(float);
-    auto vload = [&](int g, float* vb) __attribute__((always_inline)) {
-        const uint4* cr = reinterpret_cast<const uint4*>(chain + 16 * g);
+    const uint32_t dbytes = static_cast<uint32_t>(32 * wave + 2 * qq) * sizeof(float);   // this lane's two dimensions
+    auto vload = [&](int g, af2* vb) __attribute__((always_inline)) {
 #pragma unroll
-        for (int u4 = 0; u4 < 4; ++u4) {
-            const uint4 kr = cr[u4];
-            vb[4 * u4 + 0] = *reinterpret_cast<const float*>(vbase + (kr.x + dbytes));
-            vb[4 * u4 + 1] = *reinterpret_cast<const float*>(vbase + (kr.y + dbytes));
-            vb[4 * u4 + 2] = *reinterpret_cast<const float*>(vbase + (kr.z + dbytes));
-            vb[4 * u4 + 3] = *reinterpret_cast<const float*>(vbase + (kr.w + dbytes));
-        }
+        for (int u = 0; u < 4; ++u)
+            vb[u] = *reinterpret_cast<const af2*>(vbase + (chain[16 * g + 4 * u + qj] + dbytes));
     };
-    float vb0[16], vb1[16], vb2[16], vb3[16];
+    af2 vb0[4], vb1[4], vb2[4], vb3[4];
     auto gclamp = [&](int g) { return g < ntiles ? g : ntiles - 1; };
-    if (pwave == 0 || pwave == 1) {   // the first 64 keys' values go out now
-        vload(0, vb0);
-        vload(gclamp(1), vb1);
-        vload(gclamp(2), vb2);
-        vload(gclamp(3), vb3);
-    }
+    vload(0, vb0);   // the first 64 keys' values go out now
+    vload(gclamp(1), vb1);
+    vload(gclamp(2), vb2);
+    vload(gclamp(3), vb3);
     {
         const float mq = fmaxf(fmaxf(wmx[0][qi], wmx[1][qi]), fmaxf(wmx[2][qi], wmx[3][qi]));
         float* const srow = sc + qi * sw;
@@ -342,40 +344,49 @@ k_attention_group(const float* __restrict__ q, const float* __restrict__ k, cons
     }
     __syncthreads();
 
-    // ---- values: out[q][d] = chain over keys of p v[d] (waves pw0, pw0 + 1) ----
-    if (pwave != 0 && pwave != 1) return;
-    ag16_t o = {};   // register 4 j + t: dimension 64 pwave + 16 j + lane % 16, query 4 (lane / 16) + t
+    // ---- values: out[q][d] = chain over keys of p v[d] ----
+    ag4_t o[2] = {};   // register t of o[i]: query 4 (lane / 16) + t, dimension 32 wave + 2 (lane % 16) + i
     {
-        const float* prow = sc + qq * sw;                   // A: query lane % 16
-        auto group = [&](int g, float* vb) __attribute__((always_inline)) {
-            float vc[16];
+        const float* prow = sc + qq * sw + qj;   // A: query lane % 16, key lane / 16 of a step
+        float pa[2][4];
+        auto pload = [&](int g, float* p) __attribute__((always_inline)) {
 #pragma unroll
-            for (int u = 0; u < 16; ++u) vc[u] = vb[u];
-            vload(gclamp(g + 4), vb);   // unconditional, as for the scores
-            if (g >= ntiles) return;                           // wave-uniform
-            float pa[16];
-#pragma unroll
-            for (int u = 0; u < 16; ++u) pa[u] = prow[16 * g + u];
-#pragma unroll
-            for (int u = 0; u < 16; ++u) o = __builtin_amdgcn_mfma_f32_16x16x1f32(pa[u], vc[u], o, 0, 0, 0);
+            for (int u = 0; u < 4; ++u) p[u] = prow[16 * g + 4 * u];
         };
+        auto group = [&](int g, af2* vb, int s) __attribute__((always_inline)) {
+            pload(gclamp(g + 1), pa[s ^ 1]);
+            if (g < ntiles) {   // wave-uniform
+                if (16 * g + 16 > W) {   // the last tile's padding: no value at all
+#pragma unroll
+                    for (int u = 0; u < 4; ++u)
+                        if (16 * g + 4 * u + qj >= W) vb[u] = af2{0.0f, 0.0f};
+                }
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+#pragma unroll
+                    for (int i = 0; i < 2; ++i)
+                        o[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(pa[s][u], vb[u][i], o[i], 0, 0, 0);
+            }
+            vload(gclamp(g + 4), vb);   // unconditional, as for the scores
+        };
+        pload(0, pa[0]);
         for (int g = 0; g < ntiles; g += 4) {
-            group(g, vb0);
-            group(g + 1, vb1);
-            group(g + 2, vb2);
-            group(g + 3, vb3);
+            group(g, vb0, 0);
+            group(g + 1, vb1, 1);
+            group(g + 2, vb2, 0);
+            group(g + 3, vb3, 1);
         }
     }
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-            const int qx = 4 * qj + t;                      // query: row qx / 4, head qx % 4
-            const int r = qx / kGroup;
-            if (r < nr)
-                out[((r0 + r) * q_heads + kh * kGroup + qx % kGroup) * kHeadDim + 64 * pwave + 16 * j + qq] =
-                    o[4 * j + t];
-        }
+    for (int t = 0; t < 4; ++t) {
+        const int qx = 4 * qj + t;   // query: row qx / 4, head qx % 4
+        const int r = qx / kGroup;
+        if (r < nr)
+            *reinterpret_cast<af2*>(out + ((r0 + r) * q_heads + kh * kGroup + qx % kGroup) * kHeadDim + 32 * wave +
+                                    2 * qq) = af2{o[0][t], o[1][t]};
+    }
+    __syncthreads();   // the next run writes the chain and the scores
+    }
 }
 
 // Dynamic LDS: scores [wmax][4] fp32, then chain [wmax] u32.
@@ -389,8 +400,7 @@ template <bool PACKED>
 __global__ void __launch_bounds__(kAttnThreads)
 k_attention_tree(const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v,
                  float* __restrict__ out, const uint32_t* __restrict__ row_pos, const uint32_t* __restrict__ anc,
-                 int64_t anc_stride, int64_t rows, int q_heads, int kv_heads, int wmax, float scale,
-                 int group_cap) {
+                 int64_t anc_stride, int64_t rows, int q_heads, int kv_heads, int wmax, float scale) {
     extern __shared__ __align__(16) float dyn[];
     float* sc = dyn;                                                  // [w][g]
     uint32_t* chain = reinterpret_cast<uint32_t*>(dyn + static_cast<int64_t>(wmax) * kGroup);
@@ -400,9 +410,6 @@ k_attention_tree(const float* __restrict__ q, const float* __restrict__ k, const
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int64_t row = blockIdx.x / kv_heads;
     const int kh = static_cast<int>(blockIdx.x % kv_heads);
-    if (group_cap > 0 &&
-        group_is_path<PACKED>(row_pos, anc, anc_stride, rows, row / kGroupRows * kGroupRows, wmax, group_cap, lane))
-        return;  // k_attention_group's row
     // Positions past the ancestor table and key rows past the end are
     // clamped, for memory safety only: the C++ layer checks them (through
     // RowIndexBuffer::max_row and the packed segment table), and direct
@@ -592,12 +599,27 @@ k_attention_any(const float* __restrict__ q, const float* __restrict__ k, const 
 
 }  // namespace
 
-hipError_t launch_rope_tree(float* x, const uint32_t* row_pos, int64_t rows, int heads, int head_dim,
-                            const float* cosv, const float* sinv, int64_t max_seq, hipStream_t s) {
-    const int64_t pairs = rows * heads * (head_dim / 2);
-    if (pairs <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_rope_tree, dim3(static_cast<unsigned>(ceil_div(pairs, 256))), dim3(256), 0, s, x, row_pos,
-                       rows, heads, head_dim / 2, cosv, sinv, max_seq);
+hipError_t launch_rope_tree(float* q, float* k, const uint32_t* row_pos, int64_t rows, int q_heads, int kv_heads,
+                            int head_dim, const float* cosv, const float* sinv, int64_t max_seq, hipStream_t s) {
+    const int half = head_dim / 2;
+    if (kv_heads > 0 && q < k + rows * kv_heads * head_dim && k < q + rows * q_heads * head_dim) {
+        const hipError_t e = launch_rope_tree(q, q, row_pos, rows, q_heads, 0, head_dim, cosv, sinv, max_seq, s);
+        return e != hipSuccess
+                   ? e
+                   : launch_rope_tree(k, k, row_pos, rows, kv_heads, 0, head_dim, cosv, sinv, max_seq, s);
+    }
+    const uintptr_t addr = reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k) |
+                           reinterpret_cast<uintptr_t>(cosv) | reinterpret_cast<uintptr_t>(sinv);
+    const bool vec = half % 4 == 0 && (addr & 15u) == 0;
+    const int64_t n = rows * (q_heads + kv_heads) * (vec ? half / 4 : half);
+    if (n <= 0) return hipSuccess;
+    const dim3 grid(static_cast<unsigned>(ceil_div(n, 256)));
+    if (vec)
+        hipLaunchKernelGGL(k_rope_tree<4>, grid, dim3(256), 0, s, q, k, row_pos, rows, q_heads, kv_heads, half, cosv,
+                           sinv, max_seq);
+    else
+        hipLaunchKernelGGL(k_rope_tree<1>, grid, dim3(256), 0, s, q, k, row_pos, rows, q_heads, kv_heads, half, cosv,
+                           sinv, max_seq);
     return hipGetLastError();
 }
 
@@ -610,6 +632,32 @@ hipError_t launch_attention_tree(const float* q, const float* k, const float* v,
     const int64_t keys = anc_stride < window_max ? anc_stride : window_max;
     if (keys > kAttnMaxWindow) return hipErrorInvalidValue;
     const int wmax = static_cast<int>(keys);
+    // 1 / sqrtf(head_dim), both correctly rounded, as the reference kernel computes it
+    const float root = sqrtf(static_cast<float>(head_dim));
+    const float scale = 1.0f / root;
+    // path groups on the matrix cores when their scores fit in LDS (16
+    // queries x the group's key range), q, k, v are 16-byte and out 8-byte
+    // aligned; the rest per row
+    const int64_t span = ceil_div(keys + kGroupRows - 1, kKeyTile) * kKeyTile;
+    const int sw = static_cast<int>(span) | 1;   // odd row stride: 16 queries, 16 bank groups
+    const size_t glds = static_cast<size_t>(kGroupQueries + 1) * sw * sizeof(float);
+    const bool group = glds <= 150 * 1024 && rows * kv_heads * kHeadDim * static_cast<int64_t>(sizeof(float)) <= 0xFFFFFFFFll &&
+                       ((reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k) |
+                         reinterpret_cast<uintptr_t>(v)) & 15u) == 0 &&
+                       (reinterpret_cast<uintptr_t>(out) & 7u) == 0;
+    if (group) {
+        // (splitting one launch into a long- and a short-range launch lost
+        // more to the first one's tail than the short ranges gained)
+        auto gk = packed ? &k_attention_group<true> : &k_attention_group<false>;
+        if (glds > 65536) {
+            const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(gk),
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(glds));
+            if (e != hipSuccess) return e;
+        }
+        hipLaunchKernelGGL(gk, dim3(static_cast<unsigned>(ceil_div(rows, kGroupRows) * kv_heads)), dim3(256), glds, s,
+                           q, k, v, out, row_pos, anc, anc_stride, rows, q_heads, kv_heads, wmax, scale, sw);
+        return hipGetLastError();
+    }
     const size_t lds = static_cast<size_t>(wmax) * (kGroup * sizeof(float) + sizeof(uint32_t));
     // dynamic LDS past 64 KB needs the function's limit raised first
     auto kern = packed ? &k_attention_tree<true> : &k_attention_tree<false>;
@@ -618,39 +666,8 @@ hipError_t launch_attention_tree(const float* q, const float* k, const float* v,
                                                  hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
         if (e != hipSuccess) return e;
     }
-    // 1 / sqrtf(head_dim), both correctly rounded, as the reference kernel computes it
-    const float root = sqrtf(static_cast<float>(head_dim));
-    const float scale = 1.0f / root;
-    // path groups on the matrix cores when their scores fit in LDS (16
-    // queries x the group's key range) and q, k, v are 16-byte aligned; the
-    // rest per row
-    const int64_t span = ceil_div(keys + kGroupRows - 1, kKeyTile) * kKeyTile;
-    const int sw = static_cast<int>(span) | 1;   // odd row stride: 16 queries, 16 bank groups
-    const size_t glds = static_cast<size_t>(kGroupQueries + 1) * sw * sizeof(float);
-    const bool group = glds <= 150 * 1024 && rows * kv_heads * kHeadDim * static_cast<int64_t>(sizeof(float)) <= 0xFFFFFFFFll &&
-                       ((reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k) |
-                         reinterpret_cast<uintptr_t>(v)) & 15u) == 0;
-    if (group) {
-        // three workgroups per CU (registers trimmed to 168) when three key
-        // ranges fit the LDS, else two.  (Splitting one launch into a long-
-        // and a short-range launch lost more to the first one's tail than
-        // the short ranges gained.)
-        const bool three = 3 * (glds + 384) <= 160 * 1024;
-        auto gk = three ? (packed ? &k_attention_group<true, 3> : &k_attention_group<false, 3>)
-                        : (packed ? &k_attention_group<true, 2> : &k_attention_group<false, 2>);
-        if (glds > 65536) {
-            const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(gk),
-                                                     hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(glds));
-            if (e != hipSuccess) return e;
-        }
-        hipLaunchKernelGGL(gk, dim3(static_cast<unsigned>(ceil_div(rows, kGroupRows) * kv_heads)), dim3(256), glds, s,
-                           q, k, v, out, row_pos, anc, anc_stride, rows, q_heads, kv_heads, wmax, scale, sw);
-        const hipError_t e = hipGetLastError();
-        if (e != hipSuccess) return e;
-    }
     hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(rows * kv_heads)), dim3(kAttnThreads), lds, s, q, k, v, out,
-                       row_pos, anc, anc_stride, rows, q_heads, kv_heads, wmax, scale,
-                       group ? static_cast<int>(span) : 0);
+                       row_pos, anc, anc_stride, rows, q_heads, kv_heads, wmax, scale);
     return hipGetLastError();
 }
 

@@ -776,9 +776,7 @@ int aps_rope_tree(float* q, float* k, const uint32_t* row_pos, int64_t rows, int
     if (rows == 0) return APS_OK;
     if (!q || !k || !row_pos || !cos_table || !sin_table) return fail(APS_ERR_ARG, "rope: NULL pointer");
     const hipStream_t s = static_cast<hipStream_t>(stream);
-    APS_HIP(aps::launch_rope_tree(q, row_pos, rows, q_heads, head_dim, cos_table, sin_table, max_seq, s),
-            "rope launch");
-    APS_HIP(aps::launch_rope_tree(k, row_pos, rows, kv_heads, head_dim, cos_table, sin_table, max_seq, s),
+    APS_HIP(aps::launch_rope_tree(q, k, row_pos, rows, q_heads, kv_heads, head_dim, cos_table, sin_table, max_seq, s),
             "rope launch");
     return APS_OK;
 }

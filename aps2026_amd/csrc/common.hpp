@@ -195,8 +195,9 @@ hipError_t launch_prefix_ancestors(const uint32_t* parent, const uint32_t* depth
 
 // RoPE in place on x [rows][heads][head_dim] at each row's position (pairs
 // j, j + head_dim / 2); rows whose position is >= max_seq are left as they are.
-hipError_t launch_rope_tree(float* x, const uint32_t* row_pos, int64_t rows, int heads, int head_dim,
-                            const float* cosv, const float* sinv, int64_t max_seq, hipStream_t s);
+// q and k in one launch; arrays that overlap are rotated one after the other.
+hipError_t launch_rope_tree(float* q, float* k, const uint32_t* row_pos, int64_t rows, int q_heads, int kv_heads,
+                            int head_dim, const float* cosv, const float* sinv, int64_t max_seq, hipStream_t s);
 
 // GQA-4 tree attention, head_dim 128 (the reference kernel's arithmetic).
 // A workgroup keeps 20 bytes of LDS per key of its window (four scores and

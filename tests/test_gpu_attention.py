@@ -247,6 +247,59 @@ def test_attention_excluded_keys_take_no_part(gpu_device, window):
     np.testing.assert_array_equal(got.view(np.uint32), want.view(np.uint32))
 
 
+@pytest.mark.parametrize("window", [2047, 3])
+def test_attention_branching_groups_bit_exact(gpu_device, window):
+    """Groups of four rows that fall into several runs: prompts that branch
+    after every few tokens, ends of chains inside a group, row counts of
+    every remainder by four, key counts around the 16-key tiles."""
+    note(f"attention tree branching groups window={window}")
+    for tail in (1, 2, 3, 4):
+        batch = [[7, 8, 9] + [i] * (i % 3 + 1) for i in range(6)] + [[7, 8, 9, 0, 5] + list(range(30 + tail))]
+        plan, q, k, v = trie_inputs(batch, q_heads=16, kv_heads=4, seed=tail)
+        out = torch.empty((plan.nodes, 16 * 128), dtype=torch.float32, device=gpu_device)
+        attention.attention_tree_gpu(dev(q, gpu_device), dev(k, gpu_device), dev(v, gpu_device), out,
+                                     plan.node_depth, plan.node_anc, plan.max_len, window=window)
+        torch.cuda.synchronize()
+        want = oracle.attention_tree(q, k, v, plan.node_depth, plan.node_anc, plan.max_len, 16, 4, 128, window)
+        np.testing.assert_array_equal(out.cpu().numpy().view(np.uint32), want.view(np.uint32))
+
+
+@pytest.mark.parametrize("hd", [10, 128])
+def test_rope_overlapping_and_unaligned(gpu_device, hd):
+    """q and k at an address that is not 16-byte aligned, a head dimension
+    whose half is not a multiple of four, and k the same array as q (rotated
+    twice): the bits of one rotation after the other."""
+    from aps2026_amd import capi
+    from aps2026_amd.moe import _ptr, _stream
+    rows, heads, seq = 5, 3, 9
+    rng = np.random.default_rng(hd)
+    pos = np.array([0, 3, 8, 1, 8], np.int32)
+    cs = rng.standard_normal((2, seq, hd // 2)).astype(np.float32)
+    c, s = (dev(a, gpu_device) for a in cs)
+    pd = dev(pos, gpu_device)
+    flat = dev(rng.standard_normal(1 + 2 * rows * heads * hd).astype(np.float32), gpu_device)
+
+    def rope(q, k):
+        rc = capi.lib().aps_rope_tree(_ptr(q), _ptr(k), _ptr(pd), rows, heads, heads, hd, _ptr(c), _ptr(s), seq,
+                                      _stream(q.device))
+        assert rc == 0, capi.last_error()
+        torch.cuda.synchronize()
+
+    n = rows * heads * hd
+    q0, k0 = flat[:n].clone(), flat[n:2 * n].clone()     # aligned
+    rope(q0, k0)
+    off = flat.clone()
+    off[1:] = flat[:-1]
+    q1, k1 = off[1:1 + n], off[1 + n:1 + 2 * n]          # 4 bytes past it
+    rope(q1, k1)
+    assert torch.equal(q0.view(torch.int32), q1.view(torch.int32))
+    assert torch.equal(k0.view(torch.int32), k1.view(torch.int32))
+    twice = flat[:n].clone()
+    rope(twice, twice)
+    rope(q0, torch.empty_like(k0))                        # q0 has been rotated once above
+    assert torch.equal(q0.view(torch.int32), twice.view(torch.int32))
+
+
 def test_attention_nodes_equal_token_rows(gpu_device):
     note("attention tree nodes vs token rows")
     batch = shared_batch(4, groups=2, per=4, pre=60, suf=20)
