@@ -89,6 +89,32 @@ def test_linear_tc_gpu_matches_the_split_products(gpu_device, rows, k, n, all_te
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("rows,k,n", [(1, 64, 4), (127, 128, 68), (128, 192, 132), (2049, 64, 2052), (5000, 64, 1668)])
+def test_linear_tc_block_widths(gpu_device, rows, k, n):
+    """One to six stages of 32 k and each block width (64 columns up to a few
+    hundred rows, 128 and 256 past that), with partly filled row and column
+    blocks and an absent second weight image: every output against the split
+    products in fp64, the last row and column among them."""
+    from aps2026_amd import attention
+    print(f"[case] linear tc block widths rows={rows} k={k} n={n}", flush=True)
+    rng = np.random.default_rng(rows + k + n)
+    x = rng.standard_normal((rows, k)).astype(np.float32)
+    w = (0.02 * rng.standard_normal((n, k))).astype(np.float32)
+    xd = torch.from_numpy(x).to(gpu_device)
+    packed = attention.linear_tc_prepare(torch.from_numpy(w).to(gpu_device))
+    xs = attention.linear_tc_split(xd)
+    xh, xl = oracle.bf16_split(x)
+    wh, wl = oracle.bf16_split(w)
+    d = np.float64
+    three = xh.astype(d) @ wh.T.astype(d) + xh.astype(d) @ wl.T.astype(d) + xl.astype(d) @ wh.T.astype(d)
+    for all_terms in (False, True):
+        want = three + (xl.astype(d) @ wl.T.astype(d) if all_terms else 0.0)
+        got = attention.linear_tc_gpu(xs, packed, n, None, all_terms).cpu().numpy()
+        # fp32 accumulation of at most 4 k = 768 products: 768 x 2^-24 of the scale at worst
+        assert (np.abs(got - want) / _scale(x, w)).max() < 768 * 2.0 ** -24
+
+
+@pytest.mark.gpu
 def test_linear_tc_multi_equals_single_launches(gpu_device):
     """aps_linear_tc_multi (q, k and v of one split input in one launch)
     equals one aps_linear_tc per output bit for bit."""
