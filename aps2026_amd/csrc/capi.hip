@@ -240,7 +240,9 @@ int grouped_from_logits(const WeightSet& w, const void* x, bool x_is_f32, const 
         APS_HIP(aps::launch_ffn_up_fp8(xq, xs, offsets, arows, w.q13, w.s1, w.s3, act, rows, w.H, w.F, w.E, s),
                 "ffn_up_fp8 launch");
         APS_HIP(aps::launch_quant_rows_e4m3(act, w.F, w.F, actq, kp, as, 2 * rows, s), "quantise act launch");
-        if (fold) {
+        // few rows: the one-wave w2 tiles and the combine (the fold's two
+        // passes over all of w2 cost more than y's round trip)
+        if (fold && !aps::ffn_small_fits(true, rows, w.F, w.E)) {
             // slot-0 rows to y's bytes as [rows][H] by token, then slot-1 rows
             // combined with them straight into out
             APS_HIP(aps::launch_ffn_down_fold_fp8(actq, as, offsets, slot1, srows, stoks, w.q2, w.s2,

@@ -283,6 +283,15 @@ hipError_t launch_ffn_down_fp8(const uint8_t* actq, const float* act_scale, cons
 // token, then slot-1 rows combined with them into out [rows][hidden] bf16.
 // ffn_down_fold_fits: the shapes it serves.
 bool ffn_down_fold_fits(int64_t rows, int hidden, int ffn);
+// One-wave tiles for few rows (ffn_small.hip): the rule and the launches that
+// the bf16 and fp8 launchers above take under it.
+bool ffn_small_fits(bool fp8, int64_t rows, int ffn, int experts);
+hipError_t launch_ffn_up_small(bool fp8, const uint8_t* x, const float* sx, const uint32_t* offsets,
+                               const uint32_t* assignment_rows, const uint8_t* w13, const float* s1, const float* s3,
+                               bf16_t* act, int64_t rows, int hidden, int ffn, int experts, hipStream_t s);
+hipError_t launch_ffn_down_small(bool fp8, const uint8_t* act, const float* sa, const uint32_t* offsets,
+                                 const uint8_t* w2, const float* s2, bf16_t* y, int64_t rows, int hidden, int ffn,
+                                 int experts, hipStream_t s);
 hipError_t launch_ffn_down_fold_fp8(const uint8_t* actq, const float* act_scale, const uint32_t* offsets,
                                     const uint32_t* slot1, const uint32_t* slot_rows, const uint32_t* slot_tokens,
                                     const uint8_t* w2, const float* w2_scale, bf16_t* ya, bf16_t* out,

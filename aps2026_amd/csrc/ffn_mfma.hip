@@ -1278,6 +1278,10 @@ hipError_t launch_ffn_up_bf16(const bf16_t* x, const uint32_t* offsets,
                               hipStream_t s) {
     if (rows <= 0) return hipSuccess;
     if (hidden % 64 != 0 || ffn % 64 != 0) return hipErrorInvalidValue;
+    if (ffn_small_fits(false, rows, ffn, experts))
+        return launch_ffn_up_small(false, reinterpret_cast<const uint8_t*>(x), nullptr, offsets, assignment_rows,
+                                   reinterpret_cast<const uint8_t*>(w13), nullptr, nullptr, act, rows, hidden, ffn,
+                                   experts, s);
     hipLaunchKernelGGL(k_ffn_up<Bf16Fmt>, grid_up(), dim3(256), 0, s,
                        reinterpret_cast<const uint8_t*>(x), static_cast<int64_t>(hidden) * 2, offsets,
                        assignment_rows, reinterpret_cast<const uint8_t*>(w13), act, hidden, ffn, experts,
@@ -1290,6 +1294,9 @@ hipError_t launch_ffn_down_bf16(const bf16_t* act, const uint32_t* offsets, cons
                                 hipStream_t s) {
     if (rows <= 0) return hipSuccess;
     if (hidden % 128 != 0 || ffn % 64 != 0) return hipErrorInvalidValue;
+    if (ffn_small_fits(false, rows, ffn, experts))
+        return launch_ffn_down_small(false, reinterpret_cast<const uint8_t*>(act), nullptr, offsets,
+                                     reinterpret_cast<const uint8_t*>(w2), nullptr, y, rows, hidden, ffn, experts, s);
     if (auto kern = down_ar_kernel<Bf16Fmt>(ffn / 64)) {
         hipLaunchKernelGGL(kern, grid_ar(rows, experts), dim3(256), 0, s,
                            reinterpret_cast<const uint8_t*>(act), static_cast<int64_t>(ffn) * 2, offsets,
@@ -1310,6 +1317,9 @@ hipError_t launch_ffn_up_fp8(const uint8_t* xq, const float* x_scale, const uint
                              int experts, hipStream_t s) {
     if (rows <= 0) return hipSuccess;
     if (hidden % 128 != 0 || ffn % 64 != 0) return hipErrorInvalidValue;
+    if (ffn_small_fits(true, rows, ffn, experts))
+        return launch_ffn_up_small(true, xq, x_scale, offsets, assignment_rows, w13, w1_scale, w3_scale, act, rows,
+                                   hidden, ffn, experts, s);
     hipLaunchKernelGGL(k_ffn_up<Fp8Fmt>, grid_up(), dim3(256), 0, s,
                        xq, static_cast<int64_t>(hidden), offsets, assignment_rows, w13, act, hidden, ffn, experts,
                        x_scale, w1_scale, w3_scale);
@@ -1321,6 +1331,8 @@ hipError_t launch_ffn_down_fp8(const uint8_t* actq, const float* act_scale, cons
                                int ffn, int experts, hipStream_t s) {
     if (rows <= 0) return hipSuccess;
     if (hidden % 128 != 0 || ffn % 64 != 0) return hipErrorInvalidValue;
+    if (ffn_small_fits(true, rows, ffn, experts))
+        return launch_ffn_down_small(true, actq, act_scale, offsets, w2, w2_scale, y, rows, hidden, ffn, experts, s);
     const int kpad = static_cast<int>(ceil_div(ffn, 128) * 128);
     if (auto kern = down_ar_kernel<Fp8Fmt>(kpad / 128)) {
         hipLaunchKernelGGL(kern, grid_ar(rows, experts), dim3(256), 0, s, actq,

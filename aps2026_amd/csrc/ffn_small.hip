@@ -1,0 +1,284 @@
+// Grouped expert FFN for few rows per expert (a decode step, a small serving
+// batch): the same products as ffn_mfma.hip, bit for bit, in one-wave tiles.
+//
+// With a handful of rows per expert the GEMMs are bound by the weights' bytes
+// (bf16, 16 experts: 117 MB for w1||w3, 59 MB for w2), or for one or two
+// active experts by how many CUs share them and by latency.  The row tiles of
+// ffn_mfma.hip stage 128 or 256 activation rows whatever their number, two
+// bytes of copies for every byte of weights, through a ring that holds 16 KB
+// of weights per CU.  Here a wave owns 32 rows x 32 packed weight rows over
+// the whole K and loads both MFMA operands straight into registers, several
+// stages ahead: no LDS, no barriers, 4 KB of weights in flight per stage, and
+// rows past the expert's end re-read its last row (the same cache lines).
+//  * w1||w3: 16 gate rows and the same 16 up rows, so that SwiGLU closes inside
+//    each lane.  Eight stages of 128 bytes per row in flight: 64 loads, what
+//    the wave can count (twelve were slower).
+//  * w2: 32 hidden columns; K = F is short enough for every operand fragment
+//    of the tile to be in flight at once.
+// Every output element accumulates the same MFMA sequence over k ascending as
+// in ffn_mfma.hip, so a row's bits do not depend on its batch.
+//   Measured, bf16: 37 tokens w1||w3 27 -> 21 us (5.6 TB/s), w2 19 -> 11 us (5.5
+// TB/s); one token 23 -> 12.5 and 13 -> 3.8 us.  fp8, 65 tokens: 17 -> 14 us, w2
+// with its combine 38 -> 11 us.
+//
+// The packed images are read at their swizzled 16-byte chunks: the four (bf16)
+// reads of a 128-byte image row follow each other and share its cache line.
+#include "mfma_ring.hpp"
+
+namespace aps {
+namespace {
+
+constexpr int kSmRows = 32;      // rows per tile
+constexpr int kSmXcds = 8;
+constexpr int kSmAhead = 8;      // w1||w3 stages in flight
+
+struct SmallTile {
+    int expert, col;             // expert, column group
+    uint32_t m0, end;            // first position, expert's end
+};
+
+// Tile b of the list expert -> column group -> 32-row tile, dealt to the XCDs
+// in contiguous slices (workgroup b runs on XCD b % 8), so that the row tiles
+// of an expert read a weight tile in one L2.  `bn`: column groups.  A block
+// takes every (gridDim.x / 8)-th tile of its slice; the grid covers 2 rows
+// assignments in one round, a caller's plan may hold more.
+template <class Body>
+__device__ inline void each_small(const uint32_t* __restrict__ offsets, int E, int bn, Body body) {
+    const int lane = threadIdx.x & 63;
+    const uint32_t lo = lane < E ? offsets[lane] : 0u;
+    const uint32_t hi = lane < E ? offsets[lane + 1] : 0u;
+    const int tiles = static_cast<int>((hi - lo + kSmRows - 1) / kSmRows);
+    int incl = tiles * bn;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const int v = __shfl_up(incl, d);
+        if (lane >= d) incl += v;
+    }
+    const int total = __shfl(incl, 63);
+    const int per = (total + kSmXcds - 1) / kSmXcds;
+    const int first = static_cast<int>(blockIdx.x % kSmXcds) * per;
+    for (int l = static_cast<int>(blockIdx.x) / kSmXcds; l < per; l += static_cast<int>(gridDim.x) / kSmXcds) {
+        const int t = first + l;
+        if (t >= total) return;
+        const int e = __ffsll(static_cast<unsigned long long>(__ballot(incl > t))) - 1;
+        const int i = t - (e > 0 ? __shfl(incl, e - 1) : 0);
+        const int n = __shfl(tiles, e);
+        SmallTile u;
+        u.expert = __builtin_amdgcn_readfirstlane(e);
+        u.col = __builtin_amdgcn_readfirstlane(i / n);
+        u.m0 = __builtin_amdgcn_readfirstlane(__shfl(lo, e) + static_cast<uint32_t>(i % n) * kSmRows);
+        u.end = __builtin_amdgcn_readfirstlane(__shfl(hi, e));
+        body(u);
+    }
+}
+
+// One 128-byte stage of a lane's row: kSub fragments, each 16 (bf16) or 32
+// (fp8) bytes of the k half lane / 32.
+template <class Fmt>
+struct SmallStage {
+    typename Fmt::frag_t f[Fmt::kSub];
+};
+// Byte offset of part p of fragment kk in a row's stage (logical chunk order).
+template <class Fmt>
+__device__ inline int small_chunk(int kk, int p, int lane) {
+    return (8 / Fmt::kSub) * kk + Fmt::kParts * (lane >> 5) + p;
+}
+template <class Fmt, class At>
+__device__ inline void small_load(SmallStage<Fmt>& d, At at) {
+#pragma unroll
+    for (int kk = 0; kk < Fmt::kSub; ++kk) {
+        u32x4_t v[Fmt::kParts];
+#pragma unroll
+        for (int p = 0; p < Fmt::kParts; ++p) v[p] = *reinterpret_cast<const u32x4_t*>(at(kk, p));
+        if constexpr (Fmt::kParts == 1) d.f[kk] = __builtin_bit_cast(typename Fmt::frag_t, v[0]);
+        else
+            d.f[kk] = __builtin_bit_cast(typename Fmt::frag_t, __builtin_shufflevector(v[0], v[1], 0, 1, 2, 3, 4, 5, 6, 7));
+    }
+}
+
+// act[p][n], as ffn_mfma.hip's up_piece.
+template <class Fmt>
+__global__ void __launch_bounds__(64, 1)
+k_ffn_up_small(const uint8_t* __restrict__ x, uint32_t x_row_bytes, const uint32_t* __restrict__ offsets,
+               const uint32_t* __restrict__ assignment_rows, const uint8_t* __restrict__ w13,
+               bf16_t* __restrict__ act, int H, int F, int E, const float* __restrict__ sx,
+               const float* __restrict__ s1, const float* __restrict__ s3) {
+    constexpr bool kFp8 = Fmt::kElt == 1;
+    each_small(offsets, E, F / 16, [&](const SmallTile& u) __attribute__((always_inline)) {
+    const int lane = threadIdx.x, r = lane & 31, h = lane >> 5;
+    const int KT = H * Fmt::kElt / kRowBytes;
+    const uint32_t p = u.m0 + r < u.end ? u.m0 + r : u.end - 1;
+    const uint32_t token = assignment_rows[p];
+    // image row of this lane: gate row 16 (col % 4) + r, then the same up rows
+    const int ir = 16 * (u.col & 3) + (r < 16 ? r : 64 + (r - 16));
+    const uint8_t* image = w13 + (static_cast<int64_t>(u.expert) * (F / 64) + u.col / 4) * KT * kImageBytes;
+    uint32_t ao[Fmt::kSub][Fmt::kParts], bo[Fmt::kSub][Fmt::kParts];
+#pragma unroll
+    for (int kk = 0; kk < Fmt::kSub; ++kk)
+#pragma unroll
+        for (int q = 0; q < Fmt::kParts; ++q) {
+            ao[kk][q] = token * x_row_bytes + 16u * small_chunk<Fmt>(kk, q, lane);
+            bo[kk][q] = static_cast<uint32_t>(swz(ir, small_chunk<Fmt>(kk, q, lane)));
+        }
+    SmallStage<Fmt> a[kSmAhead], b[kSmAhead];
+    // unconditional (a stage past the end re-reads the last), so that the
+    // waits count the stages in flight
+    auto load = [&](int d, int kt) __attribute__((always_inline)) {
+        kt = kt < KT ? kt : KT - 1;
+        const uint8_t* xb = x + static_cast<int64_t>(kt) * kRowBytes;
+        const uint8_t* wb = image + static_cast<int64_t>(kt) * kImageBytes;
+        small_load<Fmt>(b[d], [&](int kk, int q) __attribute__((always_inline)) { return wb + bo[kk][q]; });
+        small_load<Fmt>(a[d], [&](int kk, int q) __attribute__((always_inline)) { return xb + ao[kk][q]; });
+        APS_PIN();
+    };
+#pragma unroll
+    for (int d = 0; d < kSmAhead; ++d) load(d, d);
+    f32x16_t acc = {};
+    for (int k0 = 0; k0 < KT; k0 += kSmAhead)
+#pragma unroll
+        for (int d = 0; d < kSmAhead; ++d) {
+            if (k0 + d < KT)   // wave-uniform
+#pragma unroll
+                for (int kk = 0; kk < Fmt::kSub; ++kk) acc = Fmt::mma(b[d].f[kk], a[d].f[kk], acc);
+            APS_PIN();
+            load(d, k0 + d + kSmAhead);
+        }
+    // lane: row r; register 4 q + v: packed row 8 q + 4 h + v, i.e. gate column
+    // 8 q + 4 h + v for q < 2 and its up value at q + 2
+    if (u.m0 + r >= u.end) return;
+    const int c0 = 16 * u.col + 4 * h;
+    const float rs = kFp8 ? sx[token] : 1.0f;
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+        float g[4], up[4];
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            g[v] = acc[4 * q + v];
+            up[v] = acc[4 * (q + 2) + v];
+            if constexpr (kFp8) {
+                const int at = u.expert * F + c0 + 8 * q + v;
+                g[v] = g[v] * rs * s1[at];
+                up[v] = up[v] * rs * s3[at];
+            }
+        }
+        *reinterpret_cast<u32x2_t*>(act + static_cast<int64_t>(p) * F + c0 + 8 * q) =
+            u32x2_t{pack2_bf16(swiglu(g[0], up[0]), swiglu(g[1], up[1])),
+                    pack2_bf16(swiglu(g[2], up[2]), swiglu(g[3], up[3]))};
+    }
+    });
+}
+
+// y[p][n], as ffn_mfma.hip's w2 GEMM.  KT: 128-byte stages of an act row.
+template <class Fmt, int KT>
+__global__ void __launch_bounds__(64, 2)
+k_ffn_down_small(const uint8_t* __restrict__ act, int64_t act_row_bytes, const uint32_t* __restrict__ offsets,
+                 const uint8_t* __restrict__ w2, bf16_t* __restrict__ y, int H, int E, const float* __restrict__ sa,
+                 const float* __restrict__ s2) {
+    constexpr bool kFp8 = Fmt::kElt == 1;
+    each_small(offsets, E, H / 32, [&](const SmallTile& u) __attribute__((always_inline)) {
+    const int lane = threadIdx.x, r = lane & 31, h = lane >> 5;
+    const uint32_t p = u.m0 + r < u.end ? u.m0 + r : u.end - 1;
+    const uint8_t* image = w2 + (static_cast<int64_t>(u.expert) * (H / 128) + u.col / 4) * KT * kImageBytes;
+    const uint8_t* arow = act + static_cast<int64_t>(p) * act_row_bytes;
+    const int ir = 32 * (u.col & 3) + r;
+    SmallStage<Fmt> a[KT], b[KT];
+#pragma unroll
+    for (int kt = 0; kt < KT; ++kt) {
+        small_load<Fmt>(b[kt], [&](int kk, int q) __attribute__((always_inline)) {
+            return image + kt * kImageBytes + swz(ir, small_chunk<Fmt>(kk, q, lane));
+        });
+        small_load<Fmt>(a[kt], [&](int kk, int q) __attribute__((always_inline)) {
+            return arow + kt * kRowBytes + 16 * small_chunk<Fmt>(kk, q, lane);
+        });
+        APS_PIN();
+    }
+    f32x16_t acc = {};
+#pragma unroll
+    for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+        for (int kk = 0; kk < Fmt::kSub; ++kk) acc = Fmt::mma(b[kt].f[kk], a[kt].f[kk], acc);
+    if (u.m0 + r >= u.end) return;
+    const int c0 = 32 * u.col + 4 * h;
+    const float rs = kFp8 ? sa[p] : 1.0f;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        float o[4];
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            o[v] = acc[4 * q + v];
+            if constexpr (kFp8) o[v] = o[v] * rs * s2[u.expert * H + c0 + 8 * q + v];
+        }
+        *reinterpret_cast<u32x2_t*>(y + static_cast<int64_t>(p) * H + c0 + 8 * q) =
+            u32x2_t{pack2_bf16(o[0], o[1]), pack2_bf16(o[2], o[3])};
+    }
+    });
+}
+
+typedef void (*down_small_fn)(const uint8_t*, int64_t, const uint32_t*, const uint8_t*, bf16_t*, int, int,
+                              const float*, const float*);
+// The w2 kernel for KT stages, or null (the operands of longer rows do not fit
+// the registers).
+template <class Fmt>
+down_small_fn down_small_kernel(int KT) {
+    constexpr int kMax = Fmt::kElt == 1 ? 4 : 7;
+    switch (KT) {
+        case 1: return k_ffn_down_small<Fmt, 1>;
+        case 2: return k_ffn_down_small<Fmt, 2>;
+        case 3: return k_ffn_down_small<Fmt, 3>;
+        case 4: return k_ffn_down_small<Fmt, 4>;
+        case 5: return kMax >= 5 ? k_ffn_down_small<Fmt, (kMax >= 5 ? 5 : 1)> : nullptr;
+        case 6: return kMax >= 6 ? k_ffn_down_small<Fmt, (kMax >= 6 ? 6 : 1)> : nullptr;
+        case 7: return kMax >= 7 ? k_ffn_down_small<Fmt, (kMax >= 7 ? 7 : 1)> : nullptr;
+        default: return nullptr;
+    }
+}
+
+// Blocks of a tile list of 2 rows assignments: every expert's last tile may be
+// partly filled, and an expert has a tile only if it has a row.
+dim3 grid_small(int64_t rows, int experts, int bn) {
+    const int64_t some = 2 * rows < experts ? 2 * rows : experts;
+    const int64_t tiles = (2 * rows) / kSmRows + some;
+    return dim3(static_cast<unsigned>(ceil_div(tiles * bn, kSmXcds) * kSmXcds));
+}
+
+int small_kt(bool fp8, int ffn) { return static_cast<int>(fp8 ? ceil_div(ffn, 128) : ffn / 64); }
+
+}  // namespace
+
+// Up to 12 rows per expert on average in bf16, 24 in fp8, whose MFMAs and w2
+// passes weigh less against the weights' bytes: a tile reads its weights for
+// 32 rows, so more rows read them again.  Whole MoE block, 16 experts, us with
+// the row tiles of ffn_mfma.hip -> here, even (Zipf 1.1) expert loads:
+//   bf16  1 token 60 -> 40 (60 -> 40), 37 69 -> 56 (68 -> 56), 96 70 -> 58 (69 ->
+//         64), 128 69 -> 59 (70 -> 78), 256 70 -> 83 (73 -> 84)
+//   fp8   1 token 74 -> 44 (73 -> 44), 65 86 -> 58 (86 -> 61), 192 87 -> 63 (87 ->
+//         71), 384 87 -> 82 (91 -> 83), 613 88 -> 114 (95 -> 117)
+bool ffn_small_fits(bool fp8, int64_t rows, int ffn, int experts) {
+    return 2 * rows <= (fp8 ? 24 : 12) * static_cast<int64_t>(experts) && small_kt(fp8, ffn) <= (fp8 ? 4 : 7);
+}
+
+hipError_t launch_ffn_up_small(bool fp8, const uint8_t* x, const float* sx, const uint32_t* offsets,
+                               const uint32_t* assignment_rows, const uint8_t* w13, const float* s1, const float* s3,
+                               bf16_t* act, int64_t rows, int hidden, int ffn, int experts, hipStream_t s) {
+    const dim3 grid = grid_small(rows, experts, ffn / 16);
+    if (fp8)
+        hipLaunchKernelGGL(k_ffn_up_small<Fp8Fmt>, grid, dim3(64), 0, s, x, static_cast<uint32_t>(hidden), offsets,
+                           assignment_rows, w13, act, hidden, ffn, experts, sx, s1, s3);
+    else
+        hipLaunchKernelGGL(k_ffn_up_small<Bf16Fmt>, grid, dim3(64), 0, s, x, static_cast<uint32_t>(hidden) * 2u,
+                           offsets, assignment_rows, w13, act, hidden, ffn, experts, sx, s1, s3);
+    return hipGetLastError();
+}
+
+hipError_t launch_ffn_down_small(bool fp8, const uint8_t* act, const float* sa, const uint32_t* offsets,
+                                 const uint8_t* w2, const float* s2, bf16_t* y, int64_t rows, int hidden, int ffn,
+                                 int experts, hipStream_t s) {
+    const int KT = small_kt(fp8, ffn);
+    const down_small_fn kern = fp8 ? down_small_kernel<Fp8Fmt>(KT) : down_small_kernel<Bf16Fmt>(KT);
+    if (!kern) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(kern, grid_small(rows, experts, hidden / 32), dim3(64), 0, s, act,
+                       static_cast<int64_t>(fp8 ? KT * 128 : ffn * 2), offsets, w2, y, hidden, experts, sa, s2);
+    return hipGetLastError();
+}
+
+}  // namespace aps

@@ -1,0 +1,80 @@
+"""GPU tests of the few-row expert tiles (ffn_small.hip): a batch small enough
+to take them gives, bit for bit, the rows that the same tokens have in a batch
+past the rule, which the 128- and 256-row tiles serve (those are held to the
+oracle elsewhere).  Batches of one token, around the 32-row tile, at the rule's
+edge (2 rows <= 12 experts in bf16, 24 in fp8) and one past it; experts with
+several tiles, one and no row; K shorter and longer than the stages in flight,
+F of one to seven column blocks."""
+import sys
+
+import numpy as np
+import pytest
+import torch
+
+from aps2026_amd import moe, synth
+
+pytestmark = pytest.mark.gpu
+BIG = 700
+
+
+def weights(dtype, E, H, F, dev, seed):
+    g = torch.Generator(device=dev)
+    g.manual_seed(seed)
+    w = [torch.randn((E,) + s, generator=g, device=dev) * 0.05 for s in ((F, H), (H, F), (F, H))]
+    if dtype == "bf16":
+        return moe.register_moe_weights_gpu(*[list(t.bfloat16().unbind(0)) for t in w], compute_dtype=torch.bfloat16)
+    scales = [t.abs().amax(dim=-1) / synth.FP8_E4M3_MAX for t in w]
+    codes = [(t / s[..., None]).to(torch.float8_e4m3fn) for t, s in zip(w, scales)]
+    return moe.register_moe_weights_gpu(*[list(t.unbind(0)) for t in codes], compute_dtype=torch.float8_e4m3fn,
+                                        scales=tuple(list(s.contiguous().unbind(0)) for s in scales))
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "fp8"])
+@pytest.mark.parametrize("E,H,F,skew", [(16, 4096, 448, False), (16, 512, 448, True), (8, 256, 64, True),
+                                        (24, 768, 192, False), (16, 1024, 320, True)])
+def test_few_rows_equal_the_row_tiles(gpu_device, dtype, E, H, F, skew):
+    edge = (24 if dtype == "fp8" else 12) * E // 2
+    print(f"[gpu-case] few rows {dtype} E={E} H={H} F={F} skew={skew} edge={edge}", flush=True)
+    sys.stdout.flush()
+    w = weights(dtype, E, H, F, gpu_device, E + H)
+    g = torch.Generator(device=gpu_device)
+    g.manual_seed(F)
+    x = torch.randn((BIG, H), generator=g, device=gpu_device)
+    gate = torch.randn((E, H), generator=g, device=gpu_device) * 0.05
+    if skew:   # nearly every token to the same two experts
+        x[:, 0] = 4.0
+        gate[1, 0], gate[E - 1, 0] = 8.0, 4.0
+    x = x.bfloat16()
+    big = moe.moe_forward_gpu(x, gate, w).clone()
+    for n in (1, 2, 31, 33, edge, edge + 1):
+        got = moe.moe_forward_gpu(x[:n].contiguous(), gate, w)
+        torch.cuda.synchronize()
+        assert torch.isfinite(got).all()
+        assert torch.equal(got.view(torch.int16), big[:n].view(torch.int16)), n
+    w.release()
+
+
+def test_few_rows_plan_past_two_assignments_per_row(gpu_device):
+    """The staged w1||w3 call with a plan of more positions than 2 rows: the
+    grid covers the rest in further rounds."""
+    from aps2026_amd import capi
+    E, H, F, rows, A = 16, 512, 448, 20, 1500
+    w = weights("bf16", E, H, F, gpu_device, 3)
+    rng = np.random.default_rng(4)
+    x = torch.from_numpy(rng.standard_normal((rows, H)).astype(np.float32)).to(gpu_device).bfloat16()
+    big = x.repeat(40, 1).contiguous()      # 800 rows: the row tiles
+    arows = torch.from_numpy(rng.integers(0, rows, A).astype(np.int32)).to(gpu_device)
+    cuts = np.sort(rng.integers(0, A + 1, E - 1))
+    offsets = torch.from_numpy(np.concatenate([[0], cuts, [A]]).astype(np.int32)).to(gpu_device)
+    out = []
+    for xs in (x, big):
+        act = torch.full((A, F), float("nan"), dtype=torch.bfloat16, device=gpu_device)
+        rc = capi.lib().aps_moe_ffn_up(w.handle, xs.data_ptr(), capi.DTYPE_BF16, xs.shape[0], offsets.data_ptr(),
+                                       arows.data_ptr(), act.data_ptr(), None,
+                                       torch.cuda.current_stream(gpu_device).cuda_stream)
+        assert rc == 0, capi.last_error()
+        torch.cuda.synchronize()
+        out.append(act)
+    assert torch.isfinite(out[0]).all()
+    assert torch.equal(out[0].view(torch.int16), out[1].view(torch.int16))
+    w.release()
