@@ -201,9 +201,10 @@ bool fold_combine(const WeightSet& w, int64_t rows, int32_t out_dtype) {
 }
 
 // xq_ready: the router has written the fp8 codes and scales of x (fp8 path).
+// few: it was the few-token router, which writes no tile histogram.
 int grouped_from_logits(const WeightSet& w, const void* x, bool x_is_f32, const float* logits, int64_t rows,
                         void* out, int32_t out_dtype, char* ws, const aps_moe_ws_layout& L,
-                        hipStream_t s, bool fold = false, bool xq_ready = false) {
+                        hipStream_t s, bool fold = false, bool xq_ready = false, bool few = false) {
     auto* routes = reinterpret_cast<uint8_t*>(ws + L.routes);
     auto* tiles = reinterpret_cast<uint32_t*>(ws + L.tile_counts);
     auto* counts = reinterpret_cast<uint32_t*>(ws + L.counts);
@@ -220,6 +221,7 @@ int grouped_from_logits(const WeightSet& w, const void* x, bool x_is_f32, const 
     auto* slot1 = reinterpret_cast<uint32_t*>(ws + L.slot1);
     auto* srows = reinterpret_cast<uint32_t*>(ws + L.slot_rows);
     auto* stoks = reinterpret_cast<uint32_t*>(ws + L.slot_tokens);
+    if (few) tiles = tiles0 = nullptr;
     if (fold)
         APS_HIP(aps::launch_dispatch_scatter(routes, tiles, rows, w.E, counts, offsets, arows, rpos, nullptr, s,
                                              tiles0, slot1, srows, stoks),
@@ -939,12 +941,18 @@ int aps_moe_forward(uint64_t handle, const void* x, int32_t x_dtype, const float
                               aps::router_quantises_x(w->H, w->E);
     auto* xq = xq_in_router ? reinterpret_cast<uint8_t*>(ws + L.xq) : nullptr;
     auto* xqs = xq_in_router ? reinterpret_cast<float*>(ws + L.xq_scale) : nullptr;
-    APS_HIP(aps::launch_router(x, x_dtype == APS_DTYPE_BF16, gate, rows, w->H, w->E, logits, routes, tiles, tiles0,
-                               xb, xq, xqs, s),
-            "router launch");
-    if (copy) return grouped_from_logits(*w, xb, false, nullptr, rows, out, out_dtype, ws, L, s, fold);
+    const bool few = aps::router_few_fits(rows, w->H, w->E);
+    if (few)
+        APS_HIP(aps::launch_router_few(x, x_dtype == APS_DTYPE_BF16, gate, rows, w->H, w->E, logits, routes, xb, xq,
+                                       xqs, s),
+                "router launch");
+    else
+        APS_HIP(aps::launch_router(x, x_dtype == APS_DTYPE_BF16, gate, rows, w->H, w->E, logits, routes, tiles, tiles0,
+                                   xb, xq, xqs, s),
+                "router launch");
+    if (copy) return grouped_from_logits(*w, xb, false, nullptr, rows, out, out_dtype, ws, L, s, fold, false, few);
     return grouped_from_logits(*w, x, x_dtype == APS_DTYPE_F32, nullptr, rows, out, out_dtype, ws, L, s, fold,
-                               xq_in_router);
+                               xq_in_router, few);
 }
 
 // ---- allocation-free forward --------------------------------------------

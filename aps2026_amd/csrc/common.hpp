@@ -138,6 +138,42 @@ __device__ inline void e4m3_chunk_codes(const e4m3_words_t& w, float sc, float r
     hi = e4m3_pack2<true>(q[6], q[7], e4m3_pack2<false>(q[4], q[5], 0u));
 }
 
+// One wave quantises one row of n bf16 values (n % 8 == 0, n <= 512 * CH): each
+// lane holds up to CH chunks of 8 values.  Writes n codes then zeros up to
+// dst_stride (a multiple of 8), and the row's scale.
+template <int CH>
+__device__ inline void e4m3_quant_row(const bf16_t* __restrict__ s, int n, uint8_t* __restrict__ d8,
+                                      int64_t dst_stride, float* __restrict__ scale, int lane) {
+    typedef uint32_t words2_t __attribute__((ext_vector_type(2)));
+    const int nch = n / 8;
+    e4m3_words_t v[CH];
+    float amax = 0.0f;
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+        const int ch = lane + 64 * c;
+        v[c] = ch < nch ? *reinterpret_cast<const e4m3_words_t*>(s + ch * 8) : e4m3_words_t{0u, 0u, 0u, 0u};
+        amax = e4m3_amax8(amax, v[c]);
+    }
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) amax = fmaxf(amax, __shfl_xor(amax, d));
+    const float sc = e4m3_row_scale(amax);
+    const float rc = __fdiv_rn(1.0f, sc);
+    const bool fast = sc >= kMinFastScale;  // wave-uniform
+    if (lane == 0) *scale = sc;
+    const int dch = static_cast<int>(dst_stride / 8);
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+        const int ch = lane + 64 * c;
+        if (ch >= dch) continue;
+        uint32_t lo = 0, hi = 0;
+        if (ch < nch) {
+            if (fast) e4m3_chunk_codes<true>(v[c], sc, rc, lo, hi);
+            else e4m3_chunk_codes<false>(v[c], sc, rc, lo, hi);
+        }
+        *reinterpret_cast<words2_t*>(d8 + ch * 8) = words2_t{lo, hi};
+    }
+}
+
 // Caller-supplied routes (aps_moe_dispatch) are made memory-safe before they
 // are counted or ranked: an expert id >= E is clamped to E - 1 (and reported
 // by the caller-visible counter), a token whose two slots name the same
@@ -170,6 +206,15 @@ bool router_quantises_x(int hidden, int experts);
 hipError_t launch_router(const void* x, bool x_bf16, const float* gate, int64_t rows, int hidden,
                          int experts, float* logits, uint8_t* routes, uint32_t* tile_counts,
                          uint32_t* tile_counts0, bf16_t* x_copy, uint8_t* xq, float* xq_scale, hipStream_t s);
+// The same logits, routes and x copies for few tokens (router_few.hip), but no
+// tile histogram: the dispatch that follows counts the routes itself
+// (launch_dispatch_scatter with tile_counts == nullptr).
+constexpr int64_t kDispatchFewRows = 256;   // one workgroup of four 64-token tiles
+bool router_few_fits(int64_t rows, int hidden, int experts);
+hipError_t launch_router_few(const void* x, bool x_bf16, const float* gate, int64_t rows, int hidden, int experts,
+                             float* logits, uint8_t* routes, bf16_t* x_copy, uint8_t* xq, float* xq_scale,
+                             hipStream_t s);
+
 hipError_t launch_route_top2(const float* logits, int64_t rows, int experts, uint8_t* routes,
                              uint32_t* tile_counts, hipStream_t s);
 // status (may be null): one u32 that counts the route ids >= experts the

@@ -60,7 +60,7 @@ k_tile_hist(const uint8_t* __restrict__ routes, int64_t rows, int E,
     if (tile < ntiles && lane < E) tile_counts[tile * E + lane] = mine;
 }
 
-template <bool SLOTS>
+template <bool SLOTS, bool COUNT = false>
 __global__ void __launch_bounds__(256)
 k_dispatch_scatter(const uint8_t* __restrict__ routes, const uint32_t* __restrict__ tile_counts,
                    int64_t rows, int E, uint32_t* __restrict__ counts,
@@ -96,8 +96,31 @@ k_dispatch_scatter(const uint8_t* __restrict__ routes, const uint32_t* __restric
     const bool active = lane < tpl * E;
     // [0]: all routes, [1]: slot-0 routes (SLOTS)
     uint32_t tot[2] = {0, 0}, bef0[2] = {0, 0}, bef1[2] = {0, 0}, bef2[2] = {0, 0}, bef3[2] = {0, 0};
+    if constexpr (COUNT) {
+        // one workgroup, no histogram: each wave counts its own tile
+        int first = 255, second = 255;
+        if (t < rows) {
+            first = r0;
+            second = r1;
+            clamp_routes(first, second, E);
+        }
+        for (int e = 0; e < E; ++e) {
+            const int n0 = __popcll(__ballot(first == e)), n1 = __popcll(__ballot(second == e));
+            if (lane == e) {
+                tot[0] = static_cast<uint32_t>(n0 + n1);
+                tot[1] = static_cast<uint32_t>(n0);
+            }
+        }
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {   // bef0: no tile before the first
+            bef1[h] = wave < 1 ? tot[h] : 0u;
+            bef2[h] = wave < 2 ? tot[h] : 0u;
+            bef3[h] = wave < 3 ? tot[h] : 0u;
+        }
+    }
     // eight loads in flight per batch: unconditional (index clamped), used
     // only where the tile exists
+    if constexpr (!COUNT)
     for (int64_t j0 = static_cast<int64_t>(wave) * tpl; j0 < ntiles; j0 += 32 * tpl) {
         uint32_t c[2][8];
 #pragma unroll
@@ -122,7 +145,7 @@ k_dispatch_scatter(const uint8_t* __restrict__ routes, const uint32_t* __restric
     }
 #pragma unroll
     for (int h = 0; h < (SLOTS ? 2 : 1); ++h)
-        for (int d = E; d < 64 && tpl > 1; d <<= 1) {  // lanes e, e + E, e + 2E, ...
+        for (int d = E; !COUNT && d < 64 && tpl > 1; d <<= 1) {  // lanes e, e + E, e + 2E, ...
             tot[h] += __shfl_xor(tot[h], d);
             bef0[h] += __shfl_xor(bef0[h], d);
             bef1[h] += __shfl_xor(bef1[h], d);
@@ -259,8 +282,10 @@ hipError_t launch_dispatch_scatter(const uint8_t* routes, const uint32_t* tile_c
                                    const uint32_t* tile_counts0, uint32_t* slot1, uint32_t* slot_rows,
                                    uint32_t* slot_tokens) {
     if (experts <= 0 || experts > kMaxExperts) return hipErrorInvalidValue;
-    const bool slots = tile_counts0 != nullptr;
-    if (slots && (!slot1 || !slot_rows || !slot_tokens)) return hipErrorInvalidValue;
+    const bool slots = slot1 != nullptr;
+    if (slots && (!slot_rows || !slot_tokens)) return hipErrorInvalidValue;
+    if (slots && (tile_counts != nullptr) != (tile_counts0 != nullptr)) return hipErrorInvalidValue;
+    if (rows > kDispatchFewRows && !tile_counts) return hipErrorInvalidValue;
     if (rows <= 0) {
         // empty batch: counts and offsets are all zero
         hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(128), 0, s, counts, experts);
@@ -270,7 +295,15 @@ hipError_t launch_dispatch_scatter(const uint8_t* routes, const uint32_t* tile_c
     }
     const int64_t ntiles = ceil_div(rows, kWave);
     const dim3 grid(static_cast<unsigned>(ceil_div(ntiles, 4)));
-    if (slots)
+    if (!tile_counts && slots)
+        hipLaunchKernelGGL((k_dispatch_scatter<true, true>), dim3(1), dim3(256), 0, s, routes, nullptr, rows, experts,
+                           counts, offsets, assignment_rows, route_positions, status, nullptr, slot1, slot_rows,
+                           slot_tokens);
+    else if (!tile_counts)
+        hipLaunchKernelGGL((k_dispatch_scatter<false, true>), dim3(1), dim3(256), 0, s, routes, nullptr, rows, experts,
+                           counts, offsets, assignment_rows, route_positions, status, nullptr, nullptr, nullptr,
+                           nullptr);
+    else if (slots)
         hipLaunchKernelGGL(k_dispatch_scatter<true>, grid, dim3(256), 0, s, routes, tile_counts, rows, experts,
                            counts, offsets, assignment_rows, route_positions, status, tile_counts0, slot1,
                            slot_rows, slot_tokens);

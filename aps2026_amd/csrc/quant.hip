@@ -13,51 +13,15 @@
 namespace aps {
 namespace {
 
-typedef e4m3_words_t u32x4_t;
-typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
-
-// The arithmetic (scale, quotient, code) is in common.hpp, shared with the
-// router's x quantisation.
-
-// One wave per row of n bf16 values (n % 8 == 0, n <= 512 * CH): each lane
-// holds up to CH chunks of 8 values.  Writes n codes then zeros up to
-// dst_stride (a multiple of 8), and the row's scale.
+// One wave per row (e4m3_quant_row, common.hpp).
 template <int CH>
 __global__ void __launch_bounds__(64)
 k_quant_rows(const bf16_t* __restrict__ src, int64_t src_stride, int n, uint8_t* __restrict__ dst,
              int64_t dst_stride, float* __restrict__ scale, int64_t rows) {
     const int64_t row = blockIdx.x;
     if (row >= rows) return;
-    const int lane = threadIdx.x;
-    const int nch = n / 8;
-    const bf16_t* s = src + row * src_stride;
-    u32x4_t v[CH];
-    float amax = 0.0f;
-#pragma unroll
-    for (int c = 0; c < CH; ++c) {
-        const int ch = lane + 64 * c;
-        v[c] = ch < nch ? *reinterpret_cast<const u32x4_t*>(s + ch * 8) : u32x4_t{0u, 0u, 0u, 0u};
-        amax = e4m3_amax8(amax, v[c]);
-    }
-#pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) amax = fmaxf(amax, __shfl_xor(amax, d));
-    const float sc = e4m3_row_scale(amax);
-    const float rc = __fdiv_rn(1.0f, sc);
-    const bool fast = sc >= kMinFastScale;  // wave-uniform
-    if (lane == 0) scale[row] = sc;
-    uint8_t* d8 = dst + row * dst_stride;
-    const int dch = static_cast<int>(dst_stride / 8);
-#pragma unroll
-    for (int c = 0; c < CH; ++c) {
-        const int ch = lane + 64 * c;
-        if (ch >= dch) continue;
-        uint32_t lo = 0, hi = 0;
-        if (ch < nch) {
-            if (fast) e4m3_chunk_codes<true>(v[c], sc, rc, lo, hi);
-            else e4m3_chunk_codes<false>(v[c], sc, rc, lo, hi);
-        }
-        *reinterpret_cast<u32x2_t*>(d8 + ch * 8) = u32x2_t{lo, hi};
-    }
+    e4m3_quant_row<CH>(src + row * src_stride, n, dst + row * dst_stride, dst_stride, scale + row,
+                       static_cast<int>(threadIdx.x));
 }
 
 // fp8 weight tile images: 128 rows x 128 bytes (128 k) per image, 16-byte

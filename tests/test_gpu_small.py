@@ -78,3 +78,44 @@ def test_few_rows_plan_past_two_assignments_per_row(gpu_device):
     assert torch.isfinite(out[0]).all()
     assert torch.equal(out[0].view(torch.int16), out[1].view(torch.int16))
     w.release()
+
+
+@pytest.mark.parametrize("dtype,x32", [("bf16", False), ("bf16", True), ("fp8", False), ("f32", True)])
+@pytest.mark.parametrize("E,H", [(16, 4096), (5, 1536), (16, 512), (2, 1024)])
+def test_few_token_router_equals_the_token_major_router(gpu_device, dtype, x32, E, H):
+    """Up to 256 tokens the router takes a workgroup per token and the dispatch
+    counts the routes itself: logits, routes and block outputs are, bit for
+    bit, those of the same tokens in a larger batch, and the plan is the
+    stable sort of the routes (one, full and partly filled 64-token tiles)."""
+    F = 64
+    print(f"[gpu-case] few-token router {dtype} x32={x32} E={E} H={H}", flush=True)
+    sys.stdout.flush()
+    g = torch.Generator(device=gpu_device)
+    g.manual_seed(E * H)
+    if dtype == "f32":
+        ws = [list((torch.randn((E,) + sh, generator=g, device=gpu_device) * 0.05).unbind(0))
+              for sh in ((F, H), (H, F), (F, H))]
+        w = moe.register_moe_weights_gpu(*ws, compute_dtype=torch.float32)
+    else:
+        w = weights(dtype, E, H, F, gpu_device, E + H)
+    x = torch.randn((BIG, H), generator=g, device=gpu_device)
+    gate = torch.randn((E, H), generator=g, device=gpu_device) * 0.05
+    if not x32:
+        x = x.bfloat16()
+    big = moe.moe_forward_gpu(x, gate, w).clone()
+    view = w.plan_views(BIG)
+    logits, routes = view["logits"].clone(), view["routes"].clone()
+    for n in (1, 3, 64, 65, 200, 256, 257):
+        got = moe.moe_forward_gpu(x[:n].contiguous(), gate, w)
+        view = w.plan_views(n)
+        torch.cuda.synchronize()
+        assert torch.equal(view["logits"].view(torch.int32), logits[:n].view(torch.int32)), n
+        assert torch.equal(view["routes"], routes[:n]), n
+        r = routes[:n].cpu().numpy().astype(np.int64).reshape(-1)
+        order = np.argsort(r, kind="stable")
+        assert np.array_equal(view["assignment_rows"].cpu().numpy(), order // 2), n
+        assert np.array_equal(view["route_positions"].cpu().numpy().reshape(-1)[order], np.arange(2 * n)), n
+        assert np.array_equal(view["offsets"].cpu().numpy(), np.searchsorted(r[order], np.arange(E + 1))), n
+        bits = torch.int32 if got.dtype == torch.float32 else torch.int16
+        assert torch.equal(got.view(bits), big[:n].view(bits)), n
+    w.release()
