@@ -222,11 +222,15 @@ int grouped_from_logits(const WeightSet& w, const void* x, bool x_is_f32, const 
     auto* srows = reinterpret_cast<uint32_t*>(ws + L.slot_rows);
     auto* stoks = reinterpret_cast<uint32_t*>(ws + L.slot_tokens);
     if (few) tiles = tiles0 = nullptr;
-    if (fold)
+    // few tokens on the one-wave tiles: the w1||w3 launch makes the plan itself
+    const aps::SmallPlan plan{routes, counts, offsets, arows, rpos, fold ? slot1 : nullptr, srows, stoks};
+    const bool planned = few && w.compute != APS_DTYPE_F32 &&
+                         aps::ffn_small_fits(w.compute == APS_DTYPE_E4M3, rows, w.F, w.E);
+    if (!planned && fold)
         APS_HIP(aps::launch_dispatch_scatter(routes, tiles, rows, w.E, counts, offsets, arows, rpos, nullptr, s,
                                              tiles0, slot1, srows, stoks),
                 "dispatch launch");
-    else
+    else if (!planned)
         APS_HIP(aps::launch_dispatch_scatter(routes, tiles, rows, w.E, counts, offsets, arows, rpos, nullptr, s),
                 "dispatch launch");
     if (w.compute == APS_DTYPE_E4M3) {
@@ -239,8 +243,13 @@ int grouped_from_logits(const WeightSet& w, const void* x, bool x_is_f32, const 
         if (!xq_ready)
             APS_HIP(aps::launch_quant_rows_e4m3(static_cast<const aps::bf16_t*>(x), w.H, w.H, xq, w.H, xs, rows, s),
                     "quantise x launch");
-        APS_HIP(aps::launch_ffn_up_fp8(xq, xs, offsets, arows, w.q13, w.s1, w.s3, act, rows, w.H, w.F, w.E, s),
-                "ffn_up_fp8 launch");
+        if (planned)
+            APS_HIP(aps::launch_ffn_up_small(true, xq, xs, nullptr, nullptr, &plan, w.q13, w.s1, w.s3, act, rows, w.H,
+                                             w.F, w.E, s),
+                    "ffn_up_fp8 launch");
+        else
+            APS_HIP(aps::launch_ffn_up_fp8(xq, xs, offsets, arows, w.q13, w.s1, w.s3, act, rows, w.H, w.F, w.E, s),
+                    "ffn_up_fp8 launch");
         APS_HIP(aps::launch_quant_rows_e4m3(act, w.F, w.F, actq, kp, as, 2 * rows, s), "quantise act launch");
         // few rows: the one-wave w2 tiles and the combine (the fold's two
         // passes over all of w2 cost more than y's round trip)
@@ -256,6 +265,12 @@ int grouped_from_logits(const WeightSet& w, const void* x, bool x_is_f32, const 
         APS_HIP(aps::launch_ffn_down_fp8(actq, as, offsets, w.q2, w.s2, reinterpret_cast<aps::bf16_t*>(ws + L.y),
                                          rows, w.H, w.F, w.E, s),
                 "ffn_down_fp8 launch");
+    } else if (planned) {
+        APS_HIP(aps::launch_ffn_up_small(false, static_cast<const uint8_t*>(x), nullptr, nullptr, nullptr, &plan,
+                                         reinterpret_cast<const uint8_t*>(w.w13), nullptr, nullptr,
+                                         reinterpret_cast<aps::bf16_t*>(ws + L.act), rows, w.H, w.F, w.E, s),
+                "ffn_up_bf16 launch");
+        if (int rc = run_ffn_down(w, ws + L.act, rows, offsets, ws + L.y, s)) return rc;
     } else {
         int rc = run_ffn(w, x, rows, offsets, arows, ws + L.act, ws + L.y, s);
         if (rc) return rc;

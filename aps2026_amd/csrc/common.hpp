@@ -331,9 +331,17 @@ bool ffn_down_fold_fits(int64_t rows, int hidden, int ffn);
 // One-wave tiles for few rows (ffn_small.hip): the rule and the launches that
 // the bf16 and fp8 launchers above take under it.
 bool ffn_small_fits(bool fp8, int64_t rows, int ffn, int experts);
+// plan (null: offsets and assignment_rows are given): the routes to sort and
+// where the plan goes, slot1 .. slot_tokens null unless wanted; rows <=
+// kDispatchFewRows.
+struct SmallPlan {
+    const uint8_t* routes;
+    uint32_t *counts, *offsets, *assignment_rows, *route_positions, *slot1, *slot_rows, *slot_tokens;
+};
 hipError_t launch_ffn_up_small(bool fp8, const uint8_t* x, const float* sx, const uint32_t* offsets,
-                               const uint32_t* assignment_rows, const uint8_t* w13, const float* s1, const float* s3,
-                               bf16_t* act, int64_t rows, int hidden, int ffn, int experts, hipStream_t s);
+                               const uint32_t* assignment_rows, const SmallPlan* plan, const uint8_t* w13,
+                               const float* s1, const float* s3, bf16_t* act, int64_t rows, int hidden, int ffn,
+                               int experts, hipStream_t s);
 hipError_t launch_ffn_down_small(bool fp8, const uint8_t* act, const float* sa, const uint32_t* offsets,
                                  const uint8_t* w2, const float* s2, bf16_t* y, int64_t rows, int hidden, int ffn,
                                  int experts, hipStream_t s);

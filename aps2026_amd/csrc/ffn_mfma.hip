@@ -1280,7 +1280,7 @@ hipError_t launch_ffn_up_bf16(const bf16_t* x, const uint32_t* offsets,
     if (hidden % 64 != 0 || ffn % 64 != 0) return hipErrorInvalidValue;
     if (ffn_small_fits(false, rows, ffn, experts))
         return launch_ffn_up_small(false, reinterpret_cast<const uint8_t*>(x), nullptr, offsets, assignment_rows,
-                                   reinterpret_cast<const uint8_t*>(w13), nullptr, nullptr, act, rows, hidden, ffn,
+                                   nullptr, reinterpret_cast<const uint8_t*>(w13), nullptr, nullptr, act, rows, hidden, ffn,
                                    experts, s);
     hipLaunchKernelGGL(k_ffn_up<Bf16Fmt>, grid_up(), dim3(256), 0, s,
                        reinterpret_cast<const uint8_t*>(x), static_cast<int64_t>(hidden) * 2, offsets,
@@ -1318,7 +1318,7 @@ hipError_t launch_ffn_up_fp8(const uint8_t* xq, const float* x_scale, const uint
     if (rows <= 0) return hipSuccess;
     if (hidden % 128 != 0 || ffn % 64 != 0) return hipErrorInvalidValue;
     if (ffn_small_fits(true, rows, ffn, experts))
-        return launch_ffn_up_small(true, xq, x_scale, offsets, assignment_rows, w13, w1_scale, w3_scale, act, rows,
+        return launch_ffn_up_small(true, xq, x_scale, offsets, assignment_rows, nullptr, w13, w1_scale, w3_scale, act, rows,
                                    hidden, ffn, experts, s);
     hipLaunchKernelGGL(k_ffn_up<Fp8Fmt>, grid_up(), dim3(256), 0, s,
                        xq, static_cast<int64_t>(hidden), offsets, assignment_rows, w13, act, hidden, ffn, experts,

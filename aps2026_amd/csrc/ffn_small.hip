@@ -39,14 +39,13 @@ struct SmallTile {
 
 // Tile b of the list expert -> column group -> 32-row tile, dealt to the XCDs
 // in contiguous slices (workgroup b runs on XCD b % 8), so that the row tiles
-// of an expert read a weight tile in one L2.  `bn`: column groups.  A block
-// takes every (gridDim.x / 8)-th tile of its slice; the grid covers 2 rows
-// assignments in one round, a caller's plan may hold more.
+// of an expert read a weight tile in one L2.  lo, hi: this lane's expert's
+// positions (lane = expert, 0 past the last); `bn`: column groups.  A block of
+// `blocks` takes every (blocks / 8)-th tile of its slice; the grid covers 2
+// rows assignments in one round, a caller's plan may hold more.
 template <class Body>
-__device__ inline void each_small(const uint32_t* __restrict__ offsets, int E, int bn, Body body) {
+__device__ inline void each_small(uint32_t lo, uint32_t hi, int bn, int blocks, Body body) {
     const int lane = threadIdx.x & 63;
-    const uint32_t lo = lane < E ? offsets[lane] : 0u;
-    const uint32_t hi = lane < E ? offsets[lane + 1] : 0u;
     const int tiles = static_cast<int>((hi - lo + kSmRows - 1) / kSmRows);
     int incl = tiles * bn;
 #pragma unroll
@@ -57,7 +56,7 @@ __device__ inline void each_small(const uint32_t* __restrict__ offsets, int E, i
     const int total = __shfl(incl, 63);
     const int per = (total + kSmXcds - 1) / kSmXcds;
     const int first = static_cast<int>(blockIdx.x % kSmXcds) * per;
-    for (int l = static_cast<int>(blockIdx.x) / kSmXcds; l < per; l += static_cast<int>(gridDim.x) / kSmXcds) {
+    for (int l = static_cast<int>(blockIdx.x) / kSmXcds; l < per; l += blocks / kSmXcds) {
         const int t = first + l;
         if (t >= total) return;
         const int e = __ffsll(static_cast<unsigned long long>(__ballot(incl > t))) - 1;
@@ -70,6 +69,122 @@ __device__ inline void each_small(const uint32_t* __restrict__ offsets, int E, i
         u.end = __builtin_amdgcn_readfirstlane(__shfl(hi, e));
         body(u);
     }
+}
+
+// ---- the routing plan inside the w1||w3 launch ------------------------------
+// After the few-token router the plan (dispatch.hip states it) is a stable sort
+// of at most 512 route bytes: every wave of the w1||w3 launch counts the routes
+// itself and ranks those of its own expert, and one further block writes the
+// plan out for the kernels after it.  That saves the dispatch's launch between
+// the router and the GEMM for 1 us in it: one bf16 token 35.0 -> 33.2 us a block,
+// 37 tokens 52.0 -> 49.9, fp8 65 tokens 45.9 -> 43.6.
+constexpr int kPlanTiles = static_cast<int>(kDispatchFewRows / kWave);
+
+struct Routes {
+    int first[kPlanTiles], second[kPlanTiles];   // token 64 k + lane (255: none)
+    int nt;                                      // 64-token tiles
+    __device__ void load(const uint8_t* __restrict__ routes, int64_t rows) {
+        nt = static_cast<int>((rows + kWave - 1) / kWave);
+#pragma unroll
+        for (int k = 0; k < kPlanTiles; ++k) {
+            const int64_t t = kWave * k + (threadIdx.x & 63);
+            first[k] = t < rows ? routes[2 * t] : 255;
+            second[k] = t < rows ? routes[2 * t + 1] : 255;
+        }
+    }
+    __device__ uint64_t slot0(int k, int e) const { return __ballot(first[k] == e); }
+    __device__ uint64_t slot1(int k, int e) const { return __ballot(second[k] == e); }
+};
+
+// This lane's expert's positions [lo, hi), counted from the routes.
+__device__ inline void plan_counts(const Routes& r, int E, uint32_t& lo, uint32_t& hi) {
+    const int lane = threadIdx.x & 63;
+    uint32_t run = 0;
+    lo = hi = 0;
+    for (int e = 0; e < E; ++e) {
+        uint32_t n = 0;
+#pragma unroll
+        for (int k = 0; k < kPlanTiles; ++k)
+            if (k < r.nt) n += static_cast<uint32_t>(__popcll(r.slot0(k, e)) + __popcll(r.slot1(k, e)));
+        if (lane == e) {
+            lo = run;
+            hi = run + n;
+        }
+        run += n;
+    }
+}
+
+// The whole plan, by one wave (router's routes: two distinct experts a token).
+__device__ inline void plan_write(const Routes& r, int64_t rows, int E, uint32_t lo, uint32_t hi, const SmallPlan& p) {
+    const int lane = threadIdx.x & 63;
+    const uint64_t below = (1ull << lane) - 1ull;
+    uint32_t p0[kPlanTiles], p1[kPlanTiles], i0[kPlanTiles], i1[kPlanTiles];
+    for (int e = 0; e < E; ++e) {
+        uint32_t at = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(lo), e));
+        uint32_t n0 = 0;
+#pragma unroll
+        for (int k = 0; k < kPlanTiles; ++k)
+            if (k < r.nt) n0 += static_cast<uint32_t>(__popcll(r.slot0(k, e)));
+        uint32_t l0 = at, l1 = at + n0;   // slot-0 routes of e, then its slot-1 routes
+        if (lane == 0 && p.slot1) p.slot1[e] = l1;
+#pragma unroll
+        for (int k = 0; k < kPlanTiles; ++k) {
+            if (k >= r.nt) continue;   // wave-uniform
+            const uint64_t m0 = r.slot0(k, e), m1 = r.slot1(k, e);
+            const uint32_t b0 = static_cast<uint32_t>(__popcll(m0 & below)), b1 = static_cast<uint32_t>(__popcll(m1 & below));
+            if (r.first[k] == e) {
+                p0[k] = at + b0 + b1;
+                i0[k] = l0 + b0;
+            }
+            if (r.second[k] == e) {
+                p1[k] = at + b0 + b1;
+                i1[k] = l1 + b1;
+            }
+            at += static_cast<uint32_t>(__popcll(m0) + __popcll(m1));
+            l0 += static_cast<uint32_t>(__popcll(m0));
+            l1 += static_cast<uint32_t>(__popcll(m1));
+        }
+    }
+    if (lane < E) {
+        p.counts[lane] = hi - lo;
+        p.offsets[lane] = lo;
+        if (lane == E - 1) p.offsets[E] = hi;
+    }
+#pragma unroll
+    for (int k = 0; k < kPlanTiles; ++k) {
+        const uint32_t t = static_cast<uint32_t>(kWave * k + lane);
+        if (t >= rows) continue;
+        p.assignment_rows[p0[k]] = t;
+        p.assignment_rows[p1[k]] = t;
+        p.route_positions[2 * t] = p0[k];
+        p.route_positions[2 * t + 1] = p1[k];
+        if (p.slot1) {
+            p.slot_rows[i0[k]] = p0[k];
+            p.slot_tokens[i0[k]] = t;
+            p.slot_rows[i1[k]] = p1[k];
+            p.slot_tokens[i1[k]] = t;
+        }
+    }
+}
+
+// Token of row (lane % 32) of tile u, through tok[32] in LDS; rows past the
+// expert's end get its last token.
+__device__ inline uint32_t plan_token(const Routes& r, uint32_t expert_lo, const SmallTile& u, uint32_t* tok) {
+    const int lane = threadIdx.x & 63;
+    const uint64_t below = (1ull << lane) - 1ull;
+    uint32_t at = expert_lo;
+    __builtin_amdgcn_wave_barrier();   // the previous tile's reads come first
+#pragma unroll
+    for (int k = 0; k < kPlanTiles; ++k) {
+        if (k >= r.nt) continue;   // wave-uniform
+        const uint64_t m = r.slot0(k, u.expert) | r.slot1(k, u.expert);
+        const uint32_t i = at + static_cast<uint32_t>(__popcll(m & below)) - u.m0;   // wraps for rows before m0
+        if ((m >> lane & 1) && i < static_cast<uint32_t>(kSmRows)) tok[i] = static_cast<uint32_t>(kWave * k + lane);
+        at += static_cast<uint32_t>(__popcll(m));
+    }
+    __builtin_amdgcn_wave_barrier();   // (a wave's LDS accesses complete in order)
+    const uint32_t n = u.end - u.m0, row = lane & 31;
+    return tok[row < n ? row : n - 1];
 }
 
 // One 128-byte stage of a lane's row: kSub fragments, each 16 (bf16) or 32
@@ -96,19 +211,40 @@ __device__ inline void small_load(SmallStage<Fmt>& d, At at) {
     }
 }
 
-// act[p][n], as ffn_mfma.hip's up_piece.
-template <class Fmt>
+// act[p][n], as ffn_mfma.hip's up_piece.  ROUTES: the plan comes from
+// plan.routes and the last block writes it out; else from offsets and
+// assignment_rows.
+template <class Fmt, bool ROUTES>
 __global__ void __launch_bounds__(64, 1)
 k_ffn_up_small(const uint8_t* __restrict__ x, uint32_t x_row_bytes, const uint32_t* __restrict__ offsets,
-               const uint32_t* __restrict__ assignment_rows, const uint8_t* __restrict__ w13,
-               bf16_t* __restrict__ act, int H, int F, int E, const float* __restrict__ sx,
-               const float* __restrict__ s1, const float* __restrict__ s3) {
+               const uint32_t* __restrict__ assignment_rows, const SmallPlan plan, int64_t rows,
+               const uint8_t* __restrict__ w13, bf16_t* __restrict__ act, int H, int F, int E,
+               const float* __restrict__ sx, const float* __restrict__ s1, const float* __restrict__ s3) {
     constexpr bool kFp8 = Fmt::kElt == 1;
-    each_small(offsets, E, F / 16, [&](const SmallTile& u) __attribute__((always_inline)) {
+    __shared__ uint32_t tok[ROUTES ? kSmRows : 1];
     const int lane = threadIdx.x, r = lane & 31, h = lane >> 5;
+    const int blocks = static_cast<int>(gridDim.x) - (ROUTES ? 1 : 0);
+    uint32_t lo, hi;
+    Routes routes;
+    if constexpr (ROUTES) {
+        routes.load(plan.routes, rows);
+        plan_counts(routes, E, lo, hi);
+        if (static_cast<int>(blockIdx.x) == blocks) {   // block-uniform
+            plan_write(routes, rows, E, lo, hi, plan);
+            return;
+        }
+    } else {
+        lo = lane < E ? offsets[lane] : 0u;
+        hi = lane < E ? offsets[lane + 1] : 0u;
+    }
+    each_small(lo, hi, F / 16, blocks, [&](const SmallTile& u) __attribute__((always_inline)) {
     const int KT = H * Fmt::kElt / kRowBytes;
     const uint32_t p = u.m0 + r < u.end ? u.m0 + r : u.end - 1;
-    const uint32_t token = assignment_rows[p];
+    uint32_t token;
+    if constexpr (ROUTES)
+        token = plan_token(routes, static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(lo), u.expert)), u,
+                           tok);
+    else token = assignment_rows[p];
     // image row of this lane: gate row 16 (col % 4) + r, then the same up rows
     const int ir = 16 * (u.col & 3) + (r < 16 ? r : 64 + (r - 16));
     const uint8_t* image = w13 + (static_cast<int64_t>(u.expert) * (F / 64) + u.col / 4) * KT * kImageBytes;
@@ -175,8 +311,9 @@ k_ffn_down_small(const uint8_t* __restrict__ act, int64_t act_row_bytes, const u
                  const uint8_t* __restrict__ w2, bf16_t* __restrict__ y, int H, int E, const float* __restrict__ sa,
                  const float* __restrict__ s2) {
     constexpr bool kFp8 = Fmt::kElt == 1;
-    each_small(offsets, E, H / 32, [&](const SmallTile& u) __attribute__((always_inline)) {
     const int lane = threadIdx.x, r = lane & 31, h = lane >> 5;
+    const uint32_t lo = lane < E ? offsets[lane] : 0u, hi = lane < E ? offsets[lane + 1] : 0u;
+    each_small(lo, hi, H / 32, static_cast<int>(gridDim.x), [&](const SmallTile& u) __attribute__((always_inline)) {
     const uint32_t p = u.m0 + r < u.end ? u.m0 + r : u.end - 1;
     const uint8_t* image = w2 + (static_cast<int64_t>(u.expert) * (H / 128) + u.col / 4) * KT * kImageBytes;
     const uint8_t* arow = act + static_cast<int64_t>(p) * act_row_bytes;
@@ -258,15 +395,17 @@ bool ffn_small_fits(bool fp8, int64_t rows, int ffn, int experts) {
 }
 
 hipError_t launch_ffn_up_small(bool fp8, const uint8_t* x, const float* sx, const uint32_t* offsets,
-                               const uint32_t* assignment_rows, const uint8_t* w13, const float* s1, const float* s3,
-                               bf16_t* act, int64_t rows, int hidden, int ffn, int experts, hipStream_t s) {
-    const dim3 grid = grid_small(rows, experts, ffn / 16);
-    if (fp8)
-        hipLaunchKernelGGL(k_ffn_up_small<Fp8Fmt>, grid, dim3(64), 0, s, x, static_cast<uint32_t>(hidden), offsets,
-                           assignment_rows, w13, act, hidden, ffn, experts, sx, s1, s3);
-    else
-        hipLaunchKernelGGL(k_ffn_up_small<Bf16Fmt>, grid, dim3(64), 0, s, x, static_cast<uint32_t>(hidden) * 2u,
-                           offsets, assignment_rows, w13, act, hidden, ffn, experts, sx, s1, s3);
+                               const uint32_t* assignment_rows, const SmallPlan* plan, const uint8_t* w13,
+                               const float* s1, const float* s3, bf16_t* act, int64_t rows, int hidden, int ffn,
+                               int experts, hipStream_t s) {
+    if (plan && (rows > kDispatchFewRows || experts > kWave)) return hipErrorInvalidValue;
+    dim3 grid = grid_small(rows, experts, ffn / 16);
+    const uint32_t row_bytes = static_cast<uint32_t>(hidden) * (fp8 ? 1u : 2u);
+    if (plan) ++grid.x;
+    auto kern = fp8 ? (plan ? k_ffn_up_small<Fp8Fmt, true> : k_ffn_up_small<Fp8Fmt, false>)
+                    : (plan ? k_ffn_up_small<Bf16Fmt, true> : k_ffn_up_small<Bf16Fmt, false>);
+    hipLaunchKernelGGL(kern, grid, dim3(64), 0, s, x, row_bytes, offsets, assignment_rows, plan ? *plan : SmallPlan{},
+                       rows, w13, act, hidden, ffn, experts, sx, s1, s3);
     return hipGetLastError();
 }
 
