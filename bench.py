@@ -401,7 +401,7 @@ def decoder_bench(args):
             t_plan.append(time.perf_counter() - t1)
         stages["prefix_trie_and_upload_ms"] = statistics.median(t_plan) * 1e3
     # the projections dominate: one fp32 FMA chain per output (the reference's
-    # order) as chains of K = 1 fp32 MFMAs; MI355X's published fp32 matrix
+    # order) as fp32 MFMA chains; MI355X's published fp32 matrix
     # rate is 157.3 TFLOP/s
     proj_s = mt["qkv_proj"] + mt["o_proj"]
     if layer0.tc:
