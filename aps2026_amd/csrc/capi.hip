@@ -195,7 +195,8 @@ int check_x_dtype(const WeightSet& w, int32_t x_dtype) {
 // Routing (from `logits`; nullptr when the router kernel already wrote the
 // routes and tile histogram into the workspace), dispatch, FFN and combine.
 // The fp8 path with bf16 output folds the combine into the w2 GEMM when the
-// router wrote the slot-0 histogram (aps_moe_forward): no y round trip.
+// router wrote the slot-0 histogram (aps_moe_forward) and the batch is large:
+// no y round trip.  The slot lists are in the workspace at any size.
 bool fold_combine(const WeightSet& w, int64_t rows, int32_t out_dtype) {
     return w.compute == APS_DTYPE_E4M3 && out_dtype == APS_DTYPE_BF16 && aps::ffn_down_fold_fits(rows, w.H, w.F);
 }
@@ -251,9 +252,12 @@ int grouped_from_logits(const WeightSet& w, const void* x, bool x_is_f32, const 
             APS_HIP(aps::launch_ffn_up_fp8(xq, xs, offsets, arows, w.q13, w.s1, w.s3, act, rows, w.H, w.F, w.E, s),
                     "ffn_up_fp8 launch");
         APS_HIP(aps::launch_quant_rows_e4m3(act, w.F, w.F, actq, kp, as, 2 * rows, s), "quantise act launch");
-        // few rows: the one-wave w2 tiles and the combine (the fold's two
-        // passes over all of w2 cost more than y's round trip)
-        if (fold && !aps::ffn_small_fits(true, rows, w.F, w.E)) {
+        // up to 384 routes per expert w2 runs unfolded: the fold's second pass over
+        // all of w2 costs more than y's round trip.  Whole block, 16
+        // experts, us folded -> unfolded, even (Zipf 1.1) loads: 320 tokens 87 -> 68
+        // (90 -> 71), 1024 92 -> 78 (98 -> 81), 2048 111 -> 107 (122 -> 107), 3072 118
+        // -> 114 (127 -> 119), 4096 131 -> 133 (145 -> 136), 8192 223 -> 234 (223 -> 235)
+        if (fold && 2 * rows > 384 * static_cast<int64_t>(w.E)) {
             // slot-0 rows to y's bytes as [rows][H] by token, then slot-1 rows
             // combined with them straight into out
             APS_HIP(aps::launch_ffn_down_fold_fp8(actq, as, offsets, slot1, srows, stoks, w.q2, w.s2,

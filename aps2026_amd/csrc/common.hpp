@@ -330,7 +330,8 @@ hipError_t launch_ffn_down_fp8(const uint8_t* actq, const float* act_scale, cons
 bool ffn_down_fold_fits(int64_t rows, int hidden, int ffn);
 // One-wave tiles for few rows (ffn_small.hip): the rule and the launches that
 // the bf16 and fp8 launchers above take under it.
-bool ffn_small_fits(bool fp8, int64_t rows, int ffn, int experts);
+bool ffn_small_fits(bool fp8, int64_t rows, int ffn, int experts);        // w1||w3
+bool ffn_down_small_fits(bool fp8, int64_t rows, int ffn, int experts);   // w2
 // plan (null: offsets and assignment_rows are given): the routes to sort and
 // where the plan goes, slot1 .. slot_tokens null unless wanted; rows <=
 // kDispatchFewRows.

@@ -1294,7 +1294,7 @@ hipError_t launch_ffn_down_bf16(const bf16_t* act, const uint32_t* offsets, cons
                                 hipStream_t s) {
     if (rows <= 0) return hipSuccess;
     if (hidden % 128 != 0 || ffn % 64 != 0) return hipErrorInvalidValue;
-    if (ffn_small_fits(false, rows, ffn, experts))
+    if (ffn_down_small_fits(false, rows, ffn, experts))
         return launch_ffn_down_small(false, reinterpret_cast<const uint8_t*>(act), nullptr, offsets,
                                      reinterpret_cast<const uint8_t*>(w2), nullptr, y, rows, hidden, ffn, experts, s);
     if (auto kern = down_ar_kernel<Bf16Fmt>(ffn / 64)) {
@@ -1331,7 +1331,7 @@ hipError_t launch_ffn_down_fp8(const uint8_t* actq, const float* act_scale, cons
                                int ffn, int experts, hipStream_t s) {
     if (rows <= 0) return hipSuccess;
     if (hidden % 128 != 0 || ffn % 64 != 0) return hipErrorInvalidValue;
-    if (ffn_small_fits(true, rows, ffn, experts))
+    if (ffn_down_small_fits(true, rows, ffn, experts))
         return launch_ffn_down_small(true, actq, act_scale, offsets, w2, w2_scale, y, rows, hidden, ffn, experts, s);
     const int kpad = static_cast<int>(ceil_div(ffn, 128) * 128);
     if (auto kern = down_ar_kernel<Fp8Fmt>(kpad / 128)) {

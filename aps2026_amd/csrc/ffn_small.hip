@@ -394,6 +394,17 @@ bool ffn_small_fits(bool fp8, int64_t rows, int ffn, int experts) {
     return 2 * rows <= (fp8 ? 24 : 12) * static_cast<int64_t>(experts) && small_kt(fp8, ffn) <= (fp8 ? 4 : 7);
 }
 
+// w2's whole K is in flight at once and its tiles read less again, so it gains
+// up to 24 rows per expert in bf16 and 32, a full tile, in fp8.  Whole block, 16
+// experts, us with the row tiles of w2 -> here, even (Zipf 1.1) loads:
+//   bf16  97 tokens 75 -> 69 (75 -> 73), 192 77 -> 72 (77 -> 76), 256 78 -> 77 (83 ->
+//         85), 512 83 -> 91 (95 -> 100)
+//   fp8   224 tokens 56 -> 51 (57 -> 54), 256 56 -> 53 (59 -> 58), 384 69 -> 70 (73 ->
+//         73), 613 71 -> 77 (78 -> 80)
+bool ffn_down_small_fits(bool fp8, int64_t rows, int ffn, int experts) {
+    return 2 * rows <= (fp8 ? 32 : 24) * static_cast<int64_t>(experts) && small_kt(fp8, ffn) <= (fp8 ? 4 : 7);
+}
+
 hipError_t launch_ffn_up_small(bool fp8, const uint8_t* x, const float* sx, const uint32_t* offsets,
                                const uint32_t* assignment_rows, const SmallPlan* plan, const uint8_t* w13,
                                const float* s1, const float* s3, bf16_t* act, int64_t rows, int hidden, int ffn,

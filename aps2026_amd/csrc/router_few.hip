@@ -14,7 +14,8 @@
 // launch here and runs once.
 //   Bound by the chain (4096 steps: 11 us).  Measured at H = 4096, against the
 // token-major kernel: bf16 x 19 -> 14 us, with its fp8 codes 27 -> 15.5 us, fp32 x 24
-// -> 16 us; any count up to 256 tokens, past which workgroups share SIMDs.
+// -> 16 us; any count up to 256 tokens.  Past that workgroups share SIMDs (bf16
+// block of 300 tokens 81 -> 88 us, 613 85 -> 105).
 //   A workgroup's four waves are the 16 experts of one token.  The fp8 codes
 // of x come from further workgroups of the same launch, beside the chains
 // instead of after them.

@@ -120,6 +120,13 @@ def test_fold_f_widths_and_single_slot_experts(gpu_device):
         check(inp, gpu_device)
 
 
+@pytest.mark.parametrize("T,E,F", [(384, 2, 448), (385, 2, 512), (577, 3, 448), (3072, 16, 448), (3073, 16, 512)])
+def test_fold_at_its_row_rule(gpu_device, T, E, F):
+    """w2 folds past 384 routes per expert on average: both sides of the line."""
+    note(f"fold rule fp8 T={T} E={E} F={F}")
+    check(synth.make_moe_inputs(T=T, H=1024, E=E, F=F, dtype="fp8", seed=31 + T, name="fold-rule"), gpu_device)
+
+
 def test_fp32_output_takes_the_unfolded_path(gpu_device):
     inp = synth.make_moe_inputs(T=300, H=1024, E=16, F=448, dtype="fp8", seed=5, name="fold-f32")
     w = fp8_weights(inp, gpu_device)

@@ -54,6 +54,29 @@ def test_few_rows_equal_the_row_tiles(gpu_device, dtype, E, H, F, skew):
     w.release()
 
 
+@pytest.mark.parametrize("E,H,F", [(16, 4096, 448), (16, 512, 64), (8, 256, 320), (24, 768, 512)])
+@pytest.mark.parametrize("dtype", ["bf16", "fp8"])
+def test_w2_tiles_between_the_rules(gpu_device, dtype, E, H, F):
+    """w2 stays on the one-wave tiles past the w1||w3 rule, up to 24 (bf16) or
+    32 (fp8) routes per expert: that edge and one past it, against a batch of
+    row tiles."""
+    edge = (32 if dtype == "fp8" else 24) * E // 2
+    print(f"[gpu-case] w2 tiles {dtype} E={E} H={H} F={F} edge={edge}", flush=True)
+    w = weights(dtype, E, H, F, gpu_device, E * F)
+    g = torch.Generator(device=gpu_device)
+    g.manual_seed(H)
+    x = torch.randn((BIG, H), generator=g, device=gpu_device).bfloat16()
+    gate = torch.randn((E, H), generator=g, device=gpu_device) * 0.05
+    for out in (torch.bfloat16, torch.float32):
+        bits = torch.int16 if out == torch.bfloat16 else torch.int32
+        big = moe.moe_forward_gpu(x, gate, w, out_dtype=out).clone()
+        for n in (edge - 31, edge, edge + 1):
+            got = moe.moe_forward_gpu(x[:n].contiguous(), gate, w, out_dtype=out)
+            torch.cuda.synchronize()
+            assert torch.equal(got.view(bits), big[:n].view(bits)), n
+    w.release()
+
+
 def test_few_rows_plan_past_two_assignments_per_row(gpu_device):
     """The staged w1||w3 call with a plan of more positions than 2 rows: the
     grid covers the rest in further rounds."""
