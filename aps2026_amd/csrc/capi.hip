@@ -960,7 +960,9 @@ int aps_moe_forward(uint64_t handle, const void* x, int32_t x_dtype, const float
                               aps::router_quantises_x(w->H, w->E);
     auto* xq = xq_in_router ? reinterpret_cast<uint8_t*>(ws + L.xq) : nullptr;
     auto* xqs = xq_in_router ? reinterpret_cast<float*>(ws + L.xq_scale) : nullptr;
-    const bool few = aps::router_few_fits(rows, w->H, w->E);
+    // (the few-token router copies fp32 x 16 bytes at a time)
+    const bool few = aps::router_few_fits(rows, w->H, w->E) &&
+                     (x_dtype == APS_DTYPE_BF16 || (reinterpret_cast<uintptr_t>(x) & 15u) == 0);
     if (few)
         APS_HIP(aps::launch_router_few(x, x_dtype == APS_DTYPE_BF16, gate, rows, w->H, w->E, logits, routes, xb, xq,
                                        xqs, s),

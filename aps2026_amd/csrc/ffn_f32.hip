@@ -9,8 +9,8 @@
 // These kernels keep exactly that arithmetic, so for fp32 weights the result
 // equals the CPU oracle bit for bit (the only libm call, exp in double, is
 // rounded to float afterwards).  The chains run on the fp32 MFMAs, which give
-// the same bits (chain_mfma.hpp); k_linear_any, for Linear shapes those do not
-// take, is a SIMT kernel.
+// the same bits (chain_mfma.hpp); arrays that are not 16-byte aligned, and
+// Linear shapes those do not take, run on SIMT kernels.
 #include "chain_mfma.hpp"
 
 namespace aps {
@@ -154,62 +154,107 @@ k_ffn_down_f32(const float* __restrict__ act, const uint32_t* __restrict__ offse
     }
 }
 
-// y[m][n] = (fp32 FMA chain over k ascending of x[m][k] w[n][k]) + bias[n] for
-// any K, N and alignment (the reference's fallback for
-// shapes its fast kernels do not take, k_matmul_transposed_tiled,
-// src/tensor.cu:433-461): scalar loads, k past K read as zero.  A padded step
-// adds the exact product 0 * 0 to an accumulator that is never -0 (it starts
-// at +0, and a sum that cancels exactly rounds to +0), so it changes no bit:
-// every output is the chain over k = 0 .. K-1.  Row tiles are walked
-// grid-stride over gridDim.y.
-__global__ void __launch_bounds__(256)
-k_linear_any(const float* __restrict__ x, const float* __restrict__ w, const float* __restrict__ bias,
-             float* __restrict__ y, int64_t M, int K, int N) {
-    __shared__ float As[kBK][kF32BM + 1];
-    __shared__ float Bs[kBK][kF32BN + 1];
-    const int n0 = blockIdx.x * kF32BN;
-    const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
-    const int sr = tid >> 2, sk = (tid & 3) * 4;
-    const bool b_ok = n0 + sr < N;
-    const float* b_src = w + static_cast<int64_t>(b_ok ? n0 + sr : 0) * K;
-    for (int64_t m0 = static_cast<int64_t>(blockIdx.y) * kF32BM; m0 < M;
-         m0 += static_cast<int64_t>(gridDim.y) * kF32BM) {
-        const bool a_ok = m0 + sr < M;
-        const float* a_src = x + (a_ok ? m0 + sr : 0) * static_cast<int64_t>(K);
-        float acc[4][4];
+// ---- any alignment ---------------------------------------------------------
+// The same chains on the vector ALU with 4-byte accesses, for arrays that the
+// ring's 16-byte copies cannot take (and, k_linear_any, for Linear shapes it
+// does not): 64 x 64 blocks, 4 x 4 outputs per thread and operand, 16 k of
+// each operand k-major in LDS.
+constexpr int kAnyPitch = kF32BM + 4;   // a wave's transposing stores hit 64 banks
+static_assert(kF32BM == 64 && kF32BN == 64, "one row of A and of each B per four threads");
+
+template <int NB>
+struct AnyStage {
+    float a[kBK][kAnyPitch], b[NB][kBK][kAnyPitch];
+};
+
+// acc[n][r][c] += the chain of row 4 (tid / 16) + r of A against row 4 (tid %
+// 16) + c of B n.  a, b: this thread's staging row (tid / 4) of each, null past
+// the end: read as zero, as is k past K.  A padded step adds the exact product
+// 0 * 0 to an accumulator that is never -0 (it starts at +0, and a sum that
+// cancels exactly rounds to +0), so it changes no bit.
+template <int NB>
+__device__ inline void any_chains(AnyStage<NB>& st, const float* a, const float* const (&b)[NB], int K,
+                                  float (&acc)[NB][4][4]) {
+    const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4, sr = tid >> 2, sk = (tid & 3) * 4;
+    for (int k0 = 0; k0 < K; k0 += kBK) {
+        float av[4], bv[NB][4];
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
+        for (int i = 0; i < 4; ++i) {
+            const int k = k0 + sk + i;
+            av[i] = a && k < K ? a[k] : 0.0f;
 #pragma unroll
-            for (int c = 0; c < 4; ++c) acc[r][c] = 0.0f;
-        for (int k0 = 0; k0 < K; k0 += kBK) {
-            float av[4], bv[4];
+            for (int n = 0; n < NB; ++n) bv[n][i] = b[n] && k < K ? b[n][k] : 0.0f;
+        }
+        __syncthreads();
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int k = k0 + sk + i;
-                av[i] = a_ok && k < K ? a_src[k] : 0.0f;
-                bv[i] = b_ok && k < K ? b_src[k] : 0.0f;
-            }
-            __syncthreads();
+        for (int i = 0; i < 4; ++i) {
+            st.a[sk + i][sr] = av[i];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                As[sk + i][sr] = av[i];
-                Bs[sk + i][sr] = bv[i];
-            }
-            __syncthreads();
+            for (int n = 0; n < NB; ++n) st.b[n][sk + i][sr] = bv[n][i];
+        }
+        __syncthreads();
 #pragma unroll
-            for (int kk = 0; kk < kBK; ++kk) {
-                float ar[4], br[4];
+        for (int kk = 0; kk < kBK; ++kk) {
+            const cf4_t ar = *reinterpret_cast<const cf4_t*>(&st.a[kk][ty * 4]);
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    ar[i] = As[kk][ty * 4 + i];
-                    br[i] = Bs[kk][tx * 4 + i];
-                }
+            for (int n = 0; n < NB; ++n) {
+                const cf4_t br = *reinterpret_cast<const cf4_t*>(&st.b[n][kk][tx * 4]);
 #pragma unroll
                 for (int r = 0; r < 4; ++r)
 #pragma unroll
-                    for (int c = 0; c < 4; ++c) acc[r][c] = __builtin_fmaf(ar[r], br[c], acc[r][c]);
+                    for (int c = 0; c < 4; ++c) acc[n][r][c] = __builtin_fmaf(ar[r], br[c], acc[n][r][c]);
             }
         }
+    }
+}
+
+// UP: act as k_ffn_up_f32 (w = w1, w' = w3, rows by assignment_rows); else y as
+// k_ffn_down_f32 (w = w2, rows by position).  [N][K]: an expert's weight matrix.
+template <bool UP>
+__global__ void __launch_bounds__(256)
+k_ffn_any(const float* __restrict__ in, const uint32_t* __restrict__ offsets,
+          const uint32_t* __restrict__ assignment_rows, const float* __restrict__ w, const float* __restrict__ w3,
+          float* __restrict__ out, int K, int N, int E) {
+    constexpr int NB = UP ? 2 : 1;
+    __shared__ __align__(16) AnyStage<NB> st;
+    GroupTile g;
+    if (!locate_group_tile(offsets, E, kF32BM, N / kF32BN, g)) return;
+    const int tid = threadIdx.x, sr = tid >> 2, n0 = g.col * kF32BN;
+    const uint32_t p = g.m0 + sr;
+    const float* a = nullptr;
+    if (p < g.end) a = in + static_cast<int64_t>(UP ? assignment_rows[p] : p) * K;
+    const int64_t brow = (static_cast<int64_t>(g.expert) * N + n0 + sr) * K;
+    const float* b[NB];
+    b[0] = w + brow;
+    if constexpr (UP) b[1] = w3 + brow;
+    float acc[NB][4][4] = {};
+    any_chains<NB>(st, a, b, K, acc);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const uint32_t pr = g.m0 + (tid >> 4) * 4 + r;
+        if (pr >= g.end) continue;
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+            out[static_cast<int64_t>(pr) * N + n0 + (tid & 15) * 4 + c] =
+                UP ? swiglu_exact(acc[0][r][c], acc[NB - 1][r][c]) : acc[0][r][c];
+    }
+}
+
+// y[m][n] = (fp32 FMA chain over k ascending of x[m][k] w[n][k]) + bias[n] for
+// any K, N and alignment (the reference's fallback for shapes its fast kernels
+// do not take, k_matmul_transposed_tiled, src/tensor.cu:433-461).  Row tiles
+// are walked grid-stride over gridDim.y.
+__global__ void __launch_bounds__(256)
+k_linear_any(const float* __restrict__ x, const float* __restrict__ w, const float* __restrict__ bias,
+             float* __restrict__ y, int64_t M, int K, int N) {
+    __shared__ __align__(16) AnyStage<1> st;
+    const int n0 = blockIdx.x * kF32BN;
+    const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4, sr = tid >> 2;
+    const float* const b[1] = {n0 + sr < N ? w + static_cast<int64_t>(n0 + sr) * K : nullptr};
+    for (int64_t m0 = static_cast<int64_t>(blockIdx.y) * kF32BM; m0 < M;
+         m0 += static_cast<int64_t>(gridDim.y) * kF32BM) {
+        float acc[1][4][4] = {};
+        any_chains<1>(st, m0 + sr < M ? x + (m0 + sr) * K : nullptr, b, K, acc);
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const int64_t row = m0 + ty * 4 + r;
@@ -218,10 +263,16 @@ k_linear_any(const float* __restrict__ x, const float* __restrict__ w, const flo
             for (int c = 0; c < 4; ++c) {
                 const int col = n0 + tx * 4 + c;
                 if (col >= N) continue;
-                y[row * N + col] = bias ? __fadd_rn(acc[r][c], bias[col]) : acc[r][c];
+                y[row * N + col] = bias ? __fadd_rn(acc[0][r][c], bias[col]) : acc[0][r][c];
             }
         }
     }
+}
+
+// The ring copies rows of `a` 16 bytes at a time and the epilogue stores 16
+// bytes of `b`; the library's own weight arrays are always aligned.
+bool aligned16(const float* a, const float* b) {
+    return ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b)) & 15u) == 0;
 }
 
 }  // namespace
@@ -251,6 +302,12 @@ hipError_t launch_ffn_up_f32(const float* x, const uint32_t* offsets,
                              int experts, hipStream_t s) {
     if (rows <= 0) return hipSuccess;
     if (hidden % kBK != 0 || ffn % 64 != 0) return hipErrorInvalidValue;
+    if (!aligned16(x, act)) {
+        const int64_t t = max_row_tiles(2 * rows, kF32BM, experts) * ceil_div(ffn / kF32BN, kFXcds) * kFXcds;
+        hipLaunchKernelGGL(k_ffn_any<true>, dim3(static_cast<unsigned>(t)), dim3(256), 0, s, x, offsets,
+                           assignment_rows, w1, w3, act, hidden, ffn, experts);
+        return hipGetLastError();
+    }
     const int64_t mean = ceil_div(2 * rows, experts);
     // us at hidden 4096, ffn 448, 16 experts, for 1 / 43 / 512 / 1,024 / 2,048
     // tokens; the SIMT kernel before these took 468 to 476 us up to 512
@@ -271,6 +328,12 @@ hipError_t launch_ffn_down_f32(const float* act, const uint32_t* offsets, const 
                                hipStream_t s) {
     if (rows <= 0) return hipSuccess;
     if (ffn % kBK != 0 || hidden % 64 != 0) return hipErrorInvalidValue;
+    if (!aligned16(act, y)) {
+        const int64_t t = max_row_tiles(2 * rows, kF32BM, experts) * ceil_div(hidden / kF32BN, kFXcds) * kFXcds;
+        hipLaunchKernelGGL(k_ffn_any<false>, dim3(static_cast<unsigned>(t)), dim3(256), 0, s, act, offsets, nullptr,
+                           w2, nullptr, y, ffn, hidden, experts);
+        return hipGetLastError();
+    }
     const int64_t mean = ceil_div(2 * rows, experts);
     // as above; the SIMT kernel took 63 us for 43 tokens, 89 for 512
     //   16 rows x 64 columns    8  25  60 107 199

@@ -181,7 +181,9 @@ APS_API int aps_moe_dispatch(const uint8_t* routes, int64_t rows, int32_t num_ex
  * act: [2*rows][ffn] scratch of the compute dtype (f32 or bf16; for the
  * fp8 path e4m3 plus act_scale f32 [2*rows]).  y_perm: [2*rows][hidden],
  * f32 for the F32 path, bf16 otherwise.  x_dtype must match the weight
- * set: F32 for the F32 path, BF16 otherwise. */
+ * set: F32 for the F32 path, BF16 otherwise.  The F32 path takes x, act and
+ * y_perm at any 4-byte alignment (16-byte aligned arrays run on the matrix
+ * cores; the bits are the same). */
 APS_API int aps_moe_expert_ffn(uint64_t handle, const void* x, int32_t x_dtype, int64_t rows,
                        const uint32_t* offsets, const uint32_t* assignment_rows,
                        void* act, float* act_scale, void* y_perm, void* stream);

@@ -61,3 +61,63 @@ def test_fp32_experts_block_edges(gpu_device, T, E, H, F):
     for a, b in ((y, ref["y"]), (got, ref["out"])):
         err = np.linalg.norm(a.astype(np.float64) - b, axis=1) / np.linalg.norm(b.astype(np.float64), axis=1)
         assert err.max() <= 2.0 ** -23
+
+
+def off4(a):
+    """The same values 4 bytes past a 16-byte boundary."""
+    b = torch.empty(a.numel() + 1, dtype=a.dtype, device=a.device)
+    b[1:] = a.reshape(-1)
+    out = b[1:].view(a.shape)
+    assert out.data_ptr() % 16 == 4
+    return out
+
+
+# tokens: the few-token router's and the token-major router's, one to several
+# 64-row blocks per expert; an expert without rows among the staged offsets
+@pytest.mark.parametrize("T,E,H,F", [(1, 2, 512, 64), (40, 3, 512, 192), (300, 16, 256, 64), (257, 2, 768, 320)])
+def test_fp32_experts_unaligned(gpu_device, T, E, H, F):
+    """fp32 arrays that are only 4-byte aligned: the block, the staged GEMMs
+    (x, act and y alone and together) and the dense FFN give the bits that
+    the aligned arrays give."""
+    from aps2026_amd import capi
+    note(f"fp32 experts unaligned T={T} E={E} H={H} F={F}")
+    inp = synth.make_moe_inputs(T=T, H=H, E=E, F=F, dtype="f32", seed=T + H)
+    x, gate = dev(inp.x, gpu_device), dev(inp.gate, gpu_device)
+    d = lambda a: [dev(a[e], gpu_device) for e in range(E)]
+    bits = lambda a: a.view(torch.int32)
+    w = moe.register_moe_weights_gpu(d(inp.w1), d(inp.w2), d(inp.w3), torch.float32)
+    want = moe.moe_forward_gpu(x, gate, w)
+    assert torch.equal(bits(moe.moe_forward_gpu(off4(x), gate, w)), bits(want))
+    logits = w.plan_views(T)["logits"].clone()
+    assert torch.equal(bits(moe.moe_forward_grouped_gpu(off4(x), logits, w)), bits(want))
+    L, s = capi.lib(), moe._stream(gpu_device)
+    rng = np.random.default_rng(T)
+    cuts = np.sort(rng.integers(0, 2 * T + 1, E - 1))
+    cuts[0] = 0   # expert 0 has no row
+    offsets = dev(np.concatenate([[0], cuts, [2 * T]]).astype(np.int32), gpu_device)
+    arows = dev(rng.integers(0, T, 2 * T).astype(np.int32), gpu_device)
+
+    def staged(xs, act, y):
+        act.fill_(float("nan"))
+        y.fill_(float("nan"))
+        assert L.aps_moe_ffn_up(w.handle, xs.data_ptr(), capi.DTYPE_F32, T, offsets.data_ptr(), arows.data_ptr(),
+                                act.data_ptr(), None, s) == 0, capi.last_error()
+        assert L.aps_moe_ffn_down(w.handle, act.data_ptr(), None, T, offsets.data_ptr(), y.data_ptr(), s) == 0
+        return act.clone(), y.clone()
+
+    act, y = torch.empty(2 * T, F, device=gpu_device), torch.empty(2 * T, H, device=gpu_device)
+    ref = staged(x, act, y)
+    assert all(torch.isfinite(t).all() for t in ref)
+    for xs, a, o in ((off4(x), act, y), (x, off4(act), y), (x, act, off4(y)), (off4(x), off4(act), off4(y))):
+        for got, r in zip(staged(xs, a, o), ref):
+            assert torch.equal(bits(got), bits(r))
+    w.release()
+    one = moe.register_moe_weights_gpu(d(inp.w1)[:1], d(inp.w2)[:1], d(inp.w3)[:1], torch.float32)
+    n = L.aps_mlp_workspace_size(one.handle, T)
+    ws = torch.empty(n, dtype=torch.uint8, device=gpu_device)
+    out = []
+    for xs, o in ((x, torch.empty_like(x)), (off4(x), torch.empty_like(x)), (x, off4(torch.empty_like(x)))):
+        assert L.aps_mlp_forward(one.handle, xs.data_ptr(), capi.DTYPE_F32, T, o.data_ptr(), ws.data_ptr(), n, s) == 0
+        out.append(o.clone())
+    one.release()
+    assert torch.equal(bits(out[1]), bits(out[0])) and torch.equal(bits(out[2]), bits(out[0]))
