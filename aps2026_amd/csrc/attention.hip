@@ -119,7 +119,10 @@ typedef float ag4_t __attribute__((ext_vector_type(4)));
 // Every score is computed once: the run's 16 x window scores sit in LDS.
 // Keys after a row's window take p = 0, which leaves its value chains
 // unchanged except that a -0 would turn +0; keys before it keep the chain
-// at its +0 start; the last tile's padding has p = 0 and v = 0.
+// at its +0 start; the last tile's padding has p = 0 and v = 0.  Infinite and
+// NaN values of a key outside a row's window would turn its output NaN
+// (0 * inf): a run with a NaN output is done again row by row, each row on
+// its own keys alone (the check rides on the run's last barrier).
 //   K and V go from global memory straight to registers (LDS holds only the
 // scores and the chain's key rows, so two workgroups fit a CU at 1,024-key
 // windows, and three at key spans up to 784).  Scores: wave w takes the
@@ -148,6 +151,7 @@ k_attention_group(const float* __restrict__ q, const float* __restrict__ k, cons
     uint32_t* chain = reinterpret_cast<uint32_t*>(sc + kGroupQueries * sw);   // [sw - 1] key rows
     __shared__ int qlo[kGroupQueries], qhi[kGroupQueries];   // window of each query, relative to dlo
     __shared__ float wmx[4][kGroupQueries];                  // per-wave maxima
+    __shared__ int redo;                                     // the run has a NaN output
 
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     // groups in reverse row order: later rows (longer chains in trie and
@@ -160,7 +164,8 @@ k_attention_group(const float* __restrict__ q, const float* __restrict__ k, cons
         const int64_t p = row_pos[r];
         return p < anc_stride ? p : anc_stride - 1;
     };
-    for (int i0 = 0, nr; i0 < gn; i0 += nr) {
+    int most = kGroupRows;   // rows per run at most
+    for (int i0 = 0, nr; i0 < gn;) {
     const int64_t r0 = g0 + i0;
     // (opaque per run: addresses hoisted out of the loop cost spills)
     int tid = threadIdx.x;
@@ -168,7 +173,7 @@ k_attention_group(const float* __restrict__ q, const float* __restrict__ k, cons
     const int lane = tid & 63;
     // the longest run from row i0 whose key range, from its first row's
     // window on, fits the LDS (sw - 1 keys: a single row always does)
-    for (nr = gn - i0; nr > 1; --nr) {
+    for (nr = gn - i0 < most ? gn - i0 : most; nr > 1; --nr) {
         const int l = i0 + nr - 1;
         const uint32_t need = ((1u << nr) - 1u) >> 1 << i0;   // rows i0 .. l - 1
         const int64_t p0 = pos_of(r0);
@@ -281,6 +286,7 @@ k_attention_group(const float* __restrict__ q, const float* __restrict__ k, cons
 
     // ---- softmax, per query on the 16 threads of one wave (queries
     // 4 w .. 4 w + 3 on wave w), so it needs no workgroup barrier ----
+    if (tid == 0) redo = 0;   // between barriers: every wave has read the last run's
     const int qi = tid / 16, part = tid % 16;
     const char* const vbase = reinterpret_cast<const char*>(v + kh * kHeadDim);   // uniform: 32-bit lane offsets
     const uint32_t dbytes = static_cast<uint32_t>(32 * wave + 2 * qq) * sizeof(float);   // this lane's two dimensions
@@ -377,15 +383,21 @@ k_attention_group(const float* __restrict__ q, const float* __restrict__ k, cons
             group(g + 3, vb3, 1);
         }
     }
+    bool nan = false;
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
         const int qx = 4 * qj + t;   // query: row qx / 4, head qx % 4
         const int r = qx / kGroup;
-        if (r < nr)
+        if (r < nr) {
+            nan = nan || o[0][t] != o[0][t] || o[1][t] != o[1][t];
             *reinterpret_cast<af2*>(out + ((r0 + r) * q_heads + kh * kGroup + qx % kGroup) * kHeadDim + 32 * wave +
                                     2 * qq) = af2{o[0][t], o[1][t]};
+        }
     }
-    __syncthreads();   // the next run writes the chain and the scores
+    if (nan) redo = 1;
+    __syncthreads();   // also: the next run writes the chain and the scores
+    if (nr > 1 && redo) most = 1;   // again, row by row
+    else i0 += nr;
     }
 }
 

@@ -427,11 +427,8 @@ APS_API int aps_rope_tree(float* q, float* k, const uint32_t* row_pos, int64_t r
  * [rows][kv_heads][128], out [rows][q_heads][128], fp32; q_heads = 4 kv_heads
  * ("attention_tree_gpu expects GQA-4"); head_dim 128; k 16-byte aligned.
  * Ancestor entries must be < rows and positions < anc_stride (the kernel
- * clamps them, for memory safety only).  v must be finite: four rows on one
- * ancestor chain are computed together over the union of their windows,
- * and a key outside one row's window enters that row's value products with
- * weight 0, which leaves the result unchanged for a finite value (0 * inf
- * would not); the reference model's activations are finite. */
+ * clamps them, for memory safety only).  A row reads the values of its own
+ * window alone: infinite or NaN values elsewhere do not reach it. */
 APS_API int aps_attention_tree(const float* q, const float* k, const float* v, float* out, const uint32_t* row_pos,
                                const uint32_t* anc, int64_t anc_stride, int64_t rows, int32_t q_heads,
                                int32_t kv_heads, int32_t head_dim, int32_t window, void* stream);
@@ -439,8 +436,7 @@ APS_API int aps_attention_tree(const float* q, const float* k, const float* v, f
 /* Replaces tensor_ops::attention_gpu (reference include/tensor.h:
  * 95-98, src/tensor.cu:3318-3340, kernel k_attention_grouped_gqa4
  * :2267-2405): the same attention and arithmetic as aps_attention_tree, over
- * packed token sequences instead of trie nodes (and with its precondition
- * on v: finite values) -- row r of a segment that
+ * packed token sequences instead of trie nodes -- row r of a segment that
  * starts at row seg_offset[r] sits at position seg_pos[r] in it, and its
  * keys are rows seg_offset[r] + begin .. seg_offset[r] + seg_pos[r] (begin =
  * max(0, pos + 1 - window)).  max_seq bounds every segment length (the
@@ -448,8 +444,8 @@ APS_API int aps_attention_tree(const float* q, const float* k, const float* v, f
  * kernel (head_dim 128, k 16-byte aligned); any other layout with q_heads a
  * multiple of kv_heads and head_dim <= 128 the reference's generic kernel's
  * arithmetic (k_attention, :2209-2274: each score one fma chain over d, the
- * same softmax and value chains; any v, no finiteness precondition).  RoPE
- * of packed rows is aps_rope_tree with row_pos = seg_pos. */
+ * same softmax and value chains).  RoPE of packed rows is aps_rope_tree with
+ * row_pos = seg_pos. */
 APS_API int aps_attention_packed(const float* q, const float* k, const float* v, float* out,
                                  const uint32_t* seg_offset, const uint32_t* seg_pos, int64_t max_seq, int64_t rows,
                                  int32_t q_heads, int32_t kv_heads, int32_t head_dim, int32_t window, void* stream);

@@ -211,8 +211,7 @@ def test_attention_packed_other_head_layouts_bit_exact(gpu_device, q_heads, kv_h
 
 @pytest.mark.parametrize("window", [2047, 5])
 def test_attention_excluded_keys_take_no_part(gpu_device, window):
-    """Precondition of the path-group kernel: value rows are finite.  A key
-    inside a four-row group's span but outside one row's window (a later row
+    """A key inside a four-row group's span but outside one row's window (a later row
     of the group, causally, or a key past the sliding window) enters that
     row's value MFMAs with p = 0, which leaves its chains unchanged for every
     finite value; the reference's row kernel never reads such keys.  Value
@@ -298,6 +297,50 @@ def test_rope_overlapping_and_unaligned(gpu_device, hd):
     rope(twice, twice)
     rope(q0, torch.empty_like(k0))                        # q0 has been rotated once above
     assert torch.equal(q0.view(torch.int32), twice.view(torch.int32))
+
+
+@pytest.mark.parametrize("window", [2047, 5])
+@pytest.mark.parametrize("packed", [False, True])
+def test_attention_non_finite_values_outside_the_window(gpu_device, packed, window):
+    """An infinite or NaN value row reaches the rows that have it in their
+    window and no other: not an earlier row of its group (causally), not a
+    later one that slid past it, not one on another branch."""
+    from aps2026_amd import capi
+    from aps2026_amd.moe import _ptr, _stream
+    note(f"attention: non-finite values outside the window packed={packed} window={window}")
+    if packed:
+        lens = [41, 1, 1, 2, 7, 30]
+        rows, stride = sum(lens), max(lens)
+        off = np.repeat(np.cumsum([0] + lens[:-1]), lens).astype(np.uint32)
+        pos = np.concatenate([np.arange(n) for n in lens]).astype(np.uint32)
+        anc = np.zeros((rows, stride), np.uint32)
+        for r in range(rows):
+            anc[r, :pos[r] + 1] = off[r] + np.arange(pos[r] + 1)
+    else:
+        pre = list(range(21))
+        plan = prefix.prefix_dedup([pre + [100 + i] for i in range(9)] + [pre[:9] + [200, i] for i in range(5)])
+        rows, stride, pos, anc = plan.nodes, plan.max_len, plan.node_depth, plan.node_anc
+    rng = np.random.default_rng(window)
+    q = rng.standard_normal((rows, 16 * 128)).astype(np.float32)
+    k = rng.standard_normal((rows, 4 * 128)).astype(np.float32)
+    qd, kd = dev(q, gpu_device), dev(k, gpu_device)
+    pd = dev(np.asarray(pos).view(np.int32), gpu_device)
+    td = dev((off if packed else np.asarray(anc, np.uint32)).view(np.int32), gpu_device)
+    for bad in (3, 18, 20, rows - 12, rows - 5, rows - 2):
+        v = rng.standard_normal((rows, 4 * 128)).astype(np.float32)
+        v[bad, ::3], v[bad, 1::3] = np.inf, np.nan
+        vd = dev(v, gpu_device)
+        out = torch.empty((rows, 16 * 128), dtype=torch.float32, device=gpu_device)
+        f = capi.lib().aps_attention_packed if packed else capi.lib().aps_attention_tree
+        tabs = (_ptr(td), _ptr(pd)) if packed else (_ptr(pd), _ptr(td))
+        rc = f(_ptr(qd), _ptr(kd), _ptr(vd), _ptr(out), *tabs, stride, rows, 16, 4, 128, window, _stream(qd.device))
+        assert rc == 0, capi.last_error()
+        torch.cuda.synchronize()
+        want = oracle.attention_tree(q, k, v, pos, anc, stride, 16, 4, 128, window)
+        got = out.cpu().numpy()
+        np.testing.assert_array_equal(np.isnan(got), np.isnan(want))
+        ok = ~np.isnan(want)
+        np.testing.assert_array_equal(got.view(np.uint32)[ok], want.view(np.uint32)[ok])
 
 
 def test_attention_nodes_equal_token_rows(gpu_device):
