@@ -86,23 +86,202 @@ constexpr int kGroupRows = 4;
 constexpr int kGroupQueries = kGroupRows * kGroup;   // 16: query q = 4 row + head
 constexpr int kKeyTile = 16;                         // keys per score tile / value group
 
-// Bit 4 l + r: row r0 + r (r < l < nr) lies on the chain of row r0 + l.
+// Bit 4 l + r: row r0 + r (r < l < nr) lies on the chain of row r0 + l.  pos:
+// in lanes 4 l .. 4 l + 3 the position of row r0 + l.
 template <bool PACKED>
 __device__ inline uint32_t chain_pairs(const uint32_t* __restrict__ row_pos, const uint32_t* __restrict__ anc,
-                                       int64_t anc_stride, int64_t r0, int nr, int lane) {
+                                       int64_t anc_stride, int64_t r0, int nr, int lane, uint32_t& pos) {
     const int r = lane & 3, l = (lane >> 2) & 3;
     bool ok = false;
-    if (lane < 16 && r < l && l < nr) {
+    pos = 0;
+    if (lane < 16 && l < nr) {
         const int64_t row = r0 + r, last = r0 + l;
-        int64_t pr = row_pos[row], pl = row_pos[last];
+        int64_t pr = r < l ? row_pos[row] : 0, pl = row_pos[last];
         pr = pr < anc_stride ? pr : anc_stride - 1;
         pl = pl < anc_stride ? pl : anc_stride - 1;
-        ok = pr <= pl && (PACKED ? anc[row] == anc[last] : anc[last * anc_stride + pr] == static_cast<uint32_t>(row));
+        pos = static_cast<uint32_t>(pl);
+        ok = r < l && pr <= pl && (PACKED ? anc[row] == anc[last] : anc[last * anc_stride + pr] == static_cast<uint32_t>(row));
     }
     return static_cast<uint32_t>(__ballot(ok));
 }
 
 typedef float ag4_t __attribute__((ext_vector_type(4)));
+
+// Scores s[0 .. n) of one query -> probabilities: p = e / den in the window
+// [l0, h0], 0 elsewhere; by the query's 16 threads (part: thread % 16), which
+// are in one wave.
+__device__ inline void window_softmax(float* srow, int l0, int h0, int n, float mq, int part) {
+    // e = (float)exp((double)(s - m)) over the window, in place
+    int w = l0 + part;
+    for (; w + 48 <= h0; w += 64) {
+        float x[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) x[u] = srow[w + 16 * u];
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            srow[w + 16 * u] = static_cast<float>(exp(static_cast<double>(__fsub_rn(x[u], mq))));
+    }
+    for (; w <= h0; w += 16) srow[w] = static_cast<float>(exp(static_cast<double>(__fsub_rn(srow[w], mq))));
+    // the denominator in key order on the query's first lane (the
+    // wave's LDS accesses complete in program order), 16 reads ahead;
+    // the wave barrier keeps the compiler from moving the other lanes'
+    // stores past that lane's reads (they communicate through LDS)
+    __builtin_amdgcn_wave_barrier();
+    float den = 0.0f;
+    if (part == 0) {
+        int x = l0;
+        for (; x + 16 <= h0 + 1; x += 16) {
+            float e[16];
+#pragma unroll
+            for (int u = 0; u < 16; ++u) e[u] = srow[x + u];
+#pragma unroll
+            for (int u = 0; u < 16; ++u) den = __fadd_rn(den, e[u]);
+        }
+        for (; x <= h0; ++x) den = __fadd_rn(den, srow[x]);
+    }
+    den = __shfl(den, static_cast<int>(threadIdx.x & 63) & ~15);
+    // p = e / den in the window, 0 elsewhere over the tiles
+    int x = part;
+    for (; x + 48 < n; x += 64) {
+        float e[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) e[u] = srow[x + 16 * u];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int xu = x + 16 * u;
+            srow[xu] = (xu >= l0 && xu <= h0) ? __fdiv_rn(e[u], den) : 0.0f;
+        }
+    }
+    for (; x < n; x += 16) srow[x] = (x >= l0 && x <= h0) ? __fdiv_rn(srow[x], den) : 0.0f;
+}
+
+// One row and KV head by one wave: the same arithmetic on the same MFMAs with
+// the four heads' rows of the query operand repeated, so that lane l ends with
+// head l / 16.  Keys in blocks of 64, a lane per key's row offset, read a block
+// ahead and passed on by shuffles; K goes two tiles ahead into the registers a
+// tile has used up, V two groups of 16 keys.  sc: this wave's 4 score rows.
+// LDS is the wave's own: no workgroup barrier.
+template <bool PACKED>
+__device__ inline void attend_row(const float* __restrict__ q, const float* __restrict__ k,
+                                  const float* __restrict__ v, float* __restrict__ out,
+                                  const uint32_t* __restrict__ anc, int64_t anc_stride, int64_t rows, int q_heads,
+                                  int kv_heads, int wmax, float scale, float* sc, int sw, int kh, int64_t row,
+                                  int64_t pos) {
+    const int lane = threadIdx.x & 63, qq = lane & 15, qj = lane >> 4;
+    const int64_t begin = pos + 1 > wmax ? pos + 1 - wmax : 0;
+    const int W = static_cast<int>(pos - begin + 1);
+    const int ntiles = (W + kKeyTile - 1) / kKeyTile;
+    const uint32_t kvs_bytes = static_cast<uint32_t>(kv_heads) * kHeadDim * sizeof(float);
+    const int64_t first = (PACKED ? static_cast<int64_t>(anc[row]) : row * anc_stride) + begin;
+    // byte offset of key w's K / V row (past the window: the last key's)
+    auto key = [&](int w) __attribute__((always_inline)) {
+        w = w < W ? w : W - 1;
+        const int64_t a = PACKED ? first + w : static_cast<int64_t>(anc[first + w]);
+        return static_cast<uint32_t>(a < rows ? a : rows - 1) * kvs_bytes;
+    };
+    auto pick = [&](const ag4_t& x) { return qj == 0 ? x[0] : qj == 1 ? x[1] : qj == 2 ? x[2] : x[3]; };
+    float* const srow = sc + qj * sw;   // this lane's head
+
+    // ---- scores ----
+    const af4* qsrc =
+        reinterpret_cast<const af4*>(q + (row * q_heads + kh * kGroup + qq % kGroup) * kHeadDim + 4 * qj);
+    af4 qv[8];
+#pragma unroll
+    for (int a = 0; a < 8; ++a) qv[a] = qsrc[4 * a];
+    float m = -3.402823466e+38f;
+    {
+        const char* const kbase = reinterpret_cast<const char*>(k + kh * kHeadDim) + 16 * qj;
+        uint32_t cur = key(lane), next = key(kWave + lane);
+        auto ksrc = [&](uint32_t block, int t) __attribute__((always_inline)) {
+            return reinterpret_cast<const af4*>(kbase + __shfl(block, 16 * t + qq));
+        };
+        af4 kb[2][8];
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            const af4* src = ksrc(cur, t);
+#pragma unroll
+            for (int a = 0; a < 8; ++a) kb[t][a] = src[4 * a];
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        for (int t0 = 0; t0 < ntiles; t0 += 4) {
+            const uint32_t after = key(16 * t0 + 2 * kWave + lane);
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                if (t0 + t >= ntiles) break;   // wave-uniform
+                const af4* src = ksrc(t < 2 ? cur : next, (t + 2) & 3);
+                ag4_t acc[4] = {};
+#pragma unroll
+                for (int a = 0; a < 8; ++a) {
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+                        acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(qv[a][j], kb[t & 1][a][j], acc[j], 0, 0, 0);
+                    __builtin_amdgcn_sched_barrier(0);
+                    kb[t & 1][a] = src[4 * a];
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                const int w = 16 * (t0 + t) + qq;
+                const float s = __fmul_rn(__fadd_rn(__fadd_rn(pick(acc[0]), pick(acc[1])),
+                                                    __fadd_rn(pick(acc[2]), pick(acc[3]))), scale);
+                srow[w] = s;
+                if (w < W) m = fmaxf(m, s);
+            }
+            cur = next;
+            next = after;
+        }
+    }
+#pragma unroll
+    for (int o = 8; o >= 1; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
+    __builtin_amdgcn_wave_barrier();   // (the wave's LDS accesses complete in order)
+
+    // ---- softmax and values, the first 32 keys' loads under the softmax ----
+    const char* const vbase = reinterpret_cast<const char*>(v + kh * kHeadDim) + 32 * qq;   // this lane's 8 dimensions
+    uint32_t cur = key(lane), next = key(kWave + lane);
+    af4 vb[2][4][2];
+    auto vload = [&](af4 (&d)[4][2], uint32_t block, int g) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const af4* src = reinterpret_cast<const af4*>(vbase + __shfl(block, 16 * g + 4 * u + qj));
+            d[u][0] = src[0];
+            d[u][1] = src[1];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    vload(vb[0], cur, 0);
+    vload(vb[1], cur, 1);
+    window_softmax(srow, 0, W - 1, ntiles * kKeyTile, m, qq);
+    __builtin_amdgcn_wave_barrier();
+    const float* const prow = sc + (qq % kGroup) * sw + qj;   // A: query lane % 16, key lane / 16 of a step
+    ag4_t o[8] = {};   // register t of o[i]: head t, dimension 8 (lane % 16) + i
+    for (int g0 = 0; g0 < ntiles; g0 += 4) {
+        const uint32_t after = key(16 * g0 + 2 * kWave + lane);
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            if (g0 + g >= ntiles) break;   // wave-uniform
+            const int w0 = 16 * (g0 + g);
+            af4 (&d)[4][2] = vb[g & 1];
+            float pa[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) pa[u] = prow[w0 + 4 * u];
+            if (w0 + 16 > W) {   // the last tile's padding: no value at all
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+                    if (w0 + 4 * u + qj >= W) d[u][0] = d[u][1] = af4{0.0f, 0.0f, 0.0f, 0.0f};
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+#pragma unroll
+                for (int i = 0; i < 8; ++i)
+                    o[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(pa[u], d[u][i / 4][i % 4], o[i], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            vload(d, g < 2 ? cur : next, (g + 2) & 3);
+        }
+        cur = next;
+        next = after;
+    }
+    float* const dst = out + (row * q_heads + kh * kGroup + qj) * kHeadDim + 8 * qq;   // 8-byte aligned
+#pragma unroll
+    for (int i = 0; i < 8; i += 2) *reinterpret_cast<af2*>(dst + i) = af2{pick(o[i]), pick(o[i + 1])};
+}
 
 // One workgroup = one row group x one KV head.  Per run of rows: 16 queries
 // (up to 4 rows x the KV head's 4 query heads) against the keys chain[dlo ..
@@ -138,9 +317,12 @@ typedef float ag4_t __attribute__((ext_vector_type(4)));
 // (exp, division, addresses).  Measured, 4,096 rows of 512-token prompts: 249
 // us -> 177; 10,240 rows, 16 prompts of 1,024 with shared halves: 1345 -> 1016,
 // against the K = 1 MFMA with its operands transposed across lanes and the
-// values on two of the four waves.  Serving every group here, run by run,
-// instead of leaving branching groups to a second launch over all rows saves
-// that launch: 9.7 and 22 us, and 19 -> 12 us for 43 rows.
+// values on two of the four waves.  Serving every group here instead of
+// leaving branching groups to a second launch over all rows saves that launch:
+// 9.7 and 22 us, and 14 -> 8 us for 43 rows.  Groups that branch much go row by
+// row (attend_row): 4,096 single-token prompts 68 us in two launches, 150 run by
+// run, 56 row by row; 4,096 leaves of a 1,000-token prompt 1650, 1990, 1430, of
+// a 100-token prompt 207, 328, 222.
 template <bool PACKED>
 __global__ void __launch_bounds__(256, 3)
 k_attention_group(const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v,
@@ -159,41 +341,66 @@ k_attention_group(const float* __restrict__ q, const float* __restrict__ k, cons
     const int64_t g0 = static_cast<int64_t>(gridDim.x / kv_heads - 1 - blockIdx.x / kv_heads) * kGroupRows;
     const int kh = static_cast<int>(blockIdx.x % kv_heads);
     const int gn = static_cast<int>(rows - g0 < kGroupRows ? rows - g0 : kGroupRows);
-    const uint32_t pairs = __builtin_amdgcn_readfirstlane(chain_pairs<PACKED>(row_pos, anc, anc_stride, g0, gn, threadIdx.x & 63));
-    auto pos_of = [&](int64_t r) -> int64_t {
-        const int64_t p = row_pos[r];
-        return p < anc_stride ? p : anc_stride - 1;
+    uint32_t group_pos;
+    const uint32_t pairs = __builtin_amdgcn_readfirstlane(
+        chain_pairs<PACKED>(row_pos, anc, anc_stride, g0, gn, threadIdx.x & 63, group_pos));
+    auto pos_of = [&](int i) -> int64_t {   // of the group's row i
+        return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(group_pos), 4 * i));
     };
-    int most = kGroupRows;   // rows per run at most
-    for (int i0 = 0, nr; i0 < gn;) {
+    // the longest run from row i0 whose key range, from its first row's
+    // window on, fits the LDS (sw - 1 keys: a single row always does)
+    auto run_rows = [&](int i0) __attribute__((always_inline)) {
+        const int64_t p0 = pos_of(i0);
+        int nr = gn - i0;
+        for (; nr > 1; --nr) {
+            const int l = i0 + nr - 1;
+            const uint32_t need = ((1u << nr) - 1u) >> 1 << i0;   // rows i0 .. l - 1
+            bool fits = ((pairs >> (4 * l)) & need) == need &&
+                        pos_of(l) - (p0 + 1 > wmax ? p0 + 1 - wmax : 0) + 1 <= sw - 1;
+            for (int r = 1; r + 1 < nr; ++r) fits = fits && pos_of(i0 + r) >= p0;
+            if (fits) break;
+        }
+        return nr;
+    };
+    int runs = 0;
+    uint32_t run_at = 0;   // 4 bits per row: the rows of the run that starts there
+    int64_t longest = 0;
+    for (int i0 = 0; i0 < gn; ++runs) {
+        const int nr = run_rows(i0);
+        run_at |= static_cast<uint32_t>(nr) << (4 * i0);
+        i0 += nr;
+        const int64_t p = pos_of(i0 - 1);
+        longest = p > longest ? p : longest;
+    }
+    // Rows of several runs one per wave: always with four runs, with fewer while
+    // the windows are short and the runs' latencies, one after the other,
+    // weigh more than the repeated query rows.  us by run -> by row at windows of
+    // 33 / 101 / 201 / 501 keys, leaves of a shared prompt: four runs (512 rows)
+    // 33 -> 20, 53 -> 35, 79 -> 57, 152 -> 121; three 33 -> 27, 53 -> 51, 82 -> 83,
+    // 160 -> 180; two 34 -> 34, 54 -> 64, 80 -> 108, 152 -> 241.
+    const int64_t window = longest + 1 < wmax ? longest + 1 : wmax;
+    bool by_row = runs == 4 || (runs == 3 && window <= 160) || (runs == 2 && window <= 32);
+    for (int i0 = 0, nr; !by_row && i0 < gn;) {
     const int64_t r0 = g0 + i0;
     // (opaque per run: addresses hoisted out of the loop cost spills)
     int tid = threadIdx.x;
     asm volatile("" : "+v"(tid));
     const int lane = tid & 63;
-    // the longest run from row i0 whose key range, from its first row's
-    // window on, fits the LDS (sw - 1 keys: a single row always does)
-    for (nr = gn - i0 < most ? gn - i0 : most; nr > 1; --nr) {
-        const int l = i0 + nr - 1;
-        const uint32_t need = ((1u << nr) - 1u) >> 1 << i0;   // rows i0 .. l - 1
-        const int64_t p0 = pos_of(r0);
-        bool fits = ((pairs >> (4 * l)) & need) == need &&
-                    pos_of(g0 + l) - (p0 + 1 > wmax ? p0 + 1 - wmax : 0) + 1 <= sw - 1;
-        for (int r = 1; r + 1 < nr; ++r) fits = fits && pos_of(r0 + r) >= p0;
-        if (fits) break;
-    }
+    nr = (run_at >> (4 * i0)) & 15;
     const int64_t last = r0 + nr - 1;
-    const int64_t plast = pos_of(last);
-    const int64_t p0 = pos_of(r0);
+    const int64_t plast = pos_of(i0 + nr - 1);
+    const int64_t p0 = pos_of(i0);
     const int dlo = static_cast<int>(p0 + 1 > wmax ? p0 + 1 - wmax : 0);
     const int dhi = static_cast<int>(plast);
     const int W = dhi - dlo + 1;
     const int ntiles = (W + kKeyTile - 1) / kKeyTile;   // 16-key tiles (at most capacity / 16)
     const int64_t seg = PACKED ? static_cast<int64_t>(anc[last]) : 0;
+    // (a shuffle reads active lanes only: before the branch)
+    const uint32_t query_pos = static_cast<uint32_t>(__shfl(static_cast<int>(group_pos), 4 * i0 + lane));
     if (tid < kGroupQueries) {
         const int r = tid / kGroup;
         if (r < nr) {
-            const int64_t pr = pos_of(r0 + r);
+            const int64_t pr = query_pos;
             qhi[tid] = static_cast<int>(pr) - dlo;
             qlo[tid] = static_cast<int>(pr + 1 > wmax ? pr + 1 - wmax : 0) - dlo;
         } else {
@@ -303,50 +510,7 @@ k_attention_group(const float* __restrict__ q, const float* __restrict__ k, cons
     vload(gclamp(3), vb3);
     {
         const float mq = fmaxf(fmaxf(wmx[0][qi], wmx[1][qi]), fmaxf(wmx[2][qi], wmx[3][qi]));
-        float* const srow = sc + qi * sw;
-        const int l0 = qlo[qi], h0 = qhi[qi];
-        // e = (float)exp((double)(s - m)) over the window, in place
-        int w = l0 + part;
-        for (; w + 48 <= h0; w += 64) {
-            float x[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) x[u] = srow[w + 16 * u];
-#pragma unroll
-            for (int u = 0; u < 4; ++u)
-                srow[w + 16 * u] = static_cast<float>(exp(static_cast<double>(__fsub_rn(x[u], mq))));
-        }
-        for (; w <= h0; w += 16) srow[w] = static_cast<float>(exp(static_cast<double>(__fsub_rn(srow[w], mq))));
-        // the denominator in key order on the query's first lane (the
-        // wave's LDS accesses complete in program order), 16 reads ahead;
-        // the wave barrier keeps the compiler from moving the other lanes'
-        // stores past that lane's reads (they communicate through LDS)
-        __builtin_amdgcn_wave_barrier();
-        float den = 0.0f;
-        if (part == 0) {
-            int x = l0;
-            for (; x + 16 <= h0 + 1; x += 16) {
-                float e[16];
-#pragma unroll
-                for (int u = 0; u < 16; ++u) e[u] = srow[x + u];
-#pragma unroll
-                for (int u = 0; u < 16; ++u) den = __fadd_rn(den, e[u]);
-            }
-            for (; x <= h0; ++x) den = __fadd_rn(den, srow[x]);
-        }
-        den = __shfl(den, lane & ~15);
-        // p = e / den in the window, 0 elsewhere over the tiles
-        int x = part;
-        for (; x + 48 < ntiles * kKeyTile; x += 64) {
-            float e[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) e[u] = srow[x + 16 * u];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const int xu = x + 16 * u;
-                srow[xu] = (xu >= l0 && xu <= h0) ? __fdiv_rn(e[u], den) : 0.0f;
-            }
-        }
-        for (; x < ntiles * kKeyTile; x += 16) srow[x] = (x >= l0 && x <= h0) ? __fdiv_rn(srow[x], den) : 0.0f;
+        window_softmax(sc + qi * sw, qlo[qi], qhi[qi], ntiles * kKeyTile, mq, part);
     }
     __syncthreads();
 
@@ -396,9 +560,12 @@ k_attention_group(const float* __restrict__ q, const float* __restrict__ k, cons
     }
     if (nan) redo = 1;
     __syncthreads();   // also: the next run writes the chain and the scores
-    if (nr > 1 && redo) most = 1;   // again, row by row
-    else i0 += nr;
+    by_row = nr > 1 && redo;
+    i0 += nr;
     }
+    if (by_row && wave < gn)   // wave-uniform
+        attend_row<PACKED>(q, k, v, out, anc, anc_stride, rows, q_heads, kv_heads, wmax, scale,
+                           sc + wave * kGroup * sw, sw, kh, g0 + wave, pos_of(wave));
 }
 
 // Dynamic LDS: scores [wmax][4] fp32, then chain [wmax] u32.

@@ -299,6 +299,28 @@ def test_rope_overlapping_and_unaligned(gpu_device, hd):
     assert torch.equal(q0.view(torch.int32), twice.view(torch.int32))
 
 
+# shared prompt lengths on both sides of the 16-key tiles, the 64-key blocks and
+# the rule's lines for two and three runs (32 and 160 keys)
+@pytest.mark.parametrize("pre", [0, 13, 15, 16, 29, 31, 62, 64, 126, 128, 157, 160, 191])
+def test_attention_groups_row_by_row_bit_exact(gpu_device, pre):
+    """Groups of four, three and two runs (leaves of a shared prompt with one or
+    two tokens of their own), served row by row by one wave each or run by
+    run; a last group of one to four rows; window 40 slides past the root."""
+    note(f"attention groups row by row pre={pre}")
+    rng = np.random.default_rng(pre)
+    shared = rng.integers(0, 32064, pre).tolist()
+    for leaves, lens in ((9, (1,)), (8, (2,)), (10, (1, 2)), (10, (1, 1, 2)), (6, (3, 1))):
+        batch = [shared + [i] + [7] * (lens[i % len(lens)] - 1) for i in range(leaves)]
+        plan, q, k, v = trie_inputs(batch, q_heads=8, kv_heads=2, seed=pre + leaves)
+        for window in (2047, 40):
+            out = torch.full((plan.nodes, 8 * 128), float("nan"), device=gpu_device)
+            attention.attention_tree_gpu(dev(q, gpu_device), dev(k, gpu_device), dev(v, gpu_device), out,
+                                         plan.node_depth, plan.node_anc, plan.max_len, q_heads=8, kv_heads=2,
+                                         window=window)
+            want = oracle.attention_tree(q, k, v, plan.node_depth, plan.node_anc, plan.max_len, 8, 2, 128, window)
+            np.testing.assert_array_equal(out.cpu().numpy().view(np.uint32), want.view(np.uint32))
+
+
 @pytest.mark.parametrize("window", [2047, 5])
 @pytest.mark.parametrize("packed", [False, True])
 def test_attention_non_finite_values_outside_the_window(gpu_device, packed, window):
