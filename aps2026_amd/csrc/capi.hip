@@ -193,10 +193,11 @@ int check_x_dtype(const WeightSet& w, int32_t x_dtype) {
 }
 
 // Routing (from `logits`; nullptr when the router kernel already wrote the
-// routes and tile histogram into the workspace), dispatch, FFN and combine.
-// The fp8 path with bf16 output folds the combine into the w2 GEMM when the
-// router wrote the slot-0 histogram (aps_moe_forward) and the batch is large:
-// no y round trip.  The slot lists are in the workspace at any size.
+// routes into the workspace, and past few tokens the tile histogram), dispatch,
+// FFN and combine.  The fp8 path with bf16 output folds the combine into the w2
+// GEMM of a large batch routed here (aps_moe_forward): no y round trip.  The
+// slot lists and both histograms, part of the plan that callers may read
+// back, are in the workspace at any size.
 bool fold_combine(const WeightSet& w, int64_t rows, int32_t out_dtype) {
     return w.compute == APS_DTYPE_E4M3 && out_dtype == APS_DTYPE_BF16 && aps::ffn_down_fold_fits(rows, w.H, w.F);
 }
@@ -222,17 +223,17 @@ int grouped_from_logits(const WeightSet& w, const void* x, bool x_is_f32, const 
     auto* slot1 = reinterpret_cast<uint32_t*>(ws + L.slot1);
     auto* srows = reinterpret_cast<uint32_t*>(ws + L.slot_rows);
     auto* stoks = reinterpret_cast<uint32_t*>(ws + L.slot_tokens);
-    if (few) tiles = tiles0 = nullptr;
     // few tokens on the one-wave tiles: the w1||w3 launch makes the plan itself
-    const aps::SmallPlan plan{routes, counts, offsets, arows, rpos, fold ? slot1 : nullptr, srows, stoks};
+    const aps::SmallPlan plan{routes, tiles, counts, offsets, arows, rpos, fold ? slot1 : nullptr, srows, stoks, tiles0};
     const bool planned = few && w.compute != APS_DTYPE_F32 &&
                          aps::ffn_small_fits(w.compute == APS_DTYPE_E4M3, rows, w.F, w.E);
     if (!planned && fold)
-        APS_HIP(aps::launch_dispatch_scatter(routes, tiles, rows, w.E, counts, offsets, arows, rpos, nullptr, s,
-                                             tiles0, slot1, srows, stoks),
+        APS_HIP(aps::launch_dispatch_scatter(routes, few ? nullptr : tiles, rows, w.E, counts, offsets, arows, rpos,
+                                             nullptr, s, few ? nullptr : tiles0, slot1, srows, stoks, tiles, tiles0),
                 "dispatch launch");
     else if (!planned)
-        APS_HIP(aps::launch_dispatch_scatter(routes, tiles, rows, w.E, counts, offsets, arows, rpos, nullptr, s),
+        APS_HIP(aps::launch_dispatch_scatter(routes, few ? nullptr : tiles, rows, w.E, counts, offsets, arows, rpos,
+                                             nullptr, s, nullptr, nullptr, nullptr, nullptr, tiles),
                 "dispatch launch");
     if (w.compute == APS_DTYPE_E4M3) {
         auto* xq = reinterpret_cast<uint8_t*>(ws + L.xq);
@@ -944,9 +945,9 @@ int aps_moe_forward(uint64_t handle, const void* x, int32_t x_dtype, const float
     if (!gate) return fail(APS_ERR_ARG, "forward: NULL gate");
     char* ws = static_cast<char*>(workspace);
     hipStream_t s = static_cast<hipStream_t>(stream);
-    // logits, routes and the tile histogram in one kernel (and, for fp32 x
-    // with a bf16 weight set, the FFN's bf16 copy of x); the grouped path
-    // then starts at the dispatch
+    // logits, routes and, past few tokens, the tile histogram in one kernel
+    // (and, for fp32 x with a bf16 weight set, the FFN's bf16 copy of x); the
+    // grouped path then starts at the dispatch
     float* logits = reinterpret_cast<float*>(ws + L.logits);
     auto* routes = reinterpret_cast<uint8_t*>(ws + L.routes);
     auto* tiles = reinterpret_cast<uint32_t*>(ws + L.tile_counts);

@@ -51,12 +51,12 @@ __device__ inline void route_greedy_top2(const float (&q)[EMAX], int E, int& fir
     second = best;
 }
 
-// Tile histogram word of expert e for the 64-token tile of this wave: byte q
-// counts the routes to e of tokens 16q .. 16q+15 (at most 16 each), so a word
-// sums to the tile's count with (w * 0x01010101) >> 24.  The router writes the
-// bytes one 16-token workgroup at a time.
-__device__ inline uint32_t tile_quarter_counts(int first, int second, int e) {
-    const uint64_t m0 = __ballot(first == e), m1 = __ballot(second == e);
+// Tile histogram word of an expert from the ballots of the tokens of a 64-token
+// tile whose first (second) route it is: byte q counts its routes of tokens
+// 16q .. 16q+15 (at most 16 each), so a word sums to the tile's count with (w *
+// 0x01010101) >> 24.  The router writes the bytes one 16-token workgroup at a
+// time.
+__device__ inline uint32_t tile_word(uint64_t m0, uint64_t m1) {
     uint32_t word = 0;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
@@ -64,6 +64,14 @@ __device__ inline uint32_t tile_quarter_counts(int first, int second, int e) {
         word |= static_cast<uint32_t>(__popcll(m0 & qm) + __popcll(m1 & qm)) << (8 * q);
     }
     return word;
+}
+__device__ inline uint32_t tile_quarter_counts(int first, int second, int e) {
+    return tile_word(__ballot(first == e), __ballot(second == e));
+}
+// lane e <- a wave-uniform mask (e uniform): the words of all experts are then
+// counted at once, a lane per expert
+__device__ inline void mask_to_lane(uint64_t& to, uint64_t m, int e) {
+    if (static_cast<int>(threadIdx.x & 63) == e) to = m;
 }
 __host__ __device__ inline uint32_t tile_word_total(uint32_t w) { return (w * 0x01010101u) >> 24; }
 
@@ -207,8 +215,8 @@ hipError_t launch_router(const void* x, bool x_bf16, const float* gate, int64_t 
                          int experts, float* logits, uint8_t* routes, uint32_t* tile_counts,
                          uint32_t* tile_counts0, bf16_t* x_copy, uint8_t* xq, float* xq_scale, hipStream_t s);
 // The same logits, routes and x copies for few tokens (router_few.hip), but no
-// tile histogram: the dispatch that follows counts the routes itself
-// (launch_dispatch_scatter with tile_counts == nullptr).
+// tile histogram: what makes the plan counts the routes itself and writes it
+// (launch_dispatch_scatter with tile_counts == nullptr, or SmallPlan).
 constexpr int64_t kDispatchFewRows = 256;   // one workgroup of four 64-token tiles
 bool router_few_fits(int64_t rows, int hidden, int experts);
 hipError_t launch_router_few(const void* x, bool x_bf16, const float* gate, int64_t rows, int hidden, int experts,
@@ -293,13 +301,16 @@ hipError_t launch_layer_norm(float* x, const float* residual, const float* weigh
                              int64_t rows, int hidden, float eps, hipStream_t s);
 // With tile_counts0 (the slot-0 histogram) also the slot-ordered lists:
 // slot1[e] = offsets[e] + (slot-0 routes of e); slot_rows / slot_tokens
-// [2 rows] = position / token of list entry i (see dispatch.hip).
+// [2 rows] = position / token of list entry i (see dispatch.hip).  Without
+// tile_counts (rows <= kDispatchFewRows) it counts the routes and writes the
+// histograms to counted and, with slot1, counted0.
 hipError_t launch_dispatch_scatter(const uint8_t* routes, const uint32_t* tile_counts,
                                    int64_t rows, int experts, uint32_t* counts,
                                    uint32_t* offsets, uint32_t* assignment_rows,
                                    uint32_t* route_positions, uint32_t* status, hipStream_t s,
                                    const uint32_t* tile_counts0 = nullptr, uint32_t* slot1 = nullptr,
-                                   uint32_t* slot_rows = nullptr, uint32_t* slot_tokens = nullptr);
+                                   uint32_t* slot_rows = nullptr, uint32_t* slot_tokens = nullptr,
+                                   uint32_t* counted = nullptr, uint32_t* counted0 = nullptr);
 
 // bf16 MFMA path.  w13 / w2 are packed tile images (see launch_pack_*):
 // w13 [E][F/64][H/64][128][64], w2 [E][H/128][F/64][128][64]; act/y bf16.
@@ -333,11 +344,12 @@ bool ffn_down_fold_fits(int64_t rows, int hidden, int ffn);
 bool ffn_small_fits(bool fp8, int64_t rows, int ffn, int experts);        // w1||w3
 bool ffn_down_small_fits(bool fp8, int64_t rows, int ffn, int experts);   // w2
 // plan (null: offsets and assignment_rows are given): the routes to sort and
-// where the plan goes, slot1 .. slot_tokens null unless wanted; rows <=
-// kDispatchFewRows.
+// where the plan and its tile histograms go, slot1 .. tile_counts0 null unless
+// wanted; rows <= kDispatchFewRows.
 struct SmallPlan {
     const uint8_t* routes;
-    uint32_t *counts, *offsets, *assignment_rows, *route_positions, *slot1, *slot_rows, *slot_tokens;
+    uint32_t *tile_counts, *counts, *offsets, *assignment_rows, *route_positions;
+    uint32_t *slot1, *slot_rows, *slot_tokens, *tile_counts0;
 };
 hipError_t launch_ffn_up_small(bool fp8, const uint8_t* x, const float* sx, const uint32_t* offsets,
                                const uint32_t* assignment_rows, const SmallPlan* plan, const uint8_t* w13,

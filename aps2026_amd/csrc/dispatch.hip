@@ -67,7 +67,8 @@ k_dispatch_scatter(const uint8_t* __restrict__ routes, const uint32_t* __restric
                    uint32_t* __restrict__ offsets, uint32_t* __restrict__ assignment_rows,
                    uint32_t* __restrict__ route_positions, uint32_t* __restrict__ status,
                    const uint32_t* __restrict__ tile_counts0, uint32_t* __restrict__ slot1,
-                   uint32_t* __restrict__ slot_rows, uint32_t* __restrict__ slot_tokens) {
+                   uint32_t* __restrict__ slot_rows, uint32_t* __restrict__ slot_tokens,
+                   uint32_t* __restrict__ counted, uint32_t* __restrict__ counted0) {
     const int lane = threadIdx.x & 63;
     const int64_t tile = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
     const int64_t ntiles = (rows + kWave - 1) / kWave;
@@ -97,19 +98,23 @@ k_dispatch_scatter(const uint8_t* __restrict__ routes, const uint32_t* __restric
     // [0]: all routes, [1]: slot-0 routes (SLOTS)
     uint32_t tot[2] = {0, 0}, bef0[2] = {0, 0}, bef1[2] = {0, 0}, bef2[2] = {0, 0}, bef3[2] = {0, 0};
     if constexpr (COUNT) {
-        // one workgroup, no histogram: each wave counts its own tile
+        // one workgroup, no histogram yet: each wave counts its own tile
         int first = 255, second = 255;
         if (t < rows) {
             first = r0;
             second = r1;
             clamp_routes(first, second, E);
         }
+        uint64_t m0 = 0, m1 = 0;
         for (int e = 0; e < E; ++e) {
-            const int n0 = __popcll(__ballot(first == e)), n1 = __popcll(__ballot(second == e));
-            if (lane == e) {
-                tot[0] = static_cast<uint32_t>(n0 + n1);
-                tot[1] = static_cast<uint32_t>(n0);
-            }
+            mask_to_lane(m0, __ballot(first == e), e);
+            mask_to_lane(m1, __ballot(second == e), e);
+        }
+        tot[0] = static_cast<uint32_t>(__popcll(m0) + __popcll(m1));
+        tot[1] = static_cast<uint32_t>(__popcll(m0));
+        if (tile < ntiles && lane < E) {
+            counted[tile * E + lane] = tile_word(m0, m1);
+            if (SLOTS) counted0[tile * E + lane] = tile_word(m0, 0);
         }
 #pragma unroll
         for (int h = 0; h < 2; ++h) {   // bef0: no tile before the first
@@ -280,12 +285,12 @@ hipError_t launch_dispatch_scatter(const uint8_t* routes, const uint32_t* tile_c
                                    uint32_t* offsets, uint32_t* assignment_rows,
                                    uint32_t* route_positions, uint32_t* status, hipStream_t s,
                                    const uint32_t* tile_counts0, uint32_t* slot1, uint32_t* slot_rows,
-                                   uint32_t* slot_tokens) {
+                                   uint32_t* slot_tokens, uint32_t* counted, uint32_t* counted0) {
     if (experts <= 0 || experts > kMaxExperts) return hipErrorInvalidValue;
     const bool slots = slot1 != nullptr;
     if (slots && (!slot_rows || !slot_tokens)) return hipErrorInvalidValue;
     if (slots && (tile_counts != nullptr) != (tile_counts0 != nullptr)) return hipErrorInvalidValue;
-    if (rows > kDispatchFewRows && !tile_counts) return hipErrorInvalidValue;
+    if (!tile_counts && (rows > kDispatchFewRows || !counted || (slots && !counted0))) return hipErrorInvalidValue;
     if (rows <= 0) {
         // empty batch: counts and offsets are all zero
         hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(128), 0, s, counts, experts);
@@ -298,19 +303,19 @@ hipError_t launch_dispatch_scatter(const uint8_t* routes, const uint32_t* tile_c
     if (!tile_counts && slots)
         hipLaunchKernelGGL((k_dispatch_scatter<true, true>), dim3(1), dim3(256), 0, s, routes, nullptr, rows, experts,
                            counts, offsets, assignment_rows, route_positions, status, nullptr, slot1, slot_rows,
-                           slot_tokens);
+                           slot_tokens, counted, counted0);
     else if (!tile_counts)
         hipLaunchKernelGGL((k_dispatch_scatter<false, true>), dim3(1), dim3(256), 0, s, routes, nullptr, rows, experts,
                            counts, offsets, assignment_rows, route_positions, status, nullptr, nullptr, nullptr,
-                           nullptr);
+                           nullptr, counted, nullptr);
     else if (slots)
         hipLaunchKernelGGL(k_dispatch_scatter<true>, grid, dim3(256), 0, s, routes, tile_counts, rows, experts,
                            counts, offsets, assignment_rows, route_positions, status, tile_counts0, slot1,
-                           slot_rows, slot_tokens);
+                           slot_rows, slot_tokens, nullptr, nullptr);
     else
         hipLaunchKernelGGL(k_dispatch_scatter<false>, grid, dim3(256), 0, s, routes, tile_counts, rows, experts,
                            counts, offsets, assignment_rows, route_positions, status, nullptr, nullptr,
-                           nullptr, nullptr);
+                           nullptr, nullptr, nullptr, nullptr);
     return hipGetLastError();
 }
 

@@ -74,8 +74,8 @@ __device__ inline void each_small(uint32_t lo, uint32_t hi, int bn, int blocks, 
 // ---- the routing plan inside the w1||w3 launch ------------------------------
 // After the few-token router the plan (dispatch.hip states it) is a stable sort
 // of at most 512 route bytes: every wave of the w1||w3 launch counts the routes
-// itself and ranks those of its own expert, and one further block writes the
-// plan out for the kernels after it.  That saves the dispatch's launch between
+// itself and ranks those of its own expert, and two further blocks write the
+// plan and its tile histograms out, for the kernels after it and for callers.  That saves the dispatch's launch between
 // the router and the GEMM for 1 us in it: one bf16 token 35.0 -> 33.2 us a block,
 // 37 tokens 52.0 -> 49.9, fp8 65 tokens 45.9 -> 43.6.
 constexpr int kPlanTiles = static_cast<int>(kDispatchFewRows / kWave);
@@ -167,6 +167,23 @@ __device__ inline void plan_write(const Routes& r, int64_t rows, int E, uint32_t
     }
 }
 
+// The plan's tile histograms, by one wave.
+__device__ inline void plan_histograms(const Routes& r, int E, const SmallPlan& p) {
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int k = 0; k < kPlanTiles; ++k) {
+        if (k >= r.nt) continue;   // wave-uniform
+        uint64_t m0 = 0, m1 = 0;
+        for (int e = 0; e < E; ++e) {
+            mask_to_lane(m0, r.slot0(k, e), e);
+            mask_to_lane(m1, r.slot1(k, e), e);
+        }
+        if (lane >= E) continue;
+        p.tile_counts[k * E + lane] = tile_word(m0, m1);
+        if (p.slot1) p.tile_counts0[k * E + lane] = tile_word(m0, 0);
+    }
+}
+
 // Token of row (lane % 32) of tile u, through tok[32] in LDS; rows past the
 // expert's end get its last token.
 __device__ inline uint32_t plan_token(const Routes& r, uint32_t expert_lo, const SmallTile& u, uint32_t* tok) {
@@ -212,7 +229,7 @@ __device__ inline void small_load(SmallStage<Fmt>& d, At at) {
 }
 
 // act[p][n], as ffn_mfma.hip's up_piece.  ROUTES: the plan comes from
-// plan.routes and the last block writes it out; else from offsets and
+// plan.routes and the last two blocks write it out; else from offsets and
 // assignment_rows.
 template <class Fmt, bool ROUTES>
 __global__ void __launch_bounds__(64, 1)
@@ -223,11 +240,15 @@ k_ffn_up_small(const uint8_t* __restrict__ x, uint32_t x_row_bytes, const uint32
     constexpr bool kFp8 = Fmt::kElt == 1;
     __shared__ uint32_t tok[ROUTES ? kSmRows : 1];
     const int lane = threadIdx.x, r = lane & 31, h = lane >> 5;
-    const int blocks = static_cast<int>(gridDim.x) - (ROUTES ? 1 : 0);
+    const int blocks = static_cast<int>(gridDim.x) - (ROUTES ? 2 : 0);
     uint32_t lo, hi;
     Routes routes;
     if constexpr (ROUTES) {
         routes.load(plan.routes, rows);
+        if (static_cast<int>(blockIdx.x) > blocks) {   // block-uniform
+            plan_histograms(routes, E, plan);
+            return;
+        }
         plan_counts(routes, E, lo, hi);
         if (static_cast<int>(blockIdx.x) == blocks) {   // block-uniform
             plan_write(routes, rows, E, lo, hi, plan);
@@ -412,7 +433,7 @@ hipError_t launch_ffn_up_small(bool fp8, const uint8_t* x, const float* sx, cons
     if (plan && (rows > kDispatchFewRows || experts > kWave)) return hipErrorInvalidValue;
     dim3 grid = grid_small(rows, experts, ffn / 16);
     const uint32_t row_bytes = static_cast<uint32_t>(hidden) * (fp8 ? 1u : 2u);
-    if (plan) ++grid.x;
+    if (plan) grid.x += 2;
     auto kern = fp8 ? (plan ? k_ffn_up_small<Fp8Fmt, true> : k_ffn_up_small<Fp8Fmt, false>)
                     : (plan ? k_ffn_up_small<Bf16Fmt, true> : k_ffn_up_small<Bf16Fmt, false>);
     hipLaunchKernelGGL(kern, grid, dim3(64), 0, s, x, row_bytes, offsets, assignment_rows, plan ? *plan : SmallPlan{},

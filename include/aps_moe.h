@@ -106,8 +106,11 @@ typedef struct aps_moe_ws_layout {
     size_t xq_scale;        /* fp8 path: f32 [rows] per-token scale */
     size_t actq;            /* fp8 path: e4m3 act [2*rows][ffn rounded
                                up to 128], zero padded              */
+                            /* from here on: aps_moe_forward with an fp8
+                               set of ffn 448 or 512 and bf16 output
+                               only (the folded combine's lists)        */
     size_t tile_counts0;    /* u32 [ceil(rows/64)][E]: as tile_counts,
-                               slot-0 routes only (aps_moe_forward) */
+                               slot-0 routes only                       */
     size_t slot1;           /* u32 [E]: offsets[e] + slot-0 routes of e */
     size_t slot_rows;       /* u32 [2*rows] slot-ordered list: entries
                                [offsets[e], slot1[e]) the positions of

@@ -142,3 +142,34 @@ def test_few_token_router_equals_the_token_major_router(gpu_device, dtype, x32, 
         bits = torch.int32 if got.dtype == torch.float32 else torch.int16
         assert torch.equal(got.view(bits), big[:n].view(bits)), n
     w.release()
+
+
+@pytest.mark.parametrize("dtype,E,F", [("fp8", 16, 448), ("fp8", 5, 512), ("bf16", 16, 448), ("bf16", 3, 64)])
+def test_tile_histograms_of_few_tokens(gpu_device, dtype, E, F):
+    """The tile histograms of the published plan after a forward, whatever made
+    the plan: the w1||w3 launch, the counting dispatch or the router (257
+    tokens); the slot-0 histogram with an fp8 set."""
+    H = 512
+    print(f"[gpu-case] tile histograms {dtype} E={E} F={F}", flush=True)
+    w = weights(dtype, E, H, F, gpu_device, E + F)
+    g = torch.Generator(device=gpu_device)
+    g.manual_seed(E)
+    x = torch.randn((257, H), generator=g, device=gpu_device).bfloat16()
+    gate = torch.randn((E, H), generator=g, device=gpu_device) * 0.05
+    for n in (1, 16, 17, 63, 64, 65, 130, 256, 257):
+        ws, L = w.workspace(n)
+        ws.fill_(0xEE)
+        moe.moe_forward_gpu(x[:n].contiguous(), gate, w)
+        routes = w.plan_views(n)["routes"].cpu().numpy()
+        tiles = (n + 63) // 64
+        want = np.zeros((2, tiles, E, 4), np.uint8)
+        for t in range(n):
+            for slot in range(2):
+                want[0, t // 64, routes[t, slot], t % 64 // 16] += 1
+            want[1, t // 64, routes[t, 0], t % 64 // 16] += 1
+        size = tiles * E * 4
+        for off, ref in ((L.tile_counts, want[0]), (L.tile_counts0, want[1])):
+            if off == L.tile_counts0 and dtype != "fp8":
+                continue
+            assert np.array_equal(ws[off:off + size].cpu().numpy().reshape(tiles, E, 4), ref), n
+    w.release()
