@@ -293,9 +293,10 @@ hipError_t launch_linear_mfma_f32(const float* x, const float* w, const float* b
 // count (1..3) outputs of one x in one grid, every shape linear_mfma_fits
 hipError_t launch_linear_mfma_multi(const float* x, int64_t rows, int in_f, int count, const float* const* w,
                                     const float* const* bias, float* const* y, const int* out_f, hipStream_t s);
-// the same chains for any in_f, out_f and 4-byte alignment (SIMT, scalar loads)
+// the same chains for any in_f, out_f and 4-byte alignment (SIMT, scalar
+// accesses; vec: 16-byte ones, in_f and out_f multiples of 4)
 hipError_t launch_linear_any_f32(const float* x, const float* w, const float* bias, float* y, int64_t rows, int in_f,
-                                 int out_f, hipStream_t s);
+                                 int out_f, hipStream_t s, bool vec = false);
 
 hipError_t launch_layer_norm(float* x, const float* residual, const float* weight, const float* bias, float* y,
                              int64_t rows, int hidden, float eps, hipStream_t s);

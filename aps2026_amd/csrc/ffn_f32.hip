@@ -171,19 +171,28 @@ struct AnyStage {
 // 16) + c of B n.  a, b: this thread's staging row (tid / 4) of each, null past
 // the end: read as zero, as is k past K.  A padded step adds the exact product
 // 0 * 0 to an accumulator that is never -0 (it starts at +0, and a sum that
-// cancels exactly rounds to +0), so it changes no bit.
-template <int NB>
+// cancels exactly rounds to +0), so it changes no bit.  VEC: 16-byte accesses, K
+// % 4 == 0.
+template <int NB, bool VEC = false>
 __device__ inline void any_chains(AnyStage<NB>& st, const float* a, const float* const (&b)[NB], int K,
                                   float (&acc)[NB][4][4]) {
     const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4, sr = tid >> 2, sk = (tid & 3) * 4;
     for (int k0 = 0; k0 < K; k0 += kBK) {
-        float av[4], bv[NB][4];
+        cf4_t av = {}, bv[NB] = {};
+        if constexpr (VEC) {
+            const int k = k0 + sk;
+            if (a && k < K) av = *reinterpret_cast<const cf4_t*>(a + k);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int k = k0 + sk + i;
-            av[i] = a && k < K ? a[k] : 0.0f;
+            for (int n = 0; n < NB; ++n)
+                if (b[n] && k < K) bv[n] = *reinterpret_cast<const cf4_t*>(b[n] + k);
+        } else {
 #pragma unroll
-            for (int n = 0; n < NB; ++n) bv[n][i] = b[n] && k < K ? b[n][k] : 0.0f;
+            for (int i = 0; i < 4; ++i) {
+                const int k = k0 + sk + i;
+                av[i] = a && k < K ? a[k] : 0.0f;
+#pragma unroll
+                for (int n = 0; n < NB; ++n) bv[n][i] = b[n] && k < K ? b[n][k] : 0.0f;
+            }
         }
         __syncthreads();
 #pragma unroll
@@ -243,7 +252,9 @@ k_ffn_any(const float* __restrict__ in, const uint32_t* __restrict__ offsets,
 // y[m][n] = (fp32 FMA chain over k ascending of x[m][k] w[n][k]) + bias[n] for
 // any K, N and alignment (the reference's fallback for shapes its fast kernels
 // do not take, k_matmul_transposed_tiled, src/tensor.cu:433-461).  Row tiles
-// are walked grid-stride over gridDim.y.
+// are walked grid-stride over gridDim.y.  VEC: 16-byte aligned, K and N multiples
+// of four.
+template <bool VEC>
 __global__ void __launch_bounds__(256)
 k_linear_any(const float* __restrict__ x, const float* __restrict__ w, const float* __restrict__ bias,
              float* __restrict__ y, int64_t M, int K, int N) {
@@ -251,19 +262,31 @@ k_linear_any(const float* __restrict__ x, const float* __restrict__ w, const flo
     const int n0 = blockIdx.x * kF32BN;
     const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4, sr = tid >> 2;
     const float* const b[1] = {n0 + sr < N ? w + static_cast<int64_t>(n0 + sr) * K : nullptr};
+    cf4_t bv = {};
+    if constexpr (VEC)
+        if (bias && n0 + tx * 4 < N) bv = *reinterpret_cast<const cf4_t*>(bias + n0 + tx * 4);
     for (int64_t m0 = static_cast<int64_t>(blockIdx.y) * kF32BM; m0 < M;
          m0 += static_cast<int64_t>(gridDim.y) * kF32BM) {
         float acc[1][4][4] = {};
-        any_chains<1>(st, m0 + sr < M ? x + (m0 + sr) * K : nullptr, b, K, acc);
+        any_chains<1, VEC>(st, m0 + sr < M ? x + (m0 + sr) * K : nullptr, b, K, acc);
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const int64_t row = m0 + ty * 4 + r;
             if (row >= M) continue;
-#pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                const int col = n0 + tx * 4 + c;
+            if constexpr (VEC) {
+                const int col = n0 + tx * 4;   // N % 4 == 0: a column group is all in or all out
                 if (col >= N) continue;
-                y[row * N + col] = bias ? __fadd_rn(acc[0][r][c], bias[col]) : acc[0][r][c];
+                cf4_t o;
+#pragma unroll
+                for (int c = 0; c < 4; ++c) o[c] = bias ? __fadd_rn(acc[0][r][c], bv[c]) : acc[0][r][c];
+                *reinterpret_cast<cf4_t*>(y + row * N + col) = o;
+            } else {
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    const int col = n0 + tx * 4 + c;
+                    if (col >= N) continue;
+                    y[row * N + col] = bias ? __fadd_rn(acc[0][r][c], bias[col]) : acc[0][r][c];
+                }
             }
         }
     }
@@ -278,12 +301,13 @@ bool aligned16(const float* a, const float* b) {
 }  // namespace
 
 hipError_t launch_linear_any_f32(const float* x, const float* w, const float* bias, float* y, int64_t rows, int in_f,
-                                 int out_f, hipStream_t s) {
+                                 int out_f, hipStream_t s, bool vec) {
     if (rows <= 0) return hipSuccess;
-    if (in_f <= 0 || out_f <= 0) return hipErrorInvalidValue;
+    if (in_f <= 0 || out_f <= 0 || (vec && (in_f % 4 != 0 || out_f % 4 != 0))) return hipErrorInvalidValue;
     const int64_t ty = ceil_div(rows, kF32BM);
     const dim3 grid(static_cast<unsigned>(ceil_div(out_f, kF32BN)), static_cast<unsigned>(ty < 65535 ? ty : 65535));
-    hipLaunchKernelGGL(k_linear_any, grid, dim3(256), 0, s, x, w, bias, y, rows, in_f, out_f);
+    hipLaunchKernelGGL(vec ? k_linear_any<true> : k_linear_any<false>, grid, dim3(256), 0, s, x, w, bias, y, rows,
+                       in_f, out_f);
     return hipGetLastError();
 }
 

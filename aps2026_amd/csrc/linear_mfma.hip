@@ -11,7 +11,8 @@
 //  * k_linear_mfma, many rows: 128-row x 128- (or 64-) column blocks, four
 //    waves of 64 x 64 on v_mfma_f32_32x32x2_f32;
 //  * k_linear_small, few rows: 16- to 64-row blocks on v_mfma_f32_16x16x4_f32.
-// The launcher's cost rule takes the one whose busiest CU is done first.
+// The launcher's cost rule takes the one whose busiest CU is done first, or for a
+// short K that is not a multiple of 32 the SIMT blocks of ffn_f32.hip.
 #include "chain_mfma.hpp"
 
 #include <utility>
@@ -364,6 +365,24 @@ hipError_t launch_linear_mfma_multi(const float* x, int64_t rows, int in_f, int 
     // take 14, 29, 57 us, and 114 and 228 for the two block kernels; the
     // rest is what its operand reads and copies add.
     const int64_t cus = num_cus(), rt = ceil_div(rows, kLRows);
+    // A short K that ends in half a stage (in_f % 32 == 16) on many blocks is
+    // bound by y's stores, and the ring's 64 KB of LDS leave two blocks to a CU:
+    // SIMT blocks of 64 x 64 there.  us, ring -> SIMT: 20,000 rows of 16 -> 4096 236
+    // -> 66, of 48 -> 4096 273 -> 132, of 112 -> 11008 935 -> 735; 333 rows of 16 ->
+    // 4096 7.6 -> 4.2; past the line 17 rows of 48 -> 11008 4.5 -> 5.0, 4,096 rows of
+    // 208 -> 1000 27.6 -> 29.0.
+    bool simt = in_f % kLStageK != 0 && in_f <= 176;
+    for (int i = 0; i < count; ++i) {
+        const int64_t blocks = ceil_div(out_f[i], kF32BN) * ceil_div(rows, kF32BM);
+        simt = simt && out_f[i] >= kF32BN && 8 * blocks >= 3 * cus && 70 * blocks >= cus * in_f;
+    }
+    if (simt) {
+        for (int i = 0; i < count; ++i) {
+            const hipError_t e = launch_linear_any_f32(x, w[i], bias[i], y[i], rows, in_f, out_f[i], s, true);
+            if (e != hipSuccess) return e;
+        }
+        return hipSuccess;
+    }
     auto cost = [&](int br, int bc, double us) {
         int64_t t = 0;
         for (int i = 0; i < count; ++i) t += ceil_div(out_f[i], bc);

@@ -63,6 +63,44 @@ def test_fp32_experts_block_edges(gpu_device, T, E, H, F):
         assert err.max() <= 2.0 ** -23
 
 
+# k = 16 mod 32 on both sides of the rule that sends short k to SIMT blocks (k up
+# to 176, 96 blocks and more, out of 64 and more): whole and partly filled blocks
+@pytest.mark.parametrize("rows,k,n", [(6144, 16, 64), (6080, 16, 64), (6100, 16, 60), (700, 48, 1100), (1000, 176, 2600),
+                                      (2800, 80, 516), (1000, 208, 2600)])
+@pytest.mark.parametrize("bias", [True, False])
+def test_linear_short_half_stage(gpu_device, rows, k, n, bias):
+    note(f"linear short k rows={rows} k={k} n={n} bias={bias}")
+    rng = np.random.default_rng(rows + k + n)
+    x = rng.standard_normal((rows, k)).astype(np.float32)
+    w = (0.02 * rng.standard_normal((n, k))).astype(np.float32)
+    b = (0.1 * rng.standard_normal(n)).astype(np.float32) if bias else None
+    out = torch.full((rows, n), float("nan"), device=gpu_device)
+    attention.linear_gpu(dev(x, gpu_device), dev(w, gpu_device), dev(b, gpu_device) if bias else None, out=out)
+    np.testing.assert_array_equal(out.cpu().numpy().view(np.uint32), oracle.linear(x, w, b).view(np.uint32))
+
+
+def test_linear_multi_short_half_stage(gpu_device):
+    """Outputs of different widths in one call, by SIMT blocks, and (a narrow
+    one among them) in one grid."""
+    from aps2026_amd import capi
+    import ctypes
+    rows, k = 2000, 48
+    rng = np.random.default_rng(k)
+    x = rng.standard_normal((rows, k)).astype(np.float32)
+    for ns in ((512, 256, 640), (512, 32)):
+        ws = [(0.02 * rng.standard_normal((n, k))).astype(np.float32) for n in ns]
+        bs = [(0.1 * rng.standard_normal(n)).astype(np.float32) for n in ns]
+        xd, wd, bd = dev(x, gpu_device), [dev(w, gpu_device) for w in ws], [dev(b, gpu_device) for b in bs]
+        ys = [torch.full((rows, n), float("nan"), device=gpu_device) for n in ns]
+        vp = ctypes.c_void_p * len(ns)
+        ptr = lambda ts: vp(*[t.data_ptr() for t in ts])
+        rc = capi.lib().aps_linear_multi(xd.data_ptr(), rows, k, len(ns), ptr(wd), ptr(bd),
+                                         (ctypes.c_int32 * len(ns))(*ns), ptr(ys), moe._stream(gpu_device))
+        assert rc == 0, capi.last_error()
+        for w, b, y in zip(ws, bs, ys):
+            np.testing.assert_array_equal(y.cpu().numpy().view(np.uint32), oracle.linear(x, w, b).view(np.uint32))
+
+
 def off4(a):
     """The same values 4 bytes past a 16-byte boundary."""
     b = torch.empty(a.numel() + 1, dtype=a.dtype, device=a.device)
