@@ -33,7 +33,10 @@
 // One lane per row reading staged rows from LDS four values at a time, three
 // passes over memory, took 64 (65), 78 (80), 162 (193) us; loading and storing
 // in the chains' layout (64 bytes apart across lanes) 28 (29), 49 (69), 123
-// (182) us.
+// (182) us.  Streamed widths, at 16,384 rows, one lane per row -> chains' layout
+// -> here: h = 256 10 -> 16 -> 8.5 (14 -> 21 -> 12) us, 768 29 -> 35 -> 22 (46 -> 51
+// -> 44), 2048 95 -> 82 -> 62 (131 -> 149 -> 127), 5120 242 -> 269 -> 206 (386 -> 410
+// -> 355); at 64 rows, h = 512, 10 -> 5.0 -> 5.3 (8.6 -> 5.4 -> 5.8).
 #include "common.hpp"
 
 namespace aps {
@@ -83,32 +86,16 @@ __device__ inline float ln_sum_sq(float acc, const LnChunk& t) {
     return acc;
 }
 
-__device__ inline void ln_load(LnChunk& d, const float* src) {
+__device__ inline lf4 ln_add(lf4 v, lf4 r) {
 #pragma unroll
-    for (int p = 0; p < kLnElems / 4; ++p) d.q[p] = reinterpret_cast<const lf4*>(src)[p];
-}
-__device__ inline void ln_store(float* dst, const LnChunk& v) {
-#pragma unroll
-    for (int p = 0; p < kLnElems / 4; ++p) reinterpret_cast<lf4*>(dst)[p] = v.q[p];
-}
-__device__ inline void ln_add(LnChunk& v, const LnChunk& r) {
-#pragma unroll
-    for (int p = 0; p < kLnElems / 4; ++p)
-#pragma unroll
-        for (int k = 0; k < 4; ++k) v.q[p][k] = __fadd_rn(v.q[p][k], r.q[p][k]);
+    for (int k = 0; k < 4; ++k) v[k] = __fadd_rn(v[k], r[k]);
+    return v;
 }
 __device__ inline void ln_deviation(LnChunk& v, float mean) {
 #pragma unroll
     for (int p = 0; p < kLnElems / 4; ++p)
 #pragma unroll
         for (int k = 0; k < 4; ++k) v.q[p][k] = __fsub_rn(v.q[p][k], mean);
-}
-// y = fma(t * inv, w, b)
-__device__ inline void ln_scale(LnChunk& t, float inv, const LnChunk& w, const LnChunk& b) {
-#pragma unroll
-    for (int p = 0; p < kLnElems / 4; ++p)
-#pragma unroll
-        for (int k = 0; k < 4; ++k) t.q[p][k] = __fmaf_rn(__fmul_rn(t.q[p][k], inv), w.q[p][k], b.q[p][k]);
 }
 __device__ inline float ln_inv(float var, int h, float eps) {
     // sqrtf, not __fsqrt_rn: under -fhip-fp32-correctly-rounded-divide-sqrt
@@ -118,40 +105,47 @@ __device__ inline float ln_inv(float var, int h, float eps) {
     return __fdiv_rn(1.0f, sqrtf(__fadd_rn(__fdiv_rn(var, static_cast<float>(h)), eps)));
 }
 
-// This lane's place: its row (rows past the end load the last one and store
-// nothing) and its first element in every chunk.
+// row k's value, from its DPP row, in every lane
+__device__ inline float ln_row(float v, int k) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 16 * k));
+}
+
+// Memory is read and written whole 1 KB row chunks at a time (lane s holds 16
+// bytes of each of the 4 rows); LDS turns a chunk between that layout and the
+// chains' (64 consecutive bytes of one row per lane).  Lane s's 16 bytes are
+// columns io .. io + 3 of the chunk, slot s; the piece p of chain lane L lies in
+// slot 4 L + (p ^ (L / 4)), so that 16 chain lanes read 16 different bank groups.
+__device__ inline int ln_slot(int p) {
+    const int L = threadIdx.x & 15;
+    return 4 * L + (p ^ (L >> 2));
+}
+__device__ inline void ln_turned(LnChunk& v, const lf4 (&turn)[kLnRows][64]) {
+#pragma unroll
+    for (int p = 0; p < 4; ++p) v.q[p] = turn[threadIdx.x >> 4][ln_slot(p)];
+}
 struct LnLane {
-    int64_t at;
-    bool valid;
-    int col;
+    int s, io, nr;
+    int64_t at[kLnRows];   // rows past the end load the last one and store nothing
     __device__ LnLane(int64_t rows, int h) {
-        const int lane = threadIdx.x;
-        const int64_t r = static_cast<int64_t>(blockIdx.x) * kLnRows + (lane >> 4);
-        valid = r < rows;
-        col = kLnElems * (lane & 15);
-        at = (valid ? r : rows - 1) * static_cast<int64_t>(h) + col;
+        s = threadIdx.x;
+        io = 16 * (s >> 2) + 4 * ((s & 3) ^ ((s >> 4) & 3));
+        const int64_t r0 = static_cast<int64_t>(blockIdx.x) * kLnRows;
+        nr = rows - r0 < kLnRows ? static_cast<int>(rows - r0) : kLnRows;   // wave-uniform
+#pragma unroll
+        for (int k = 0; k < kLnRows; ++k) at[k] = (r0 + (k < nr ? k : nr - 1)) * h + io;
     }
 };
 
-// h = 4096: the row in registers throughout.  Memory is read and written whole
-// 1 KB row chunks at a time (lane s holds 16 bytes of each of the 4 rows); LDS
-// turns a chunk between that layout and the chains' (64 consecutive bytes of
-// one row per lane).  Lane s's 16 bytes are columns io .. io + 3 of the chunk,
-// slot s; the piece p of chain lane L lies in slot 4 L + (p ^ (L / 4)), so that
-// 16 chain lanes read 16 different bank groups.
+// h = 4096: the row in registers throughout.
 template <bool ADD>
 __global__ void __launch_bounds__(64, 1)
 k_layer_norm_resident(float* __restrict__ x, const float* __restrict__ residual, const float* __restrict__ w,
                       const float* __restrict__ b, float* __restrict__ y, int64_t rows, float eps) {
     constexpr int NC = kLnResident, h = NC * kLnChunk;
     __shared__ lf4 turn[2][kLnRows][64];
-    const int s = threadIdx.x, L = s & 15;
-    const int io = 16 * (s >> 2) + 4 * ((s & 3) ^ ((s >> 4) & 3));
-    const int64_t r0 = static_cast<int64_t>(blockIdx.x) * kLnRows;
-    const int nr = rows - r0 < kLnRows ? static_cast<int>(rows - r0) : kLnRows;   // wave-uniform
-    int64_t at[kLnRows];   // rows past the end load the last one and store nothing
-#pragma unroll
-    for (int k = 0; k < kLnRows; ++k) at[k] = (r0 + (k < nr ? k : nr - 1)) * h + io;
+    const LnLane l(rows, h);
+    const int s = l.s, io = l.io, nr = l.nr;
+    const int64_t (&at)[kLnRows] = l.at;
     auto ld = [](const float* p) __attribute__((always_inline)) { return *reinterpret_cast<const lf4*>(p); };
 
     LnChunk v[NC];
@@ -170,15 +164,13 @@ k_layer_norm_resident(float* __restrict__ x, const float* __restrict__ residual,
         for (int k = 0; k < kLnRows; ++k) {
             lf4 u = xs[c % kLnAhead][k];
             if (ADD) {
-#pragma unroll
-                for (int j = 0; j < 4; ++j) u[j] = __fadd_rn(u[j], rs[c % kLnAhead][k][j]);
+                u = ln_add(u, rs[c % kLnAhead][k]);
                 if (k < nr) *reinterpret_cast<lf4*>(x + at[k] + c * kLnChunk) = u;
             }
             turn[c & 1][k][s] = u;
         }
         __builtin_amdgcn_wave_barrier();
-#pragma unroll
-        for (int p = 0; p < 4; ++p) v[c].q[p] = turn[c & 1][s >> 4][4 * L + (p ^ (L >> 2))];
+        ln_turned(v[c], turn[c & 1]);
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_sched_barrier(0);
     };
@@ -213,13 +205,12 @@ k_layer_norm_resident(float* __restrict__ x, const float* __restrict__ residual,
     const float inv_row = ln_inv(ln_last(var), h, eps);
     float inv[kLnRows];
 #pragma unroll
-    for (int k = 0; k < kLnRows; ++k)
-        inv[k] = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, inv_row), 16 * k));
+    for (int k = 0; k < kLnRows; ++k) inv[k] = ln_row(inv_row, k);
     // chunk c of t into the loads' layout, one chunk ahead of its use
     lf4 t[2][kLnRows];
     auto turn_back = [&](int c) __attribute__((always_inline)) {
 #pragma unroll
-        for (int p = 0; p < 4; ++p) turn[c & 1][s >> 4][4 * L + (p ^ (L >> 2))] = v[c].q[p];
+        for (int p = 0; p < 4; ++p) turn[c & 1][s >> 4][ln_slot(p)] = v[c].q[p];
         __builtin_amdgcn_wave_barrier();
 #pragma unroll
         for (int k = 0; k < kLnRows; ++k) t[c & 1][k] = turn[c & 1][k][s];
@@ -242,52 +233,100 @@ k_layer_norm_resident(float* __restrict__ x, const float* __restrict__ residual,
     }
 }
 
-// Any h (a multiple of 256): the chunks are read again for each pass, two
-// ahead.
-template <bool ADD>
+// Any h (a multiple of 256): the chunks are read again for each pass, AHEAD of
+// them in flight, in the same layout; only the two chains' passes turn them.
+template <bool ADD, int AHEAD>
 __global__ void __launch_bounds__(64)
 k_layer_norm(float* __restrict__ x, const float* __restrict__ residual, const float* __restrict__ w,
              const float* __restrict__ b, float* __restrict__ y, int64_t rows, int h, float eps) {
+    __shared__ lf4 turn[2][kLnRows][64];
     const LnLane l(rows, h);
     const int NC = h / kLnChunk;
-    // f(c, chunk c of x); chunks past the end re-read the last one
-    auto each = [&](auto f) __attribute__((always_inline)) {
-        LnChunk v[2];
-        auto load = [&](LnChunk& d, int c) __attribute__((always_inline)) {
-            ln_load(d, x + l.at + (c < NC ? c : NC - 1) * kLnChunk);
+    auto ld = [](const float* p) __attribute__((always_inline)) { return *reinterpret_cast<const lf4*>(p); };
+    // f(c, x of chunk c, a second operand of chunk c loaded by also); loads past
+    // the end re-read the last chunk, so that every load is unconditional and a
+    // chunk's wait leaves the later ones in flight
+    auto each = [&](auto also, auto f) __attribute__((always_inline)) {
+        lf4 xs[AHEAD][kLnRows];
+        decltype(also(0)) as[AHEAD];
+        auto load = [&](int d, int c) __attribute__((always_inline)) {
+            c = c < NC ? c : NC - 1;
+#pragma unroll
+            for (int k = 0; k < kLnRows; ++k) xs[d][k] = ld(x + l.at[k] + c * kLnChunk);
+            as[d] = also(c);
+            __builtin_amdgcn_sched_barrier(0);
         };
-        load(v[0], 0);
-        for (int c = 0; c < NC; c += 2) {
-            load(v[1], c + 1);
-            f(c, v[0]);
-            load(v[0], c + 2);
-            if (c + 1 < NC) f(c + 1, v[1]);
+#pragma unroll
+        for (int d = 0; d < AHEAD; ++d) load(d, d);
+        for (int c0 = 0; c0 < NC; c0 += AHEAD) {
+#pragma unroll
+            for (int d = 0; d < AHEAD; ++d) {
+                if (c0 + d >= NC) break;   // wave-uniform
+                f(c0 + d, xs[d], as[d]);
+                load(d, c0 + d + AHEAD);
+            }
         }
     };
+    struct Four {
+        lf4 r[kLnRows];
+    };
+    struct None {};
+    const auto none = [](int) { return None{}; };
+    auto turned = [&](int c, const lf4 (&u)[kLnRows]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int k = 0; k < kLnRows; ++k) turn[c & 1][k][l.s] = u[k];
+        __builtin_amdgcn_wave_barrier();
+        LnChunk v;
+        ln_turned(v, turn[c & 1]);
+        __builtin_amdgcn_wave_barrier();
+        return v;
+    };
     float acc = 0.0f;
-    each([&](int c, LnChunk& v) __attribute__((always_inline)) {
-        if (ADD) {
-            LnChunk r;
-            ln_load(r, residual + l.at + c * kLnChunk);
-            ln_add(v, r);
-            if (l.valid) ln_store(x + l.at + c * kLnChunk, v);
-        }
-        acc = ln_sum(acc, v);
-    });
+    if constexpr (ADD) {
+        each([&](int c) __attribute__((always_inline)) {
+            Four r;
+#pragma unroll
+            for (int k = 0; k < kLnRows; ++k) r.r[k] = ld(residual + l.at[k] + c * kLnChunk);
+            return r;
+        }, [&](int c, lf4 (&u)[kLnRows], const Four& r) __attribute__((always_inline)) {
+#pragma unroll
+            for (int k = 0; k < kLnRows; ++k) {
+                u[k] = ln_add(u[k], r.r[k]);
+                if (k < l.nr) *reinterpret_cast<lf4*>(x + l.at[k] + c * kLnChunk) = u[k];
+            }
+            acc = ln_sum(acc, turned(c, u));
+        });
+    } else {
+        each(none, [&](int c, lf4 (&u)[kLnRows], None) __attribute__((always_inline)) { acc = ln_sum(acc, turned(c, u)); });
+    }
     const float mean = __fdiv_rn(ln_last(acc), static_cast<float>(h));
     float var = 0.0f;
-    each([&](int c, LnChunk& v) __attribute__((always_inline)) {
+    each(none, [&](int c, lf4 (&u)[kLnRows], None) __attribute__((always_inline)) {
+        LnChunk v = turned(c, u);
         ln_deviation(v, mean);
         var = ln_sum_sq(var, v);
     });
-    const float inv = ln_inv(ln_last(var), h, eps);
-    each([&](int c, LnChunk& v) __attribute__((always_inline)) {
-        LnChunk wv, bv;
-        ln_load(wv, w + c * kLnChunk + l.col);
-        ln_load(bv, b + c * kLnChunk + l.col);
-        ln_deviation(v, mean);
-        ln_scale(v, inv, wv, bv);
-        if (l.valid) ln_store(y + l.at + c * kLnChunk, v);
+    const float inv_row = ln_inv(ln_last(var), h, eps);
+    float m[kLnRows], inv[kLnRows];
+#pragma unroll
+    for (int k = 0; k < kLnRows; ++k) {
+        m[k] = ln_row(mean, k);
+        inv[k] = ln_row(inv_row, k);
+    }
+    struct Two {
+        lf4 w, b;
+    };
+    each([&](int c) __attribute__((always_inline)) {
+        return Two{ld(w + c * kLnChunk + l.io), ld(b + c * kLnChunk + l.io)};
+    }, [&](int c, lf4 (&u)[kLnRows], const Two& p) __attribute__((always_inline)) {
+#pragma unroll
+        for (int k = 0; k < kLnRows; ++k) {
+            lf4 o;
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                o[j] = __fmaf_rn(__fmul_rn(__fsub_rn(u[k][j], m[k]), inv[k]), p.w[j], p.b[j]);
+            if (k < l.nr) *reinterpret_cast<lf4*>(y + l.at[k] + c * kLnChunk) = o;
+        }
     });
 }
 
@@ -303,10 +342,11 @@ hipError_t launch_layer_norm(float* x, const float* residual, const float* weigh
             hipLaunchKernelGGL(k_layer_norm_resident<true>, grid, dim3(64), 0, s, x, residual, weight, bias, y, rows, eps);
         else
             hipLaunchKernelGGL(k_layer_norm_resident<false>, grid, dim3(64), 0, s, x, residual, weight, bias, y, rows, eps);
-    } else if (residual) {
-        hipLaunchKernelGGL(k_layer_norm<true>, grid, dim3(64), 0, s, x, residual, weight, bias, y, rows, hidden, eps);
     } else {
-        hipLaunchKernelGGL(k_layer_norm<false>, grid, dim3(64), 0, s, x, residual, weight, bias, y, rows, hidden, eps);
+        const int nc = hidden / kLnChunk;
+        auto kern = residual ? (nc == 1 ? k_layer_norm<true, 1> : nc < 4 ? k_layer_norm<true, 2> : k_layer_norm<true, 4>)
+                             : (nc == 1 ? k_layer_norm<false, 1> : nc < 4 ? k_layer_norm<false, 2> : k_layer_norm<false, 4>);
+        hipLaunchKernelGGL(kern, grid, dim3(64), 0, s, x, residual, weight, bias, y, rows, hidden, eps);
     }
     return hipGetLastError();
 }

@@ -68,6 +68,32 @@ def test_layer_norm_row_groups(gpu_device, rows, h):
     np.testing.assert_array_equal(xd.cpu().numpy().view(np.uint32), want_v.view(np.uint32))
 
 
+@pytest.mark.parametrize("rows", [3, 9])
+@pytest.mark.parametrize("h", [256, 512, 768, 1024, 1792, 2048, 5120, 8192])
+@pytest.mark.parametrize("add", [False, True])
+def test_layer_norm_streamed_widths(gpu_device, rows, h, add):
+    """One, two and four chunks of loads in flight, chunk counts around them;
+    a last wave of one and of three rows.  Rows of NaN around the output show a
+    store past its rows."""
+    note(f"layer norm streamed rows={rows} h={h} add={add}")
+    x, r, w, b = _inputs(rows, h, rows * h + add)
+    x *= np.exp2(np.random.default_rng(rows).integers(-12, 13, (rows, h))).astype(np.float32)
+    guard = torch.full((rows + 4, h), float("nan"), device=gpu_device)
+    xd = guard.clone()
+    xd[2:-2] = _dev(x, gpu_device)
+    rd, wd, bd = (_dev(a, gpu_device) for a in (r, w, b))
+    y = guard.clone()
+    if add:
+        moe.add_layer_norm_gpu(xd[2:-2], rd, wd, bd, moe.NORM_EPS, y[2:-2])
+    else:
+        moe.layer_norm_gpu(xd[2:-2], wd, bd, moe.NORM_EPS, y[2:-2])
+    want_y, want_v, _, _ = oracle.layer_norm(x, w, b, eps=moe.NORM_EPS, residual=r if add else None)
+    for got, want in ((y, want_y), (xd, want_v if add else x)):
+        got = got.cpu().numpy()
+        np.testing.assert_array_equal(got[2:-2].view(np.uint32), want.view(np.uint32))
+        assert np.isnan(got[:2]).all() and np.isnan(got[-2:]).all()
+
+
 def test_layer_norm_known_answer_rows(gpu_device):
     """The oracle's order and fused-variance known-answer rows (the mean of
     [1e8, 1, -1e8, 0...] is 0, that of [1e8, -1e8, 1, 0...] is 2^-12; the
