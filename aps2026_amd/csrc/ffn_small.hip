@@ -411,8 +411,17 @@ int small_kt(bool fp8, int ffn) { return static_cast<int>(fp8 ? ceil_div(ffn, 12
 //         64), 128 69 -> 59 (70 -> 78), 256 70 -> 83 (73 -> 84)
 //   fp8   1 token 74 -> 44 (73 -> 44), 65 86 -> 58 (86 -> 61), 192 87 -> 63 (87 ->
 //         71), 384 87 -> 82 (91 -> 83), 613 88 -> 114 (95 -> 117)
+//   Past 128 blocks of 64 columns over all experts (E F > 8192) the row tiles
+// fill the chip by themselves, and a skewed load sends many rows to an expert
+// while the mean is low: there up to 8 experts' worth.  us row tiles -> here, 64
+// experts, hidden 2048, even (Zipf 1.1 / 2.2) loads: F = 448 bf16 64 tokens 99 -> 105
+// (88 -> 98 / 68 -> 68), 256 tokens 114 -> 123 (113 -> 136 / 83 -> 113), fp8 512 tokens
+// 90 -> 98 (94 -> 117 / 85 -> 103); F = 64, hidden 4096, bf16 256 tokens 101 -> 91 (103 ->
+// 94 / 101 -> 92); 24 experts of 448, hidden 4096, bf16 96 tokens 90 -> 87 (92 -> 94 /
+// 83 -> 92).
 bool ffn_small_fits(bool fp8, int64_t rows, int ffn, int experts) {
-    return 2 * rows <= (fp8 ? 24 : 12) * static_cast<int64_t>(experts) && small_kt(fp8, ffn) <= (fp8 ? 4 : 7);
+    const int64_t mean = fp8 ? 24 : 12, E = experts;
+    return 2 * rows <= mean * E && (E * ffn <= 8192 || 2 * rows <= mean * 8) && small_kt(fp8, ffn) <= (fp8 ? 4 : 7);
 }
 
 // w2's whole K is in flight at once and its tiles read less again, so it gains
@@ -422,7 +431,12 @@ bool ffn_small_fits(bool fp8, int64_t rows, int ffn, int experts) {
 //         85), 512 83 -> 91 (95 -> 100)
 //   fp8   224 tokens 56 -> 51 (57 -> 54), 256 56 -> 53 (59 -> 58), 384 69 -> 70 (73 ->
 //         73), 613 71 -> 77 (78 -> 80)
+//   Many experts keep the mean low whatever the load: past 512 bf16 tokens an
+// expert that takes them all reads its weights too often (64 experts, hidden
+// 4096, us row tiles -> here, even / Zipf 1.1 / every token to two experts: 512
+// tokens 230 -> 218 / 252 -> 253 / 107 -> 118, 768 231 -> 228 / 257 -> 263 / 108 -> 129).
 bool ffn_down_small_fits(bool fp8, int64_t rows, int ffn, int experts) {
+    if (!fp8 && rows > 512) return false;
     return 2 * rows <= (fp8 ? 32 : 24) * static_cast<int64_t>(experts) && small_kt(fp8, ffn) <= (fp8 ? 4 : 7);
 }
 

@@ -77,6 +77,28 @@ def test_w2_tiles_between_the_rules(gpu_device, dtype, E, H, F):
     w.release()
 
 
+@pytest.mark.parametrize("E,H,F", [(24, 512, 448), (17, 256, 512), (64, 256, 128), (64, 256, 192)])
+@pytest.mark.parametrize("dtype", ["bf16", "fp8"])
+def test_many_experts_leave_the_small_tiles_early(gpu_device, dtype, E, H, F):
+    """w1||w3 past 8192 columns over all experts: 8 experts' worth of rows, that
+    edge and one past it, and the mean's own edge, against a batch of row
+    tiles; up to 8192 columns (64 x 128) the mean alone."""
+    per = 24 if dtype == "fp8" else 12
+    print(f"[gpu-case] many experts {dtype} E={E} H={H} F={F}", flush=True)
+    w = weights(dtype, E, H, F, gpu_device, E + F)
+    g = torch.Generator(device=gpu_device)
+    g.manual_seed(E)
+    x = torch.randn((1100, H), generator=g, device=gpu_device)
+    gate = torch.randn((E, H), generator=g, device=gpu_device) * 0.05
+    x[:, 0], gate[:, 0] = 1.0, -1.1 * torch.log(torch.arange(1, E + 1, device=gpu_device).float())
+    x = x.bfloat16()
+    big = moe.moe_forward_gpu(x, gate, w).clone()
+    for n in (4 * per, 4 * per + 1, E * per // 2, E * per // 2 + 1):
+        got = moe.moe_forward_gpu(x[:n].contiguous(), gate, w)
+        assert torch.equal(got.view(torch.int16), big[:n].view(torch.int16)), n
+    w.release()
+
+
 def test_few_rows_plan_past_two_assignments_per_row(gpu_device):
     """The staged w1||w3 call with a plan of more positions than 2 rows: the
     grid covers the rest in further rounds."""
