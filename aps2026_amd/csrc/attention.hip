@@ -790,16 +790,19 @@ hipError_t launch_rope_tree(float* q, float* k, const uint32_t* row_pos, int64_t
     const uintptr_t addr = reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k) |
                            reinterpret_cast<uintptr_t>(cosv) | reinterpret_cast<uintptr_t>(sinv);
     const bool vec = half % 4 == 0 && (addr & 15u) == 0;
-    const int64_t n = rows * (q_heads + kv_heads) * (vec ? half / 4 : half);
-    if (n <= 0) return hipSuccess;
-    const dim3 grid(static_cast<unsigned>(ceil_div(n, 256)));
-    if (vec)
-        hipLaunchKernelGGL(k_rope_tree<4>, grid, dim3(256), 0, s, q, k, row_pos, rows, q_heads, kv_heads, half, cosv,
-                           sinv, max_seq);
-    else
-        hipLaunchKernelGGL(k_rope_tree<1>, grid, dim3(256), 0, s, q, k, row_pos, rows, q_heads, kv_heads, half, cosv,
-                           sinv, max_seq);
-    return hipGetLastError();
+    // (a launch of 2^32 threads or more would drop the rest without an error)
+    const int64_t per_row = static_cast<int64_t>(q_heads + kv_heads) * (vec ? half / 4 : half);
+    const int64_t most = (int64_t(1) << 31) / per_row > 0 ? (int64_t(1) << 31) / per_row : 1;
+    for (int64_t r0 = 0; r0 < rows; r0 += most) {
+        const int64_t nr = rows - r0 < most ? rows - r0 : most;
+        hipLaunchKernelGGL(vec ? k_rope_tree<4> : k_rope_tree<1>,
+                           dim3(static_cast<unsigned>(ceil_div(nr * per_row, 256))), dim3(256), 0, s,
+                           q + r0 * q_heads * head_dim, k + r0 * kv_heads * head_dim, row_pos + r0, nr, q_heads,
+                           kv_heads, half, cosv, sinv, max_seq);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
 }
 
 hipError_t launch_attention_tree(const float* q, const float* k, const float* v, float* out, const uint32_t* row_pos,

@@ -365,6 +365,27 @@ def test_attention_non_finite_values_outside_the_window(gpu_device, packed, wind
         np.testing.assert_array_equal(got.view(np.uint32)[ok], want.view(np.uint32)[ok])
 
 
+def test_rope_of_more_pairs_than_a_launch_has_threads(gpu_device):
+    """3.5 million unaligned rows: one pair per thread, 4.5e9 pairs (36 GB)."""
+    from aps2026_amd import capi
+    from aps2026_amd.moe import _ptr, _stream
+    note("rope past 2^32 pairs")
+    rows, heads, kv = 3_500_000, 16, 4
+    flat = torch.ones(1 + rows * (heads + kv) * 128, device=gpu_device)
+    q, k = flat[1:1 + rows * heads * 128].view(rows, -1), flat[1 + rows * heads * 128:].view(rows, -1)
+    pos = torch.ones(rows, dtype=torch.int32, device=gpu_device)
+    c, s = torch.full((2, 64), 0.5, device=gpu_device), torch.full((2, 64), 0.25, device=gpu_device)
+    rc = capi.lib().aps_rope_tree(_ptr(q), _ptr(k), _ptr(pos), rows, heads, kv, 128, _ptr(c), _ptr(s), 2,
+                                  _stream(gpu_device))
+    assert rc == 0, capi.last_error()
+    for x in (q, k):   # 0.5 - 0.25 and 0.5 + 0.25
+        for r0 in range(0, rows, 500_000):
+            h = x[r0:r0 + 500_000].view(-1, 2, 64)
+            assert bool((h[:, 0] == 0.25).all()) and bool((h[:, 1] == 0.75).all()), r0
+    del flat, q, k, h, x
+    torch.cuda.empty_cache()
+
+
 def test_attention_nodes_equal_token_rows(gpu_device):
     note("attention tree nodes vs token rows")
     batch = shared_batch(4, groups=2, per=4, pre=60, suf=20)
