@@ -220,8 +220,11 @@ class DecoderLayer:
             # against 170).  Past 1,024 rows each grid fills the chip by
             # itself and q alone, then k and v together, balance better
             # (2,048 rows 361 us against 368, 10,240 rows 1775 against 1861)
-            wide = [x for x in names if x[2] >= 2048 and T > 1024]
-            narrow = [x for x in names if x[2] < 2048 or T <= 1024]
+            # (the shared grid takes 16-byte aligned arrays, aps_linear any)
+            alone = lambda nm, dst, n: (n >= 2048 and T > 1024) or any(
+                t is not None and t.data_ptr() % 16 for t in (src, dst) + tuple(self.w.proj[nm]))
+            wide = [x for x in names if alone(*x)]
+            narrow = [x for x in names if not alone(*x)]
             for nm, dst, n in wide:
                 _call(L.aps_linear(_p(src), _p(self.w.proj[nm][0]), _p(self.w.proj[nm][1]), T, K, n, _p(dst),
                                    stream))

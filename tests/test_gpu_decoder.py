@@ -17,6 +17,7 @@ src/model.cu:58-64), the bf16-expert model's first layer routes exactly as
 the fp32-expert model (the reference's arithmetic), and the per-layer
 routing agreement between the two is reported.
 """
+import dataclasses
 import sys
 
 import numpy as np
@@ -131,6 +132,39 @@ def test_c3_decoder_layer_parity(gpu_device):
     note(f"C3 stages bit-exact through the router; counts {counts.tolist()}; MoE max normwise err {err.max():.3e}")
     assert err.max() <= TOL_BF16
     lw.release()
+
+
+def test_projections_of_unaligned_weights(gpu_device):
+    """Projection weights and biases that are only 4-byte aligned (views into
+    a checkpoint's storage), below and past the row count from which each wide
+    output has a grid of its own: the bits of the aligned ones."""
+    from aps2026_amd.moe import _stream
+    note("decoder projections of unaligned weights")
+    H, g = 512, torch.Generator(device=gpu_device)
+    g.manual_seed(6)
+    lw = decoder.random_layer(H, 64, 2, gpu_device, g)
+
+    def off(t):
+        b = torch.empty(t.numel() + 1, device=gpu_device)
+        b[1:] = t.reshape(-1)
+        return b[1:].view(t.shape)
+
+    names = [("q_proj", "q", decoder.QD), ("k_proj", "k", decoder.KD), ("v_proj", "v", decoder.KD)]
+    for rows in (40, 1100):
+        b = decoder.Buffers.allocate(rows, H, lw.moe, gpu_device)
+        b.normed.normal_(generator=g)
+        got = []
+        for which in ((), ("q_proj",), ("q_proj", "v_proj"), tuple(n for n, _, _ in names)):
+            proj = {n: tuple(off(t) for t in p) if n in which else p for n, p in lw.proj.items()}
+            layer = decoder.DecoderLayer(dataclasses.replace(lw, proj=proj))
+            for _, a, _ in names:
+                getattr(b, a).fill_(float("nan"))
+            layer._project(b, b.normed, [(n, getattr(b, a), w) for n, a, w in names], _stream(gpu_device))
+            got.append([getattr(b, a).view(torch.int32).clone() for _, a, _ in names])
+        assert all(torch.isfinite(t.view(torch.float32)).all() for t in got[0])
+        for other in got[1:]:
+            assert all(torch.equal(x, y) for x, y in zip(other, got[0])), rows
+    lw.moe.release()
 
 
 def test_decoder_layer_split_bf16_projections(gpu_device):
