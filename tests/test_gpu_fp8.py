@@ -54,8 +54,8 @@ def rowwise_err(got, ref):
 
 def run_block(inp, dev):
     """The fused forward (the router quantising x on the way when H = 4096
-    and E <= 16, and for F in (384, 512] the w2 GEMM with the combine folded
-    in), then the grouped forward from the router's logits (x quantised by
+    and E <= 16, and for F in (384, 512] past 384 routes per expert the w2
+    GEMM with the combine folded in), then the grouped forward from the router's logits (x quantised by
     the row quantiser, w2 to y, then k_combine), which leaves every
     intermediate in the workspace: x's codes and scales and the two outputs
     must agree bit for bit."""

@@ -2,7 +2,8 @@
 its output equals aps_moe_forward's with a caller workspace bit for bit, on
 two calls in a row with the second batch smaller than the first (the static
 scratch keeps the first call's bytes), for a bf16, an fp32 and an fp8 weight
-set (the fp8 one runs the folded combine and the router's x quantisation);
+set (the fp8 one runs the router's x quantisation, and past 3,072 tokens the
+folded combine: on two such batches and then on a small, unfolded one);
 a batch past the scratch is refused with APS_ERR_WORKSPACE."""
 import ctypes
 import sys
@@ -48,7 +49,8 @@ def _x(inp, dev):
     return torch.from_numpy(inp.x).to(dev)
 
 
-@pytest.mark.parametrize("dtype,sizes", [("bf16", (4096, 300)), ("f32", (512, 77)), ("fp8", (3000, 129))])
+@pytest.mark.parametrize("dtype,sizes", [("bf16", (4096, 300)), ("f32", (512, 77)), ("fp8", (3000, 129)),
+                                         ("fp8", (3500, 3073, 129))])
 def test_forward_noalloc_equals_workspace_forward(gpu_device, dtype, sizes):
     L = capi.lib()
     T0 = sizes[0]
