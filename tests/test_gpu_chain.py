@@ -26,7 +26,7 @@ def dev(a, d):
     (1, 16, 4), (16, 32, 16), (17, 48, 20), (16, 224, 36), (9, 256, 36), (16, 288, 68), (33, 480, 48), (16, 528, 32),
     (600, 96, 260), (600, 128, 256), (601, 112, 256), (601, 160, 252), (590, 288, 256),
     (333, 32, 4096), (321, 80, 4092), (333, 192, 2048), (333, 48, 2044), (300, 288, 2048),
-    (1000, 32, 2048), (1023, 96, 2044), (1000, 48, 2048), (4095, 32, 1024), (4096, 64, 1020), (4001, 160, 1024)])
+    (1000, 32, 2048), (1023, 96, 2044), (1023, 128, 2044), (1000, 160, 2048), (1000, 192, 2044), (1000, 48, 2048), (4095, 32, 1024), (4096, 64, 1020), (4001, 160, 1024)])
 def test_linear_block_and_stage_edges(gpu_device, rows, k, n):
     note(f"linear edges rows={rows} k={k} n={n}")
     rng = np.random.default_rng(rows + 3 * k + 7 * n)

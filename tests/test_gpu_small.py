@@ -195,3 +195,31 @@ def test_tile_histograms_of_few_tokens(gpu_device, dtype, E, F):
                 continue
             assert np.array_equal(ws[off:off + size].cpu().numpy().reshape(tiles, E, 4), ref), n
     w.release()
+
+
+@pytest.mark.parametrize("H,F", [(4096, 448), (512, 64), (256, 320)])
+def test_dense_ffn_of_few_rows(gpu_device, H, F):
+    """The bf16 one-expert set (aps_mlp_forward): w1||w3 on the one-wave tiles up
+    to 6 rows, w2 up to 12, against the same rows of a batch of row tiles."""
+    from aps2026_amd import capi
+    print(f"[gpu-case] dense ffn few rows H={H} F={F}", flush=True)
+    g = torch.Generator(device=gpu_device)
+    g.manual_seed(H + F)
+    ws = [[(torch.randn(sh, generator=g, device=gpu_device) * 0.05).bfloat16()] for sh in ((F, H), (H, F), (F, H))]
+    w = moe.register_moe_weights_gpu(*ws, compute_dtype=torch.bfloat16)
+    x = torch.randn((300, H), generator=g, device=gpu_device).bfloat16()
+    L = capi.lib()
+
+    def run(n):
+        size = L.aps_mlp_workspace_size(w.handle, n)
+        scratch = torch.empty(size, dtype=torch.uint8, device=gpu_device)
+        out = torch.full((n, H), float("nan"), dtype=torch.bfloat16, device=gpu_device)
+        rc = L.aps_mlp_forward(w.handle, x.data_ptr(), capi.DTYPE_BF16, n, out.data_ptr(), scratch.data_ptr(), size,
+                               moe._stream(gpu_device))
+        assert rc == 0, capi.last_error()
+        return out
+
+    big = run(300)
+    for n in (1, 5, 6, 7, 12, 13):
+        assert torch.equal(run(n).view(torch.int16), big[:n].view(torch.int16)), n
+    w.release()
