@@ -192,21 +192,23 @@ int check_x_dtype(const WeightSet& w, int32_t x_dtype) {
     return APS_OK;
 }
 
-// Routing (from `logits`; nullptr when the router kernel already wrote the
-// routes into the workspace, and past few tokens the tile histogram), dispatch,
-// FFN and combine.  The fp8 path with bf16 output folds the combine into the w2
-// GEMM of a large batch routed here (aps_moe_forward): no y round trip.  The
-// slot lists and both histograms, part of the plan that callers may read
-// back, are in the workspace at any size.
-bool fold_combine(const WeightSet& w, int64_t rows, int32_t out_dtype) {
+// Whether the plan has the slot lists: where the fp8 path with bf16 output can
+// fold the combine into the w2 GEMM.  They are part of the plan that callers
+// may read back, so they are there whether or not the batch folds.
+bool slot_lists(const WeightSet& w, int64_t rows, int32_t out_dtype) {
     return w.compute == APS_DTYPE_E4M3 && out_dtype == APS_DTYPE_BF16 && aps::ffn_down_fold_fits(rows, w.H, w.F);
 }
 
+// Routing (from `logits`; nullptr when the router kernel already wrote the
+// routes into the workspace, and past few tokens the tile histogram), dispatch,
+// FFN and combine.
+// slots: the plan with the slot lists (aps_moe_forward); a large batch then
+// folds the combine into w2, with no y round trip.
 // xq_ready: the router has written the fp8 codes and scales of x (fp8 path).
 // few: it was the few-token router, which writes no tile histogram.
 int grouped_from_logits(const WeightSet& w, const void* x, bool x_is_f32, const float* logits, int64_t rows,
                         void* out, int32_t out_dtype, char* ws, const aps_moe_ws_layout& L,
-                        hipStream_t s, bool fold = false, bool xq_ready = false, bool few = false) {
+                        hipStream_t s, bool slots = false, bool xq_ready = false, bool few = false) {
     auto* routes = reinterpret_cast<uint8_t*>(ws + L.routes);
     auto* tiles = reinterpret_cast<uint32_t*>(ws + L.tile_counts);
     auto* counts = reinterpret_cast<uint32_t*>(ws + L.counts);
@@ -224,10 +226,10 @@ int grouped_from_logits(const WeightSet& w, const void* x, bool x_is_f32, const 
     auto* srows = reinterpret_cast<uint32_t*>(ws + L.slot_rows);
     auto* stoks = reinterpret_cast<uint32_t*>(ws + L.slot_tokens);
     // few tokens on the one-wave tiles: the w1||w3 launch makes the plan itself
-    const aps::SmallPlan plan{routes, tiles, counts, offsets, arows, rpos, fold ? slot1 : nullptr, srows, stoks, tiles0};
+    const aps::SmallPlan plan{routes, tiles, counts, offsets, arows, rpos, slots ? slot1 : nullptr, srows, stoks, tiles0};
     const bool planned = few && w.compute != APS_DTYPE_F32 &&
                          aps::ffn_small_fits(w.compute == APS_DTYPE_E4M3, rows, w.F, w.E);
-    if (!planned && fold)
+    if (!planned && slots)
         APS_HIP(aps::launch_dispatch_scatter(routes, few ? nullptr : tiles, rows, w.E, counts, offsets, arows, rpos,
                                              nullptr, s, few ? nullptr : tiles0, slot1, srows, stoks, tiles, tiles0),
                 "dispatch launch");
@@ -258,7 +260,7 @@ int grouped_from_logits(const WeightSet& w, const void* x, bool x_is_f32, const 
         // experts, us folded -> unfolded, even (Zipf 1.1) loads: 320 tokens 87 -> 68
         // (90 -> 71), 1024 92 -> 78 (98 -> 81), 2048 111 -> 107 (122 -> 107), 3072 118
         // -> 114 (127 -> 119), 4096 131 -> 133 (145 -> 136), 8192 223 -> 234 (223 -> 235)
-        if (fold && 2 * rows > 384 * static_cast<int64_t>(w.E)) {
+        if (slots && 2 * rows > 384 * static_cast<int64_t>(w.E)) {
             // slot-0 rows to y's bytes as [rows][H] by token, then slot-1 rows
             // combined with them straight into out
             APS_HIP(aps::launch_ffn_down_fold_fp8(actq, as, offsets, slot1, srows, stoks, w.q2, w.s2,
@@ -953,8 +955,8 @@ int aps_moe_forward(uint64_t handle, const void* x, int32_t x_dtype, const float
     auto* tiles = reinterpret_cast<uint32_t*>(ws + L.tile_counts);
     const bool copy = x_dtype == APS_DTYPE_F32 && w->compute == APS_DTYPE_BF16;
     auto* xb = copy ? reinterpret_cast<aps::bf16_t*>(ws + L.xq) : nullptr;
-    const bool fold = fold_combine(*w, rows, out_dtype);
-    auto* tiles0 = fold ? reinterpret_cast<uint32_t*>(ws + L.tile_counts0) : nullptr;
+    const bool slots = slot_lists(*w, rows, out_dtype);
+    auto* tiles0 = slots ? reinterpret_cast<uint32_t*>(ws + L.tile_counts0) : nullptr;
     // fp8 weights with bf16 x: the router also writes x's e4m3 codes and row
     // scales (x read once for both)
     const bool xq_in_router = w->compute == APS_DTYPE_E4M3 && x_dtype == APS_DTYPE_BF16 &&
@@ -972,8 +974,8 @@ int aps_moe_forward(uint64_t handle, const void* x, int32_t x_dtype, const float
         APS_HIP(aps::launch_router(x, x_dtype == APS_DTYPE_BF16, gate, rows, w->H, w->E, logits, routes, tiles, tiles0,
                                    xb, xq, xqs, s),
                 "router launch");
-    if (copy) return grouped_from_logits(*w, xb, false, nullptr, rows, out, out_dtype, ws, L, s, fold, false, few);
-    return grouped_from_logits(*w, x, x_dtype == APS_DTYPE_F32, nullptr, rows, out, out_dtype, ws, L, s, fold,
+    if (copy) return grouped_from_logits(*w, xb, false, nullptr, rows, out, out_dtype, ws, L, s, slots, false, few);
+    return grouped_from_logits(*w, x, x_dtype == APS_DTYPE_F32, nullptr, rows, out, out_dtype, ws, L, s, slots,
                                xq_in_router, few);
 }
 

@@ -20,14 +20,6 @@ __device__ inline uint32_t f32_to_bf16_bits(float f) {
     return __builtin_bit_cast(uint16_t, static_cast<__bf16>(f));
 }
 
-typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-__device__ inline uint32_t pack2_bf16(float lo, float hi) {
-    bf16x2_t v;
-    v[0] = static_cast<__bf16>(lo);
-    v[1] = static_cast<__bf16>(hi);
-    return __builtin_bit_cast(uint32_t, v);
-}
-
 template <bool YBF16>
 __device__ inline void load8(const void* y, int64_t off, float v[8]) {
     if (YBF16) {

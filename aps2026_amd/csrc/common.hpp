@@ -24,6 +24,21 @@ using bf16_t = uint16_t;            // raw bfloat16 bits in memory
 
 __host__ __device__ inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
+// Two fp32 -> packed bf16, round to nearest even (one v_cvt_pk_bf16_f32).
+typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+__device__ inline uint32_t pack2_bf16(float lo, float hi) {
+    bf16x2_t v;
+    v[0] = static_cast<__bf16>(lo);
+    v[1] = static_cast<__bf16>(hi);
+    return __builtin_bit_cast(uint32_t, v);
+}
+
+// lane i of each 16-lane DPP row <- lane i - 1 (lane 0 <- lane 15)
+__device__ inline float row_ror1(float v) {
+    const int i = __builtin_bit_cast(int, v);
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(i, i, 0x121, 0xF, 0xF, true));
+}
+
 // q = sign(l) * floorf(|l| / Q + 0.5f) * Q with every step rounded on its own
 // (the _rn intrinsics keep the compiler from contracting the multiply into a
 // later add).  Reference src/layer.cu:72-77, src/tensor.cu:1300-1306.

@@ -50,11 +50,6 @@ constexpr int kLnAhead = 4;      // chunks of loads in flight
 
 typedef float lf4 __attribute__((ext_vector_type(4)));
 
-// lane i of each 16-lane row <- lane i - 1 (lane 0 <- lane 15)
-__device__ inline float ln_ror1(float v) {
-    const int i = __builtin_bit_cast(int, v);
-    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(i, i, 0x121, 0xF, 0xF, true));
-}
 // lane 15's value in every lane of its row
 __device__ inline float ln_last(float v) {
     const int i = __builtin_bit_cast(int, v);
@@ -70,7 +65,7 @@ struct LnChunk {
 __device__ inline float ln_sum(float acc, const LnChunk& v) {
 #pragma unroll 4
     for (int i = 0; i < 16; ++i) {
-        acc = __fadd_rn(ln_ror1(acc), v.q[0][0]);
+        acc = __fadd_rn(row_ror1(acc), v.q[0][0]);
 #pragma unroll
         for (int e = 1; e < kLnElems; ++e) acc = __fadd_rn(acc, v.q[e / 4][e % 4]);
     }
@@ -79,7 +74,7 @@ __device__ inline float ln_sum(float acc, const LnChunk& v) {
 __device__ inline float ln_sum_sq(float acc, const LnChunk& t) {
 #pragma unroll 4
     for (int i = 0; i < 16; ++i) {
-        acc = ln_ror1(acc);
+        acc = row_ror1(acc);
 #pragma unroll
         for (int e = 0; e < kLnElems; ++e) acc = __fmaf_rn(t.q[e / 4][e % 4], t.q[e / 4][e % 4], acc);
     }

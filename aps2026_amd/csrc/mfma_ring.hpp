@@ -15,7 +15,6 @@
 namespace aps {
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
 typedef int i32x4_t __attribute__((ext_vector_type(4)));
 typedef int i32x8_t __attribute__((ext_vector_type(8)));
@@ -35,14 +34,6 @@ constexpr int kImageBytes = 128 * kRowBytes;   // one packed weight tile image
 // row, and the eight pairs of a 16-row group get eight different chunks --
 // sixteen distinct 16-byte bank groups, no conflict.
 __device__ inline int swz(int row, int chunk) { return row * kRowBytes + ((chunk ^ ((row >> 1) & 7)) << 4); }
-
-// Two fp32 -> packed bf16, round to nearest even (one v_cvt_pk_bf16_f32).
-__device__ inline uint32_t pack2_bf16(float lo, float hi) {
-    bf16x2_t v;
-    v[0] = static_cast<__bf16>(lo);
-    v[1] = static_cast<__bf16>(hi);
-    return __builtin_bit_cast(uint32_t, v);
-}
 
 // silu(g) * u for the MFMA paths: fp32 math with the hardware exp2 and
 // reciprocal (the result is rounded to bf16, far coarser than their error).

@@ -184,16 +184,6 @@ struct RInt {
     constexpr operator int() const { return V; }
 };
 
-// Two fp32 -> packed bf16, round to nearest even (v_cvt_pk_bf16_f32), the
-// same conversion as the library's standalone fp32 -> bf16 kernel.
-__device__ inline uint32_t r_pack2_bf16(float lo, float hi) {
-    typedef __bf16 rbf16x2_t __attribute__((ext_vector_type(2)));
-    rbf16x2_t v;
-    v[0] = static_cast<__bf16>(lo);
-    v[1] = static_cast<__bf16>(hi);
-    return __builtin_bit_cast(uint32_t, v);
-}
-
 // One workgroup = 16 tokens x 16 R expert lanes.  logits [rows][E] always;
 // routes [rows][2] and the tile histogram when routes != nullptr.  XCOPY
 // (fp32 x only): the bf16 copy of x the expert FFN reads is written on the
@@ -322,8 +312,8 @@ k_router(const void* xv, const float* __restrict__ gate, int64_t rows, int H, in
         if constexpr (XCOPY) {
 #pragma unroll
             for (int wi = 0; wi < kGW; ++wi) {
-                const ru32x4_t pk = {r_pack2_bf16(c[wi][0], c[wi][1]), r_pack2_bf16(c[wi][2], c[wi][3]),
-                                     r_pack2_bf16(c[wi][4], c[wi][5]), r_pack2_bf16(c[wi][6], c[wi][7])};
+                const ru32x4_t pk = {pack2_bf16(c[wi][0], c[wi][1]), pack2_bf16(c[wi][2], c[wi][3]),
+                                     pack2_bf16(c[wi][4], c[wi][5]), pack2_bf16(c[wi][6], c[wi][7])};
                 *reinterpret_cast<ru32x4_t*>(xdst + (g * kGW + wi) * kRWin) = pk;
             }
         }

@@ -19,9 +19,7 @@
 //   A workgroup's four waves are the 16 experts of one token.  The fp8 codes
 // of x come from further workgroups of the same launch, beside the chains
 // instead of after them.
-#include <type_traits>
-
-#include "common.hpp"
+#include "chain_mfma.hpp"
 
 namespace aps {
 namespace {
@@ -32,19 +30,6 @@ constexpr int kRfMaxE = 16;
 
 typedef uint32_t rf_u4 __attribute__((ext_vector_type(4)));
 typedef float rf_f4 __attribute__((ext_vector_type(4)));
-
-__device__ inline float rf_ror1(float v) {
-    const int i = __builtin_bit_cast(int, v);
-    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(i, i, 0x121, 0xF, 0xF, true));
-}
-
-#define APS_FGP(p) ((const __attribute__((address_space(1))) void*)(p))
-#define APS_FLP(p) ((__attribute__((address_space(3))) void*)(p))
-
-template <int N>
-__device__ inline void rf_wait_vm() {
-    __builtin_amdgcn_s_waitcnt((N & 0xF) | (0x7 << 4) | (0xF << 8) | ((N >> 4) << 14));
-}
 
 // This lane's operands of a chunk.
 template <bool XBF16>
@@ -63,14 +48,6 @@ struct RfSlot {
     // physical piece of lane i's logical piece p
     __device__ static int piece(int i, int p) { return p ^ ((i >> 1) & 7); }
 };
-
-__device__ inline uint32_t rf_pack2_bf16(float lo, float hi) {
-    typedef __bf16 rbf16x2_t __attribute__((ext_vector_type(2)));
-    rbf16x2_t v;
-    v[0] = static_cast<__bf16>(lo);
-    v[1] = static_cast<__bf16>(hi);
-    return __builtin_bit_cast(uint32_t, v);
-}
 
 // Blocks 0 .. rows - 1: one token each; with xq, four rows of x per further block.
 template <bool XBF16>
@@ -114,13 +91,13 @@ k_router_few(const void* __restrict__ xv, const float* __restrict__ gate, int64_
 #pragma unroll
                 for (int k = 0; k < kRfElems; k += 8)
                     *reinterpret_cast<rf_u4*>(xcopy + t * H + c * kRfChunk + kRfElems * i + k) =
-                        rf_u4{rf_pack2_bf16(xe[k], xe[k + 1]), rf_pack2_bf16(xe[k + 2], xe[k + 3]),
-                              rf_pack2_bf16(xe[k + 4], xe[k + 5]), rf_pack2_bf16(xe[k + 6], xe[k + 7])};
+                        rf_u4{pack2_bf16(xe[k], xe[k + 1]), pack2_bf16(xe[k + 2], xe[k + 3]),
+                              pack2_bf16(xe[k + 4], xe[k + 5]), pack2_bf16(xe[k + 6], xe[k + 7])};
             }
         }
 #pragma unroll 1
         for (int r = 0; r < 16; ++r) {
-            acc = rf_ror1(acc);
+            acc = row_ror1(acc);
 #pragma unroll
             for (int k = 0; k < kRfElems; ++k) acc = __fmaf_rn(xe[k], d.g[k / 4][k % 4], acc);
         }
@@ -172,13 +149,13 @@ k_router_few(const void* __restrict__ xv, const float* __restrict__ gate, int64_
             c = c < NC ? c : NC - 1;
 #pragma unroll
             for (int j = 0; j < RfSlot::kCopies; ++j)
-                __builtin_amdgcn_global_load_lds(APS_FGP(src[j] + c * 4 * kRfChunk), APS_FLP(to + 1024 * j), 16, 0, 0);
+                __builtin_amdgcn_global_load_lds(APS_CGP(src[j] + c * 4 * kRfChunk), APS_CLP(to + 1024 * j), 16, 0, 0);
         };
         // (by LDS address: through the ring object the compiler would wait for
         // every copy in flight before each read)
         typedef const __attribute__((address_space(3))) rf_f4* lds_f4;
         typedef const __attribute__((address_space(3))) rf_u4* lds_u4;
-        const uint32_t base = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(APS_FLP(&ring[wave][0]))) + 128u * i;
+        const uint32_t base = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(APS_CLP(&ring[wave][0]))) + 128u * i;
         auto read = [&](RfRegs<XBF16>& d, int c) __attribute__((always_inline)) {
             const uint32_t s = base + (c % 3) * static_cast<uint32_t>(sizeof(RfSlot));
 #pragma unroll
@@ -194,13 +171,13 @@ k_router_few(const void* __restrict__ xv, const float* __restrict__ gate, int64_
         issue(0);
         issue(1);
         issue(2);
-        rf_wait_vm<2 * RfSlot::kCopies>();
+        chain_wait_vm<2 * RfSlot::kCopies>();
         __builtin_amdgcn_wave_barrier();
         read(regs[0], 0);
         auto step = [&](auto par, int c) __attribute__((always_inline)) {
             constexpr int P = decltype(par)::value;
-            rf_wait_vm<RfSlot::kCopies>();
-            __builtin_amdgcn_s_waitcnt(0xF | (0x7 << 4) | (0x0 << 8) | (0x3 << 14));   // chunk c's reads: its slot is free
+            chain_wait_vm<RfSlot::kCopies>();
+            chain_wait_lgkm0();   // chunk c's reads: its slot is free
             __builtin_amdgcn_sched_barrier(0);
             issue(c + 3);
             read(regs[P ^ 1], c + 1);
@@ -212,7 +189,7 @@ k_router_few(const void* __restrict__ xv, const float* __restrict__ gate, int64_
             step(std::integral_constant<int, 0>{}, c);
             if (c + 1 < NC) step(std::integral_constant<int, 1>{}, c + 1);   // wave-uniform
         }
-        rf_wait_vm<0>();   // no copy outlives its slot
+        chain_wait_vm<0>();   // no copy outlives its slot
         __syncthreads();   // every wave has read its chunks: lg takes a slot
     }
     // the row's last lane holds the logit
