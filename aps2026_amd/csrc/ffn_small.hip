@@ -17,9 +17,11 @@
 //    of the tile to be in flight at once.
 // Every output element accumulates the same MFMA sequence over k ascending as
 // in ffn_mfma.hip, so a row's bits do not depend on its batch.
-//   Measured, bf16: 37 tokens w1||w3 27 -> 21 us (5.6 TB/s), w2 19 -> 11 us (5.5
-// TB/s); one token 23 -> 12.5 and 13 -> 3.8 us.  fp8, 65 tokens: 17 -> 14 us, w2
-// with its combine 38 -> 11 us.
+//   Measured on weights that are in no cache (three sets in turn, traced), bf16:
+// 37 tokens w1||w3 36 -> 27 us (4.4 TB/s), w2 20 -> 13 us (4.6 TB/s); one token 24 ->
+// 14 and 13 -> 4.0 us.  fp8, 65 tokens: 21 -> 18 us, w2 with its combine 38 -> 13 us.
+// (One set in a loop, which the memory-side cache holds: 37 tokens 27 -> 21 and 19 ->
+// 11 us.)
 //
 // The packed images are read at their swizzled 16-byte chunks: the four (bf16)
 // reads of a 128-byte image row follow each other and share its cache line.
@@ -77,7 +79,7 @@ __device__ inline void each_small(uint32_t lo, uint32_t hi, int bn, int blocks, 
 // itself and ranks those of its own expert, and two further blocks write the
 // plan and its tile histograms out, for the kernels after it and for callers.  That saves the dispatch's launch between
 // the router and the GEMM for 1 us in it: one bf16 token 35.0 -> 33.2 us a block,
-// 37 tokens 52.0 -> 49.9, fp8 65 tokens 45.9 -> 43.6.
+// 37 tokens 52.0 -> 49.9, fp8 65 tokens 45.9 -> 43.6 (one weight set in a loop).
 constexpr int kPlanTiles = static_cast<int>(kDispatchFewRows / kWave);
 
 struct Routes {
@@ -405,8 +407,8 @@ int small_kt(bool fp8, int ffn) { return static_cast<int>(fp8 ? ceil_div(ffn, 12
 
 // Up to 12 rows per expert on average in bf16, 24 in fp8, whose MFMAs and w2
 // passes weigh less against the weights' bytes: a tile reads its weights for
-// 32 rows, so more rows read them again.  Whole MoE block, 16 experts, us with
-// the row tiles of ffn_mfma.hip -> here, even (Zipf 1.1) expert loads:
+// 32 rows, so more rows read them again.  Whole MoE block, 16 experts (one weight
+// set in a loop), us with the row tiles of ffn_mfma.hip -> here, even (Zipf 1.1) expert loads:
 //   bf16  1 token 60 -> 40 (60 -> 40), 37 69 -> 56 (68 -> 56), 96 70 -> 58 (69 ->
 //         64), 128 69 -> 59 (70 -> 78), 256 70 -> 83 (73 -> 84)
 //   fp8   1 token 74 -> 44 (73 -> 44), 65 86 -> 58 (86 -> 61), 192 87 -> 63 (87 ->
