@@ -199,6 +199,12 @@ bool slot_lists(const WeightSet& w, int64_t rows, int32_t out_dtype) {
     return w.compute == APS_DTYPE_E4M3 && out_dtype == APS_DTYPE_BF16 && aps::ffn_down_fold_fits(rows, w.H, w.F);
 }
 
+// Whether the w1||w3 launch of few tokens makes the plan (after the few-token
+// router).
+bool makes_plan(const WeightSet& w, int64_t rows) {
+    return w.compute != APS_DTYPE_F32 && aps::ffn_small_fits(w.compute == APS_DTYPE_E4M3, rows, w.F, w.E);
+}
+
 // Routing (from `logits`; nullptr when the router kernel already wrote the
 // routes into the workspace, and past few tokens the tile histogram), dispatch,
 // FFN and combine.
@@ -227,8 +233,7 @@ int grouped_from_logits(const WeightSet& w, const void* x, bool x_is_f32, const 
     auto* stoks = reinterpret_cast<uint32_t*>(ws + L.slot_tokens);
     // few tokens on the one-wave tiles: the w1||w3 launch makes the plan itself
     const aps::SmallPlan plan{routes, tiles, counts, offsets, arows, rpos, slots ? slot1 : nullptr, srows, stoks, tiles0};
-    const bool planned = few && w.compute != APS_DTYPE_F32 &&
-                         aps::ffn_small_fits(w.compute == APS_DTYPE_E4M3, rows, w.F, w.E);
+    const bool planned = few && makes_plan(w, rows);
     if (!planned && slots)
         APS_HIP(aps::launch_dispatch_scatter(routes, few ? nullptr : tiles, rows, w.E, counts, offsets, arows, rpos,
                                              nullptr, s, few ? nullptr : tiles0, slot1, srows, stoks, tiles, tiles0),
@@ -963,9 +968,14 @@ int aps_moe_forward(uint64_t handle, const void* x, int32_t x_dtype, const float
                               aps::router_quantises_x(w->H, w->E);
     auto* xq = xq_in_router ? reinterpret_cast<uint8_t*>(ws + L.xq) : nullptr;
     auto* xqs = xq_in_router ? reinterpret_cast<float*>(ws + L.xq_scale) : nullptr;
-    // (the few-token router copies fp32 x 16 bytes at a time)
+    // The few-token router copies fp32 x 16 bytes at a time.  With bf16 x a chain
+    // of 512 steps is shorter than its launch's own cost: there only where the
+    // w1||w3 launch then makes the plan (hidden 512, 16 experts of 64, us token-major
+    // router -> few: 64 tokens 18.6 -> 18.4, of 448 21.1 -> 20.2; past that rule 128
+    // tokens 20.8 -> 22.1, 256 24.2 -> 25.1, of 448 32.7 -> 33.5).
+    const bool bf16_x = x_dtype == APS_DTYPE_BF16;
     const bool few = aps::router_few_fits(rows, w->H, w->E) &&
-                     (x_dtype == APS_DTYPE_BF16 || (reinterpret_cast<uintptr_t>(x) & 15u) == 0);
+                     (bf16_x ? w->H > 512 || makes_plan(*w, rows) : (reinterpret_cast<uintptr_t>(x) & 15u) == 0);
     if (few)
         APS_HIP(aps::launch_router_few(x, x_dtype == APS_DTYPE_BF16, gate, rows, w->H, w->E, logits, routes, xb, xq,
                                        xqs, s),

@@ -166,13 +166,14 @@ def test_few_token_router_equals_the_token_major_router(gpu_device, dtype, x32, 
     w.release()
 
 
+@pytest.mark.parametrize("H", [512, 1024])
 @pytest.mark.parametrize("dtype,E,F", [("fp8", 16, 448), ("fp8", 5, 512), ("bf16", 16, 448), ("bf16", 3, 64)])
-def test_tile_histograms_of_few_tokens(gpu_device, dtype, E, F):
+def test_tile_histograms_of_few_tokens(gpu_device, dtype, E, F, H):
     """The tile histograms of the published plan after a forward, whatever made
-    the plan: the w1||w3 launch, the counting dispatch or the router (257
-    tokens); the slot-0 histogram with an fp8 set."""
-    H = 512
-    print(f"[gpu-case] tile histograms {dtype} E={E} F={F}", flush=True)
+    the plan: the w1||w3 launch, the counting dispatch (hidden 1024) or the
+    router (257 tokens, and at hidden 512 from where w1||w3 makes no plan); the
+    slot-0 histogram with an fp8 set."""
+    print(f"[gpu-case] tile histograms {dtype} E={E} F={F} H={H}", flush=True)
     w = weights(dtype, E, H, F, gpu_device, E + F)
     g = torch.Generator(device=gpu_device)
     g.manual_seed(E)
