@@ -90,16 +90,17 @@ constexpr int kKeyTile = 16;                         // keys per score tile / va
 // in lanes 4 l .. 4 l + 3 the position of row r0 + l.
 template <bool PACKED>
 __device__ inline uint32_t chain_pairs(const uint32_t* __restrict__ row_pos, const uint32_t* __restrict__ anc,
-                                       int64_t anc_stride, int64_t r0, int nr, int lane, uint32_t& pos) {
+                                       int64_t anc_stride, int64_t r0, int nr, int lane, int& pos) {
     const int r = lane & 3, l = (lane >> 2) & 3;
+    const uint32_t most = anc_stride < 0x7FFFFFFF ? static_cast<uint32_t>(anc_stride - 1) : 0x7FFFFFFEu;
     bool ok = false;
     pos = 0;
     if (lane < 16 && l < nr) {
         const int64_t row = r0 + r, last = r0 + l;
-        int64_t pr = r < l ? row_pos[row] : 0, pl = row_pos[last];
-        pr = pr < anc_stride ? pr : anc_stride - 1;
-        pl = pl < anc_stride ? pl : anc_stride - 1;
-        pos = static_cast<uint32_t>(pl);
+        uint32_t pr = r < l ? row_pos[row] : 0u, pl = row_pos[last];
+        pr = pr < most ? pr : most;
+        pl = pl < most ? pl : most;
+        pos = static_cast<int>(pl);
         ok = r < l && pr <= pl && (PACKED ? anc[row] == anc[last] : anc[last * anc_stride + pr] == static_cast<uint32_t>(row));
     }
     return static_cast<uint32_t>(__ballot(ok));
@@ -300,8 +301,8 @@ __device__ inline void attend_row(const float* __restrict__ q, const float* __re
 // unchanged except that a -0 would turn +0; keys before it keep the chain
 // at its +0 start; the last tile's padding has p = 0 and v = 0.  Infinite and
 // NaN values of a key outside a row's window would turn its output NaN
-// (0 * inf): a run with a NaN output is done again row by row, each row on
-// its own keys alone (the check rides on the run's last barrier).
+// (0 * inf): a wave with a NaN output in a run of several rows does its
+// dimensions again row by row, each row on its own keys alone.
 //   K and V go from global memory straight to registers (LDS holds only the
 // scores and the chain's key rows, so two workgroups fit a CU at 1,024-key
 // windows, and three at key spans up to 784).  Scores: wave w takes the
@@ -333,7 +334,6 @@ k_attention_group(const float* __restrict__ q, const float* __restrict__ k, cons
     uint32_t* chain = reinterpret_cast<uint32_t*>(sc + kGroupQueries * sw);   // [sw - 1] key rows
     __shared__ int qlo[kGroupQueries], qhi[kGroupQueries];   // window of each query, relative to dlo
     __shared__ float wmx[4][kGroupQueries];                  // per-wave maxima
-    __shared__ int redo;                                     // the run has a NaN output
 
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     // groups in reverse row order: later rows (longer chains in trie and
@@ -341,16 +341,15 @@ k_attention_group(const float* __restrict__ q, const float* __restrict__ k, cons
     const int64_t g0 = static_cast<int64_t>(gridDim.x / kv_heads - 1 - blockIdx.x / kv_heads) * kGroupRows;
     const int kh = static_cast<int>(blockIdx.x % kv_heads);
     const int gn = static_cast<int>(rows - g0 < kGroupRows ? rows - g0 : kGroupRows);
-    uint32_t group_pos;
+    int group_pos;
     const uint32_t pairs = __builtin_amdgcn_readfirstlane(
         chain_pairs<PACKED>(row_pos, anc, anc_stride, g0, gn, threadIdx.x & 63, group_pos));
-    auto pos_of = [&](int i) -> int64_t {   // of the group's row i
-        return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(group_pos), 4 * i));
-    };
+    // of the group's row i (32 bits: scalar compares)
+    auto pos_of = [&](int i) { return __builtin_amdgcn_readlane(group_pos, 4 * i); };
     // the longest run from row i0 whose key range, from its first row's
     // window on, fits the LDS (sw - 1 keys: a single row always does)
     auto run_rows = [&](int i0) __attribute__((always_inline)) {
-        const int64_t p0 = pos_of(i0);
+        const int p0 = pos_of(i0);
         int nr = gn - i0;
         for (; nr > 1; --nr) {
             const int l = i0 + nr - 1;
@@ -364,12 +363,12 @@ k_attention_group(const float* __restrict__ q, const float* __restrict__ k, cons
     };
     int runs = 0;
     uint32_t run_at = 0;   // 4 bits per row: the rows of the run that starts there
-    int64_t longest = 0;
+    int longest = 0;
     for (int i0 = 0; i0 < gn; ++runs) {
         const int nr = run_rows(i0);
         run_at |= static_cast<uint32_t>(nr) << (4 * i0);
         i0 += nr;
-        const int64_t p = pos_of(i0 - 1);
+        const int p = pos_of(i0 - 1);
         longest = p > longest ? p : longest;
     }
     // Rows of several runs one per wave: always with four runs, with fewer while
@@ -378,8 +377,8 @@ k_attention_group(const float* __restrict__ q, const float* __restrict__ k, cons
     // 33 / 101 / 201 / 501 keys, leaves of a shared prompt: four runs (512 rows)
     // 33 -> 20, 53 -> 35, 79 -> 57, 152 -> 121; three 33 -> 27, 53 -> 51, 82 -> 83,
     // 160 -> 180; two 34 -> 34, 54 -> 64, 80 -> 108, 152 -> 241.
-    const int64_t window = longest + 1 < wmax ? longest + 1 : wmax;
-    bool by_row = runs == 4 || (runs == 3 && window <= 160) || (runs == 2 && window <= 32);
+    const int window = longest + 1 < wmax ? longest + 1 : wmax;
+    const bool by_row = runs == 4 || (runs == 3 && window <= 160) || (runs == 2 && window <= 32);
     for (int i0 = 0, nr; !by_row && i0 < gn;) {
     const int64_t r0 = g0 + i0;
     // (opaque per run: addresses hoisted out of the loop cost spills)
@@ -388,21 +387,21 @@ k_attention_group(const float* __restrict__ q, const float* __restrict__ k, cons
     const int lane = tid & 63;
     nr = (run_at >> (4 * i0)) & 15;
     const int64_t last = r0 + nr - 1;
-    const int64_t plast = pos_of(i0 + nr - 1);
-    const int64_t p0 = pos_of(i0);
-    const int dlo = static_cast<int>(p0 + 1 > wmax ? p0 + 1 - wmax : 0);
-    const int dhi = static_cast<int>(plast);
+    const int p0 = pos_of(i0);
+    const int dlo = p0 + 1 > wmax ? p0 + 1 - wmax : 0;
+    const int dhi = pos_of(i0 + nr - 1);
     const int W = dhi - dlo + 1;
     const int ntiles = (W + kKeyTile - 1) / kKeyTile;   // 16-key tiles (at most capacity / 16)
     const int64_t seg = PACKED ? static_cast<int64_t>(anc[last]) : 0;
-    // (a shuffle reads active lanes only: before the branch)
-    const uint32_t query_pos = static_cast<uint32_t>(__shfl(static_cast<int>(group_pos), 4 * i0 + lane));
     if (tid < kGroupQueries) {
         const int r = tid / kGroup;
+        int pr = p0;
+#pragma unroll
+        for (int i = 1; i < kGroupRows; ++i)
+            if (r == i) pr = pos_of(i0 + i);
         if (r < nr) {
-            const int64_t pr = query_pos;
-            qhi[tid] = static_cast<int>(pr) - dlo;
-            qlo[tid] = static_cast<int>(pr + 1 > wmax ? pr + 1 - wmax : 0) - dlo;
+            qhi[tid] = pr - dlo;
+            qlo[tid] = (pr + 1 > wmax ? pr + 1 - wmax : 0) - dlo;
         } else {
             qhi[tid] = -1;   // a padding row: an empty window
             qlo[tid] = 0;
@@ -493,7 +492,6 @@ k_attention_group(const float* __restrict__ q, const float* __restrict__ k, cons
 
     // ---- softmax, per query on the 16 threads of one wave (queries
     // 4 w .. 4 w + 3 on wave w), so it needs no workgroup barrier ----
-    if (tid == 0) redo = 0;   // between barriers: every wave has read the last run's
     const int qi = tid / 16, part = tid % 16;
     const char* const vbase = reinterpret_cast<const char*>(v + kh * kHeadDim);   // uniform: 32-bit lane offsets
     const uint32_t dbytes = static_cast<uint32_t>(32 * wave + 2 * qq) * sizeof(float);   // this lane's two dimensions
@@ -547,20 +545,36 @@ k_attention_group(const float* __restrict__ q, const float* __restrict__ k, cons
             group(g + 3, vb3, 1);
         }
     }
+    // (lane group qj holds row qj's four heads)
     bool nan = false;
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
-        const int qx = 4 * qj + t;   // query: row qx / 4, head qx % 4
-        const int r = qx / kGroup;
-        if (r < nr) {
-            nan = nan || o[0][t] != o[0][t] || o[1][t] != o[1][t];
-            *reinterpret_cast<af2*>(out + ((r0 + r) * q_heads + kh * kGroup + qx % kGroup) * kHeadDim + 32 * wave +
-                                    2 * qq) = af2{o[0][t], o[1][t]};
+    for (int t = 0; t < 4; ++t) nan = nan || o[0][t] != o[0][t] || o[1][t] != o[1][t];
+    if (nr > 1 && __ballot(nan && qj < nr) != 0) {   // wave-uniform: this wave's dimensions again, row by row
+        for (int r = 0; r < nr; ++r) {
+            const int l0 = qlo[kGroup * r], h0 = qhi[kGroup * r];
+            ag4_t own[2] = {};
+            for (int g = l0 / kKeyTile; g <= h0 / kKeyTile; ++g) {
+                vload(g, vb0);
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const int w = 16 * g + 4 * u + qj;
+                    if (w < l0 || w > h0) vb0[u] = af2{0.0f, 0.0f};
+#pragma unroll
+                    for (int i = 0; i < 2; ++i)
+                        own[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(sc[qq * sw + w], vb0[u][i], own[i], 0, 0, 0);
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+                if (qj == r) o[i] = own[i];
         }
     }
-    if (nan) redo = 1;
-    __syncthreads();   // also: the next run writes the chain and the scores
-    by_row = nr > 1 && redo;
+#pragma unroll
+    for (int t = 0; t < 4; ++t)   // head t
+        if (qj < nr)
+            *reinterpret_cast<af2*>(out + ((r0 + qj) * q_heads + kh * kGroup + t) * kHeadDim + 32 * wave + 2 * qq) =
+                af2{o[0][t], o[1][t]};
+    __syncthreads();   // the next run writes the chain and the scores
     i0 += nr;
     }
     if (by_row && wave < gn)   // wave-uniform
