@@ -365,24 +365,6 @@ hipError_t launch_linear_mfma_multi(const float* x, int64_t rows, int in_f, int 
     // take 14, 29, 57 us, and 114 and 228 for the two block kernels; the
     // rest is what its operand reads and copies add.
     const int64_t cus = num_cus(), rt = ceil_div(rows, kLRows);
-    // A short K that ends in half a stage (in_f % 32 == 16) on many blocks is
-    // bound by y's stores, and the ring's 64 KB of LDS leave two blocks to a CU:
-    // SIMT blocks of 64 x 64 there.  us, ring -> SIMT: 20,000 rows of 16 -> 4096 236
-    // -> 66, of 48 -> 4096 273 -> 132, of 112 -> 11008 935 -> 735; 333 rows of 16 ->
-    // 4096 7.6 -> 4.2; past the line 17 rows of 48 -> 11008 4.5 -> 5.0, 4,096 rows of
-    // 208 -> 1000 27.6 -> 29.0.
-    bool simt = in_f % kLStageK != 0 && in_f <= 176;
-    for (int i = 0; i < count; ++i) {
-        const int64_t blocks = ceil_div(out_f[i], kF32BN) * ceil_div(rows, kF32BM);
-        simt = simt && out_f[i] >= kF32BN && 8 * blocks >= 3 * cus && 70 * blocks >= cus * in_f;
-    }
-    if (simt) {
-        for (int i = 0; i < count; ++i) {
-            const hipError_t e = launch_linear_any_f32(x, w[i], bias[i], y[i], rows, in_f, out_f[i], s, true);
-            if (e != hipSuccess) return e;
-        }
-        return hipSuccess;
-    }
     auto cost = [&](int br, int bc, double us) {
         int64_t t = 0;
         for (int i = 0; i < count; ++i) t += ceil_div(out_f[i], bc);
@@ -403,6 +385,24 @@ hipError_t launch_linear_mfma_multi(const float* x, int64_t rows, int in_f, int 
     int64_t waves = 0;
     for (int i = 0; i < count; ++i) waves += ceil_div(out_f[i], 16) * ceil_div(rows, 16);
     if (rows <= 16 || waves <= 2 * cus) APS_SMALL(1, 1, 1, 1, 8);
+    // A short K that ends in half a stage (in_f % 32 == 16) on many blocks is
+    // bound by y's stores, and the ring's 64 KB of LDS leave two blocks to a CU:
+    // SIMT blocks of 64 x 64 there.  us, ring -> SIMT: 20,000 rows of 16 -> 4096 236
+    // -> 66, of 48 -> 4096 273 -> 132, of 112 -> 11008 935 -> 735; 333 rows of 16 ->
+    // 4096 7.6 -> 4.2; past the line 17 rows of 48 -> 11008 4.5 -> 5.0, 4,096 rows of
+    // 176 -> 1000 24 -> 26.
+    bool simt = in_f % kLStageK != 0 && in_f <= 144;
+    for (int i = 0; i < count; ++i) {
+        const int64_t blocks = ceil_div(out_f[i], kF32BN) * ceil_div(rows, kF32BM);
+        simt = simt && out_f[i] >= kF32BN && 8 * blocks >= 3 * cus && 70 * blocks >= cus * in_f;
+    }
+    if (simt) {
+        for (int i = 0; i < count; ++i) {
+            const hipError_t e = launch_linear_any_f32(x, w[i], bias[i], y[i], rows, in_f, out_f[i], s, true);
+            if (e != hipSuccess) return e;
+        }
+        return hipSuccess;
+    }
     const bool whole = in_f % kLStageK == 0;   // the block kernels take whole stages only
     const double c11 = cost(32, 32, 22.5), c12 = cost(32, 64, 38.5), c22 = cost(64, 64, 63.5);
     const double c64 = whole ? cost(128, 64, 121.0) : 1e300, c128 = whole ? cost(128, 128, 230.0) : 1e300;

@@ -64,9 +64,9 @@ def test_fp32_experts_block_edges(gpu_device, T, E, H, F):
 
 
 # k = 16 mod 32 on both sides of the rule that sends short k to SIMT blocks (k up
-# to 176, 96 blocks and more, out of 64 and more): whole and partly filled blocks
-@pytest.mark.parametrize("rows,k,n", [(6144, 16, 64), (6080, 16, 64), (6100, 16, 60), (700, 48, 1100), (1000, 176, 2600),
-                                      (2800, 80, 516), (1000, 208, 2600)])
+# to 144, 96 blocks and more, out of 64 and more): whole and partly filled blocks
+@pytest.mark.parametrize("rows,k,n", [(6144, 16, 64), (6080, 16, 64), (6100, 16, 60), (700, 48, 1100), (1000, 144, 2600),
+                                      (2800, 80, 516), (1000, 176, 2600), (1000, 208, 2600)])
 @pytest.mark.parametrize("bias", [True, False])
 def test_linear_short_half_stage(gpu_device, rows, k, n, bias):
     note(f"linear short k rows={rows} k={k} n={n} bias={bias}")
