@@ -435,9 +435,9 @@ bool ffn_small_fits(bool fp8, int64_t rows, int ffn, int experts) {
 //         73), 613 71 -> 77 (78 -> 80)
 //   Many experts keep the mean low whatever the load: past 512 bf16 tokens (and
 // 8192 columns, as above) an expert that takes them all reads its weights too
-// often (64 experts, hidden
-// 4096, us row tiles -> here, even / Zipf 1.1 / every token to two experts: 512
-// tokens 230 -> 218 / 252 -> 253 / 107 -> 118, 768 231 -> 228 / 257 -> 263 / 108 -> 129).
+// often.  64 experts, hidden 4096, us row tiles -> here, even / Zipf 1.1 / every
+// token to two experts: 512 tokens 230 -> 218 / 252 -> 253 / 107 -> 118, 768 tokens
+// 231 -> 228 / 257 -> 263 / 108 -> 129.
 bool ffn_down_small_fits(bool fp8, int64_t rows, int ffn, int experts) {
     if (!fp8 && rows > 512 && static_cast<int64_t>(experts) * ffn > 8192) return false;
     return 2 * rows <= (fp8 ? 32 : 24) * static_cast<int64_t>(experts) && small_kt(fp8, ffn) <= (fp8 ? 4 : 7);

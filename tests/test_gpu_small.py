@@ -82,7 +82,8 @@ def test_w2_tiles_between_the_rules(gpu_device, dtype, E, H, F):
 def test_many_experts_leave_the_small_tiles_early(gpu_device, dtype, E, H, F):
     """w1||w3 past 8192 columns over all experts: 8 experts' worth of rows, that
     edge and one past it, and the mean's own edge, against a batch of row
-    tiles; up to 8192 columns (64 x 128) the mean alone."""
+    tiles; up to 8192 columns (64 x 128) the mean alone.  512 tokens is w2's own
+    line for bf16."""
     per = 24 if dtype == "fp8" else 12
     print(f"[gpu-case] many experts {dtype} E={E} H={H} F={F}", flush=True)
     w = weights(dtype, E, H, F, gpu_device, E + F)
@@ -93,7 +94,7 @@ def test_many_experts_leave_the_small_tiles_early(gpu_device, dtype, E, H, F):
     x[:, 0], gate[:, 0] = 1.0, -1.1 * torch.log(torch.arange(1, E + 1, device=gpu_device).float())
     x = x.bfloat16()
     big = moe.moe_forward_gpu(x, gate, w).clone()
-    for n in (4 * per, 4 * per + 1, E * per // 2, E * per // 2 + 1):
+    for n in (4 * per, 4 * per + 1, E * per // 2, E * per // 2 + 1, 512, 513):
         got = moe.moe_forward_gpu(x[:n].contiguous(), gate, w)
         assert torch.equal(got.view(torch.int16), big[:n].view(torch.int16)), n
     w.release()
